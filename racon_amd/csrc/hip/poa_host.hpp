@@ -115,11 +115,11 @@ struct PassLaunch {
 // estimate, or by the exact node bound when row_cap is 0), the row pitch of
 // the longest layer, DP rows capped at row_cap (0: exact, node bound + 1)
 // with a pool of kPoaHPoolRows global score rows (0: one per DP row),
-// and the deepest ring that fits lds_limit, for the default or the wide
-// kernel. False when even a ring of 0 rows does not fit (the layer bytes
+// and the deepest ring that fits lds_limit with `waves` waves per CU, for the
+// default or the wide kernel. False when even a ring of 0 rows does not fit (the layer bytes
 // alone exceed the limit).
 bool plan_pass(const PoaWindow* host, const std::vector<uint32_t>& ws, uint32_t row_cap,
-               uint32_t lds_limit, uint32_t tune_ring, bool wide, PassPlan* plan);
+               uint32_t lds_limit, uint32_t tune_ring, uint32_t waves, bool wide, PassPlan* plan);
 
 // Resident slots of a pass: the kernel's occupancy times the CUs divided by
 // the lane's share (all windows for RH_POA_STATIC, one for RH_POA_PLAIN),

@@ -8,13 +8,13 @@
 //   2. its DFS topological order (roots in increasing node id, predecessors
 //      then aligned nodes pushed, an aligned set emitted right after the
 //      node that reached it first);
-//   3. linear-gap NW of the layer against that order: lanes own 8-column
-//      strips of each DP row, predecessor rows stream from the slot, the
+//   3. linear-gap NW of the layer against that order: lanes own strips of
+//      4 to 20 columns of each DP row, predecessor rows come from LDS, the
 //      horizontal gap chain is a wave prefix-max, and each cell records the
 //      first matching move (diagonal over predecessors in in-edge order,
-//      then vertical, then horizontal) as a 16-bit code;
+//      then vertical, then horizontal);
 //   4. the traceback from the first sink row with the highest last-column
-//      score, following the codes;
+//      score, following the recorded moves;
 //   5. insertion of the layer into the graph (edge weight = w[i-1] + w[i],
 //      w = phred - 33 or 1) and a new topological order.
 // After the last layer: heaviest-bundle path with branch completion,
@@ -27,6 +27,8 @@
 // of windows in flight (persistent kernel over a size-ordered queue) and from
 // the 64-lane DP rows.
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "poa_types.hpp"
 
@@ -75,7 +77,6 @@ constexpr uint32_t kAligned = RH_POA_ALIGNED;
 constexpr int kStrip = 4;                  // DP columns per lane per tile
 constexpr int kTile = kWave * kStrip;      // 256 columns per tile
 constexpr int32_t kNegInf = -(1 << 29);
-constexpr int32_t kNegKey = -(1 << 30);  // below every (score, 255 - k) key
 // Move codes (16 bits per DP cell): bits 15-14 the move (diagonal,
 // vertical, horizontal); for diagonal and vertical moves bits 12-0 name the
 // predecessor row, as the row delta r - p, or, with kCodeViaK set, as the
@@ -85,8 +86,7 @@ constexpr uint16_t kCodeVert = 0x4000;
 constexpr uint16_t kCodeHorz = 0x8000;
 constexpr uint16_t kCodeViaK = 0x2000;
 constexpr uint32_t kCodePayload = 0x1fff;
-// Rows with one predecessor in the packed DP store only the move of each
-// cell, as a 2-bit kind 2 fd + fv from the flags fd (not diagonal) and fv
+// Band rows with one predecessor store only the move of each cell, as a 2-bit kind 2 fd + fv from the flags fd (not diagonal) and fv
 // (not vertical): 0 or 1 diagonal, 2 vertical, 3 horizontal (column j at
 // bits 2 (j - 1) % 8 of byte (j - 1) / 4 of the row's code memory). The
 // predecessor is implied, and column 0 is always vertical.
@@ -175,7 +175,7 @@ struct Slot {
   __device__ int32_t* lpath() const { return (int32_t*)(p + L->lpath); }
   __device__ int32_t* sink_score() const { return (int32_t*)(p + L->sink_score); }
   __device__ int32_t* tie_mark() const { return (int32_t*)(p + L->tie_mark); }
-  __device__ uint64_t* row_pred4() const { return (uint64_t*)(p + L->row_pred4); }
+  __device__ uint4* row_rec() const { return (uint4*)(p + L->row_rec); }
 
   int32_t n_nodes;
   int32_t n_edges;
@@ -660,114 +660,6 @@ __device__ __forceinline__ int dp_layer(CParams& P, const Slot& s, uint8_t* lds,
   return best_row;
 }
 
-// Strip rows in LDS (the one-pass DP below) are laid out quad-major: quad q
-// (strip columns j0 + 4q .. j0 + 4q + 3) of lane k sits at element
-// jq + q * qs with jq = 4k and qs = 4 * (lanes with columns <= L), so that
-// consecutive lanes touch consecutive 8-byte quads (no LDS bank conflicts);
-// column 0 sits at the row's last element. H[p][j0 - 1], the last column
-// of the previous lane's strip, comes from that lane with a DPP shift.
-__device__ __forceinline__ uint32_t from_prev_lane(uint32_t x) {
-  return static_cast<uint32_t>(
-      __builtin_amdgcn_update_dpp(0, static_cast<int>(x), 0x138, 0xf, 0xf, false));  // wave_shr:1
-}
-
-// Predecessor row p (entry e) at the lane's strip: hp[u] = H[p][j0 - 1 + u],
-// u = 0..W. Row 0 is the virtual start row (j * gap).
-template <int W>
-__device__ __forceinline__ void load_strip(const int16_t* ring, int pitch, const Slot& s, int e,
-                                           int j0, int jq, int qs, int L, int32_t gap,
-                                           int32_t* hp) {
-  const int p = e & kPredRowMask;
-  const int sl = static_cast<unsigned>(e) >> kPredRowBits;
-  if (p == 0) {
-#pragma unroll
-    for (int u = 0; u <= W; ++u) hp[u] = (j0 - 1 + u) * gap;
-  } else if (sl < kSlotGlobal) {
-    const int16_t* row = ring + sl * pitch;
-#pragma unroll
-    for (int q = 0; q < W / 4; ++q) Quad<int16_t>::load(row + jq + q * qs, hp + 1 + 4 * q);
-    const int32_t c0 = row[pitch - 1];
-    const int32_t prev = static_cast<int32_t>(from_prev_lane(static_cast<uint32_t>(hp[W])));
-    hp[0] = lane_id() == 0 ? c0 : prev;
-  } else {
-    const int32_t* row = s.H_row(p, pitch);
-#pragma unroll
-    for (int u = 0; u <= W; ++u) {
-      const int j = j0 - 1 + u;
-      hp[u] = j <= L ? row[j] : kNegInf;
-    }
-    wait_stores();
-  }
-}
-
-// Rest of one DP row once the best diagonal (bd) and vertical (bv) moves of
-// every strip column are known: horizontal chain, move codes, row storage.
-// With kKeys the moves are (score << 8 | 255 - k) keys of predecessor k,
-// else plain scores from predecessor 0. Lane 0's chain starts at column 0
-// (key or score c0, code vertical). Returns H[row][L].
-template <int W, bool kKeys>
-__device__ __forceinline__ int32_t finish_row(const int32_t* bd, const int32_t* bv, int32_t c0,
-                                              uint32_t pay0, int lane, int j0, int jq, int qs,
-                                              bool live, int L, int32_t gap, int own, int pitch,
-                                              int16_t* ring, int32_t* Hg, uint16_t* Cr,
-                                              int end_lane, int end_u) {
-  auto score = [](int32_t x) { return kKeys ? (x >> 8) : x; };
-  // code payload of the move's predecessor: the row's single predecessor
-  // (pay0: row delta or kCodeViaK), else kCodeViaK | k from the key
-  auto pred = [&](int32_t x) -> uint32_t {
-    if (!kKeys) return pay0;
-    return kCodeViaK | (255u - (static_cast<uint32_t>(x) & 255u));
-  };
-  const int32_t h0 = score(c0);
-  int32_t pm = lane == 0 ? h0 : kNegInf;
-  int32_t pre[W];
-#pragma unroll
-  for (int u = 0; u < W; ++u) {
-    pm = max(pm, score(max(bd[u], bv[u])) - (j0 + u) * gap);
-    pre[u] = pm;
-  }
-  const int32_t excl = wave_shift_right(wave_prefix_max(pm), kNegInf);
-  int32_t h[W];
-  uint32_t cd[W];
-#pragma unroll
-  for (int u = 0; u < W; ++u) {
-    h[u] = max(pre[u], excl) + (j0 + u) * gap;
-    const uint32_t c = score(bv[u]) == h[u] ? (kCodeVert | pred(bv[u])) : kCodeHorz;
-    cd[u] = score(bd[u]) == h[u] ? (kCodeDiag | pred(bd[u])) : c;
-  }
-  if (live) {
-#pragma unroll
-    for (int q = 0; q < W / 4; ++q) {
-      uint2 v;
-      v.x = cd[4 * q] | (cd[4 * q + 1] << 16);
-      v.y = cd[4 * q + 2] | (cd[4 * q + 3] << 16);
-      *reinterpret_cast<uint2*>(Cr + (j0 - 1) + 4 * q) = v;
-    }
-    if (own < kSlotGlobal) {
-      int16_t* row = ring + own * pitch;
-#pragma unroll
-      for (int q = 0; q < W / 4; ++q) Quad<int16_t>::store(row + jq + q * qs, h + 4 * q);
-    }
-  }
-  if (own == kSlotGlobal) {
-#pragma unroll
-    for (int u = 0; u < W; ++u) {
-      if (j0 + u <= L) Hg[j0 + u] = h[u];
-    }
-  }
-  if (lane == 0) {
-    if (own < kSlotGlobal) ring[own * pitch + pitch - 1] = static_cast<int16_t>(h0);
-    if (own == kSlotGlobal) Hg[0] = h0;
-    Cr[pitch - 1] = static_cast<uint16_t>(kCodeVert | pred(c0));
-  }
-  int32_t last = h[0];
-#pragma unroll
-  for (int u = 1; u < W; ++u) {
-    if (u == end_u) last = h[u];
-  }
-  return __builtin_amdgcn_readlane(last, end_lane);
-}
-
 // ---- packed 16-bit pairs: two DP columns per 32-bit register ----
 
 typedef short __attribute__((ext_vector_type(2))) I16x2;
@@ -807,6 +699,21 @@ __device__ __forceinline__ uint32_t pk_scan(uint32_t a) {
   const I16x2 v = as_i16x2(a);
   return pk_bits(__builtin_elementwise_max(v, __builtin_shufflevector(v, v, 0, 0)));
 }
+// the same for unsigned halves
+__device__ __forceinline__ uint32_t pk_max_u(uint32_t a, uint32_t b) {
+  return pk_bits(__builtin_elementwise_max(as_u16x2(a), as_u16x2(b)));
+}
+__device__ __forceinline__ uint32_t pk_max_hi_u(uint32_t a, uint32_t b) {
+  const U16x2 v = as_u16x2(b);
+  return pk_bits(__builtin_elementwise_max(as_u16x2(a), __builtin_shufflevector(v, v, 1, 1)));
+}
+__device__ __forceinline__ uint32_t pk_scan_u(uint32_t a) {
+  const U16x2 v = as_u16x2(a);
+  return pk_bits(__builtin_elementwise_max(v, __builtin_shufflevector(v, v, 0, 0)));
+}
+__device__ __forceinline__ uint32_t pk_sub_sat(uint32_t a, uint32_t b) {
+  return pk_bits(__builtin_elementwise_sub_sat(as_u16x2(a), as_u16x2(b)));
+}
 __device__ __forceinline__ uint32_t pk_splat(int32_t v) {
   return (static_cast<uint32_t>(v) & 0xffffu) * 0x10001u;
 }
@@ -814,7 +721,481 @@ __device__ __forceinline__ int32_t pk_half(uint32_t x, int hi) {
   return hi ? static_cast<int32_t>(x) >> 16 : static_cast<int32_t>(static_cast<int16_t>(x & 0xffffu));
 }
 
-// Per-lane constants of the packed rows: pair q holds strip columns
+// ---- packed DP rows (dp_rows) ----
+//
+// One pass of the wave per DP row: lane k owns columns kW .. kW + W - 1 of
+// columns 0..L (column 0 is lane 0's first), two columns per register. Every
+// value is kept as G = H - j * gap + bias in unsigned 16 bits: a horizontal
+// move keeps G, a vertical one adds gap, a diagonal one s - gap, so the
+// horizontal chain is a plain prefix max and column 0 is an ordinary column
+// (the diagonal into it comes from column -1, a value below every other).
+// G falls by |gap| per row at most and rises by max(s) - gap per column, so
+// the rows fit 16 bits while |gap| (V + 2) + (max(s) - gap)(L + 1) does
+// (rows_fit_16).
+//
+// A row's scores live in its LDS slot, column j at element j; a lane reads
+// only what it wrote itself, so rows need no ordering between lanes. The row's
+// base selects the substitution scores with one byte permute per pair: the
+// pair's letters are kept as selectors into an eight-byte table (low bytes of
+// s - gap for A, C, G, T, then the high bytes) that is built per row in scalar
+// registers.
+//
+// What a row stores for the traceback: per column a move kind (bit 1: the
+// diagonal reaches the cell's score, bit 0: the vertical does; diagonal is
+// taken before vertical before horizontal) and, for rows with two to four
+// predecessors, the index of the first predecessor with the column's best
+// score (2 bits each): the diagonal into column j takes the one of column
+// j - 1, the vertical the one of column j, which is spoa's choice. Rows
+// outside this form (more than four predecessors, the virtual start row or a
+// row in global memory among them, their own row in global memory, letters
+// other than A, C, G, T) store 16-bit codes, column j at element j.
+//
+// The rows are bound by their instructions: a wave alone issues one about
+// every 8 cycles, and 4 waves per SIMD share the issue slots. A row with one
+// predecessor takes about 70 vector and 25 scalar instructions at W = 8
+// (the form before, with per-row predecessor lists, a separate column 0 and
+// 16-bit codes for rows of several predecessors, took 117 and 95 over all
+// rows). One 500 bp window at 30 layers: DP 17.5 -> 8.5 ms; 9,980 windows of
+// 500 bp at 52 layers: DP 521 -> 282 wave-seconds, kernel 250 -> 176 ms.
+
+// Row descriptor: number of predecessors (0: the general form), 8 x the code
+// of the row's base, own slot, slots of up to four predecessors, whether the
+// single predecessor is the row before, and the sink flag.
+constexpr uint32_t kRecPreds = 7u;
+constexpr uint32_t kRecBase = 0x18u;
+constexpr int kRecOwnShift = 5;
+constexpr int kRecPredShift = 10;
+constexpr uint32_t kRecChain = 1u << 30;
+constexpr uint32_t kRecSink = 1u << 31;
+constexpr uint32_t kRecMaxPreds = 4;
+
+// Layout of a row's move record: per lane row_record_bytes(W) bytes, the kinds in
+// the first half and the predecessor indices in the second; in each half the
+// even columns' fields are followed by the odd columns', the first column in
+// the highest bits (groups of eight column pairs for W > 16).
+__device__ __forceinline__ int row_record_bytes(int W) { return W == 4 ? 2 : W == 8 ? 4 : W <= 16 ? 8 : 16; }
+
+// Byte and bit of column j's kind in the row's record (its predecessor
+// index: half a lane record later).
+struct RecordBit {
+  int byte, bit;
+};
+__device__ __forceinline__ RecordBit record_bit(int j, int W, int inv) {
+  const int ln = (j * inv) >> 16;  // j / W (inv = 65536 / W + 1; j < 4096)
+  const int u = j - ln * W;
+  const int q = u >> 1;
+  const int group = q >> 3;
+  const int pairs = min(8, W / 2 - 8 * group);
+  const int half = W == 4 ? 4 : W == 8 ? 8 : 16;
+  const int at = 32 * group + half * (u & 1) + 2 * (pairs - 1 - (q & 7));
+  return RecordBit{ln * row_record_bytes(W) + (at >> 3), at & 7};
+}
+
+// 16-bit rows hold every value of the layer (see above), with room for the
+// sums formed on the way. bias: the value of G = 0.
+__device__ __forceinline__ bool rows_fit_16(int match, int mismatch, int gap, int V, int L,
+                                            int* bias) {
+  const int top = max(match, mismatch);
+  const int max_abs = max(max(abs(match), abs(mismatch)), abs(gap));
+  if (gap > 0 || max_abs > 1024) return false;
+  const int m = 2 * max_abs;
+  const int64_t low = static_cast<int64_t>(-gap) * (V + 2) + 4 * m;
+  const int64_t high = static_cast<int64_t>(max(top - gap, 0)) * (L + 1) + 2 * m;
+  *bias = static_cast<int>(low);
+  return low + high <= 65535;
+}
+
+// Lane-private LDS bytes of a row slot (an LDS address).
+typedef __attribute__((address_space(3))) uint8_t LByte;
+typedef __attribute__((address_space(3))) uint32_t LWord;
+typedef uint32_t U32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t U32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) U32x4 LQuad;
+typedef __attribute__((address_space(3))) U32x2 LPair;
+
+template <int W>
+__device__ __forceinline__ void lds_row_load(uint32_t at, uint32_t* v) {
+  if constexpr (W % 8 == 0) {
+#pragma unroll
+    for (int q = 0; q < W / 8; ++q) {
+      const U32x4 x = ((const LQuad*)(size_t)at)[q];
+      v[4 * q] = x.x;
+      v[4 * q + 1] = x.y;
+      v[4 * q + 2] = x.z;
+      v[4 * q + 3] = x.w;
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < W / 4; ++q) {
+      const U32x2 x = ((const LPair*)(size_t)at)[q];
+      v[2 * q] = x.x;
+      v[2 * q + 1] = x.y;
+    }
+  }
+}
+
+template <int W>
+__device__ __forceinline__ void lds_row_store(uint32_t at, const uint32_t* v) {
+  if constexpr (W % 8 == 0) {
+#pragma unroll
+    for (int q = 0; q < W / 8; ++q) {
+      ((LQuad*)(size_t)at)[q] = U32x4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < W / 4; ++q) ((LPair*)(size_t)at)[q] = U32x2{v[2 * q], v[2 * q + 1]};
+  }
+}
+
+// Inclusive prefix max over the lanes of unsigned words (0 is the identity,
+// which lanes without a source read).
+__device__ __forceinline__ uint32_t wave_prefix_max_u(uint32_t x) {
+  const auto step = [](uint32_t v, auto ctrl, auto rows) {
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(
+        0, static_cast<int>(v), decltype(ctrl)::value, decltype(rows)::value, 0xf, false));
+  };
+  x = max(x, step(x, std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{}));
+  x = max(x, step(x, std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{}));
+  x = max(x, step(x, std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{}));
+  x = max(x, step(x, std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{}));
+  x = max(x, step(x, std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{}));
+  x = max(x, step(x, std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{}));
+  return x;
+}
+
+// x of the previous lane; lane 0 keeps its value of `old` (a register that
+// is passed from row to row, so that lane 0's constant costs nothing).
+__device__ __forceinline__ uint32_t shift_into(uint32_t old, uint32_t x) {
+  return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(
+      static_cast<int>(old), static_cast<int>(x), 0x138, 0xf, 0xf, false));
+}
+
+// One row from its best predecessor scores pp: diagonal (scores sub from the
+// letters) and vertical candidates, horizontal chain, scores into h, move
+// kinds into acc. prev and excl carry the lane-0 constants between rows.
+template <int W>
+__device__ __forceinline__ void row_scores(const uint32_t* pp, const uint32_t* sub,
+                                           uint32_t gap_pair, uint32_t& prev, uint32_t& excl,
+                                           uint32_t* h, uint32_t* bd, uint32_t* bv) {
+  constexpr int H2 = W / 2;
+  prev = shift_into(prev, pp[H2 - 1]);
+  uint32_t pre[H2];
+  uint32_t carry = 0;
+#pragma unroll
+  for (int q = 0; q < H2; ++q) {
+    // G[p][j - 1] of the pair
+    const uint32_t d = __builtin_amdgcn_alignbit(pp[q], q == 0 ? prev : pp[q - 1], 16);
+    bd[q] = pk_add(d, sub[q]);
+    bv[q] = pk_add(pp[q], gap_pair);
+    const uint32_t t = pk_scan_u(pk_max_u(bd[q], bv[q]));
+    carry = q == 0 ? t : pk_max_hi_u(t, carry);
+    pre[q] = carry;
+  }
+  // (the whole word goes through the scan: its high half, the strip's
+  // maximum, decides)
+  excl = shift_into(excl, wave_prefix_max_u(carry));
+#pragma unroll
+  for (int q = 0; q < H2; ++q) h[q] = pk_max_hi_u(pre[q], excl);
+}
+
+template <int W>
+__device__ __forceinline__ void row_kinds(const uint32_t* h, const uint32_t* bd,
+                                          const uint32_t* bv, uint32_t* acc) {
+  constexpr int H2 = W / 2;
+#pragma unroll
+  for (int q = 0; q < H2; ++q) {
+    // 1 where the candidate reaches the score (it is never above it)
+    const uint32_t below = pk_sub(h[q], 0x00010001u);
+    const uint32_t kind = (pk_sub_sat(bd[q], below) << 1) | pk_sub_sat(bv[q], below);
+    acc[q / 8] = (q % 8) == 0 ? kind : (acc[q / 8] << 2) | kind;
+  }
+}
+
+// One DP layer in packed rows; the end cell as dp_layer. W: 4, 8, 12, 16 or
+// 20 with 64 W > L.
+template <int W>
+__device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, int V, int L,
+                                       int bias, int* best_score, bool* tied) {
+  constexpr int H2 = W / 2;
+  constexpr int NA = (H2 + 7) / 8;
+  const int lane = lane_id();
+  const int pitch = static_cast<int>(P.caps.cols);
+  const int32_t gap = uniform(P.gap);
+  const int32_t match = uniform(P.match);
+  const int32_t mismatch = uniform(P.mismatch);
+  const uint32_t row_bytes = static_cast<uint32_t>(pitch) * 2;
+  const uint32_t strip = lds + static_cast<uint32_t>(lane) * (2 * W);
+  const LByte* seq = (const LByte*)(size_t)(
+      lds + static_cast<uint32_t>(align_up(static_cast<uint64_t>(P.ring_rows) * row_bytes, 16)));
+  const int n_live = (L + W) / W;
+  // letters of the strip (column j holds letter j - 1) as table selectors
+  uint32_t sel[H2];
+  bool plain = true;
+#pragma unroll
+  for (int q = 0; q < H2; ++q) {
+    uint32_t x = 0;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int idx = lane * W + 2 * q + u - 1;
+      const int c = idx >= 0 && idx < L ? static_cast<int>(seq[idx]) : 'A';
+      const int code = ((c >> 1) ^ (c >> 2)) & 3;
+      plain &= static_cast<int>((0x54474341u >> (8 * code)) & 0xffu) == c;
+      x |= (static_cast<uint32_t>(code) * 0x0101u + 0x0400u) << (16 * u);
+    }
+    sel[q] = x;
+  }
+  const bool layer_plain = __all(plain);
+  const uint32_t gap_pair = pk_splat(gap);
+  // score tables: s - gap of a mismatch in every byte pair, and the change
+  // to the match in the pair of code 0
+  const uint32_t miss = static_cast<uint32_t>(mismatch - gap) & 0xffffu;
+  const uint32_t flip = (static_cast<uint32_t>(match - gap) & 0xffffu) ^ miss;
+  const uint64_t table0 = static_cast<uint64_t>((miss >> 8) * 0x01010101u) << 32 |
+                          (miss & 0xffu) * 0x01010101u;
+  const uint64_t table1 = static_cast<uint64_t>(flip >> 8) << 32 | (flip & 0xffu);
+  const int max_abs = max(max(abs(match), abs(mismatch)), abs(gap));
+  // 1 in both halves, opaque to the optimizer (a visible 1 turns min(x, 1)
+  // into compares and selects per half)
+  uint32_t one = 0x00010001u;
+  asm volatile("" : "+s"(one));
+  uint32_t prev = pk_splat(2 * max_abs);  // lane 0: column -1, below every score
+  uint32_t excl = 0;                      // lane 0: nothing to its left
+  const int end_lane = L / W, end_u = L % W;
+  int32_t best = kNegInf;
+  int best_row = 0;
+  int ties = 0;
+  const int total_preds = uniform(s.pred_off()[V]);
+  uint32_t cur[H2];  // the scores of the row before
+#pragma unroll
+  for (int q = 0; q < H2; ++q) cur[q] = 0;
+  GByte* const codes = (GByte*)s.code();
+  const uint32_t rec_lane = static_cast<uint32_t>(lane * row_record_bytes(W));
+  for (int r0 = 1; r0 <= V; r0 += kWave) {
+    const int rk = r0 + lane;
+    uint32_t desc_v = 0;
+    if (rk <= V) desc_v = s.row_rec()[rk - 1].x;
+    if (!layer_plain) desc_v &= ~(kRecPreds | kRecChain);
+    const int chunk = uniform(min(kWave, V - r0 + 1));
+    // what the rows of the general form need of this chunk
+    int off_v = 0, end_v = 0, meta_v = 0, base = 0, pr0 = 0, pr1 = 0;
+    if (__any(rk <= V && (desc_v & kRecPreds) == 0)) {
+      if (rk <= V) {
+        off_v = s.pred_off()[rk - 1];
+        end_v = s.pred_off()[rk];
+        meta_v = s.row_meta()[rk - 1];
+      }
+      base = __builtin_amdgcn_readlane(off_v, 0);
+      pr0 = base + lane < total_preds ? s.pred_rows()[base + lane] : 0;
+      pr1 = base + kWave + lane < total_preds ? s.pred_rows()[base + kWave + lane] : 0;
+    }
+    // complete the chunk's loads here: otherwise the row loop would wait for
+    // them (and for every store issued before them) on each row
+    wait_stores();
+    if (lane < n_live) {
+      GByte* record = codes + static_cast<int64_t>(r0) * row_bytes;
+      for (int rr = 0; rr < chunk; ++rr) {
+        const uint32_t d = static_cast<uint32_t>(
+            __builtin_amdgcn_readlane(static_cast<int>(desc_v), rr));
+        const uint32_t np = d & kRecPreds;
+        uint32_t bd[H2], bv[H2];
+        if (np != 0) {
+          const auto slot_at = [&](int k) {
+            return strip + ((d >> (kRecPredShift + 5 * k)) & 31u) * row_bytes;
+          };
+          const uint64_t table = table0 ^ (table1 << (d & kRecBase));
+          uint32_t sub[H2];
+#pragma unroll
+          for (int q = 0; q < H2; ++q) {
+            sub[q] = __builtin_amdgcn_perm(static_cast<uint32_t>(table >> 32),
+                                           static_cast<uint32_t>(table), sel[q]);
+          }
+          uint32_t acc[NA], ack[NA];
+#pragma unroll
+          for (int a = 0; a < NA; ++a) ack[a] = 0;
+          if (np == 1) {
+            if ((d & kRecChain) == 0) lds_row_load<W>(slot_at(0), cur);
+            row_scores<W>(cur, sub, gap_pair, prev, excl, cur, bd, bv);
+          } else {
+            // best predecessor score of each column and the first
+            // predecessor reaching it (a later one only when better)
+            uint32_t mx[H2], kx[H2], p1[H2];
+            lds_row_load<W>(slot_at(0), mx);
+            lds_row_load<W>(slot_at(1), p1);
+#pragma unroll
+            for (int q = 0; q < H2; ++q) {
+              kx[q] = pk_min_u(pk_sub_sat(p1[q], mx[q]), one);
+              mx[q] = pk_max_u(mx[q], p1[q]);
+            }
+            if (np > 2) {
+              lds_row_load<W>(slot_at(2), p1);
+#pragma unroll
+              for (int q = 0; q < H2; ++q) {
+                const uint32_t g = pk_min_u(pk_sub_sat(p1[q], mx[q]), one);
+                kx[q] = pk_max_u(kx[q], g << 1);
+                mx[q] = pk_max_u(mx[q], p1[q]);
+              }
+              if (np > 3) {
+                lds_row_load<W>(slot_at(3), p1);
+#pragma unroll
+                for (int q = 0; q < H2; ++q) {
+                  const uint32_t g = pk_min_u(pk_sub_sat(p1[q], mx[q]), one);
+                  kx[q] = pk_max_u(kx[q], pk_mad(g, 0x00030003u, 0u));
+                  mx[q] = pk_max_u(mx[q], p1[q]);
+                }
+              }
+            }
+#pragma unroll
+            for (int q = 0; q < H2; ++q) {
+              ack[q / 8] = (q % 8) == 0 ? kx[q] : (ack[q / 8] << 2) | kx[q];
+            }
+            row_scores<W>(mx, sub, gap_pair, prev, excl, cur, bd, bv);
+          }
+          const uint32_t own = (d >> kRecOwnShift) & 31u;
+          if (own != static_cast<uint32_t>(kSlotNone)) {
+            lds_row_store<W>(strip + own * row_bytes, cur);
+          }
+          row_kinds<W>(cur, bd, bv, acc);
+          GByte* at = record + rec_lane;
+          if constexpr (W == 4) {
+            const uint32_t a = (acc[0] | (acc[0] >> 12)) & 0xffu;
+            const uint32_t k = (ack[0] | (ack[0] >> 12)) & 0xffu;
+            *(__attribute__((address_space(1))) uint16_t*)at = static_cast<uint16_t>(a | (k << 8));
+          } else if constexpr (W == 8) {
+            *(__attribute__((address_space(1))) uint32_t*)at =
+                __builtin_amdgcn_perm(ack[0], acc[0], 0x06040200u);
+          } else if constexpr (NA == 1) {
+            *(__attribute__((address_space(1))) U32x2*)at = U32x2{acc[0], ack[0]};
+          } else {
+            *(__attribute__((address_space(1))) U32x4*)at = U32x4{acc[0], acc[1], ack[0], ack[1]};
+          }
+        } else {
+          // the general form: any number of predecessors, in LDS, in global
+          // memory or the virtual start row; any letters; 16-bit codes
+          const int r = r0 + rr;
+          const int off = __builtin_amdgcn_readlane(off_v, rr);
+          const int n_preds = __builtin_amdgcn_readlane(end_v, rr) - off;
+          const int meta = __builtin_amdgcn_readlane(meta_v, rr);
+          const int own = (meta >> kRowMetaSlotShift) & 31;
+          const int j0 = lane * W;
+          uint32_t mx[H2], kx[H2];
+#pragma unroll
+          for (int q = 0; q < H2; ++q) mx[q] = kx[q] = 0;
+          for (int k = 0; k < n_preds; ++k) {
+            const int idx = off + k - base;
+            int e;
+            if (idx < kWave) {
+              e = __builtin_amdgcn_readlane(pr0, idx);
+            } else if (idx < 2 * kWave) {
+              e = __builtin_amdgcn_readlane(pr1, idx - kWave);
+            } else {
+              e = uniform(s.pred_rows()[off + k]);
+            }
+            const int p = e & kPredRowMask;
+            const int sl = static_cast<int>(static_cast<unsigned>(e) >> kPredRowBits);
+            uint32_t pp[H2];
+            if (p == 0) {
+#pragma unroll
+              for (int q = 0; q < H2; ++q) pp[q] = pk_splat(bias);
+            } else if (sl < kSlotGlobal) {
+              lds_row_load<W>(strip + static_cast<uint32_t>(sl) * row_bytes, pp);
+            } else {
+              const int32_t* row = s.H_row(p, pitch);
+#pragma unroll
+              for (int q = 0; q < H2; ++q) {
+                // (columns past L are never stored: any value does)
+                const int ja = min(j0 + 2 * q, L), jb = min(j0 + 2 * q + 1, L);
+                pp[q] = (static_cast<uint32_t>(row[ja]) & 0xffffu) |
+                        (static_cast<uint32_t>(row[jb]) << 16);
+              }
+            }
+            const uint32_t ks = static_cast<uint32_t>(k) * 0x10001u;
+#pragma unroll
+            for (int q = 0; q < H2; ++q) {
+              const uint32_t g = pk_min_u(pk_sub_sat(pp[q], mx[q]), one);
+              kx[q] = pk_mad(g, pk_sub(ks, kx[q]), kx[q]);
+              mx[q] = pk_max_u(mx[q], pp[q]);
+            }
+          }
+          uint32_t sub[H2];
+#pragma unroll
+          for (int q = 0; q < H2; ++q) {
+            uint32_t x = 0;
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+              const int idx = j0 + 2 * q + u - 1;
+              const bool same = idx >= 0 && idx < L && static_cast<int>(seq[idx]) == (meta & 0xff);
+              x |= (static_cast<uint32_t>((same ? match : mismatch) - gap) & 0xffffu) << (16 * u);
+            }
+            sub[q] = x;
+          }
+          row_scores<W>(mx, sub, gap_pair, prev, excl, cur, bd, bv);
+          if (own < kSlotGlobal) {
+            lds_row_store<W>(strip + static_cast<uint32_t>(own) * row_bytes, cur);
+          } else if (own == kSlotGlobal) {
+            int32_t* Hg = s.H_row(r, meta, pitch);
+#pragma unroll
+            for (int u = 0; u < W; ++u) {
+              if (j0 + u <= L) Hg[j0 + u] = static_cast<int32_t>((cur[u / 2] >> (16 * (u & 1))) & 0xffffu);
+            }
+          }
+          // codes: kCodeViaK | index of the predecessor
+          uint32_t kprev = shift_into(0u, kx[H2 - 1]);
+          uint16_t* Cr = s.code() + static_cast<int64_t>(r) * pitch;
+#pragma unroll
+          for (int q = 0; q < H2; ++q) {
+            const uint32_t kd = __builtin_amdgcn_alignbit(kx[q], q == 0 ? kprev : kx[q - 1], 16);
+            uint32_t code = 0;
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+              const uint32_t hu = (cur[q] >> (16 * u)) & 0xffffu;
+              const bool dg = ((bd[q] >> (16 * u)) & 0xffffu) == hu;
+              const bool vt = ((bv[q] >> (16 * u)) & 0xffffu) == hu;
+              const uint32_t kdu = (kd >> (16 * u)) & 0xffffu, kvu = (kx[q] >> (16 * u)) & 0xffffu;
+              const uint32_t c = dg ? (kCodeDiag | kCodeViaK | kdu)
+                                    : (vt ? (kCodeVert | kCodeViaK | kvu) : kCodeHorz);
+              code |= c << (16 * u);
+            }
+            *reinterpret_cast<uint32_t*>(Cr + j0 + 2 * q) = code;
+          }
+        }
+        if ((d & kRecSink) != 0) {
+          const int r = r0 + rr;
+          uint32_t last = cur[0];
+#pragma unroll
+          for (int q = 1; q < H2; ++q) {
+            uint32_t v = cur[q];
+            asm volatile("" : "+v"(v));  // (selected, not indexed through a stack copy)
+            if (q == (end_u >> 1)) last = v;
+          }
+          const uint32_t g = static_cast<uint32_t>(
+              __builtin_amdgcn_readlane(static_cast<int>(last), end_lane));
+          const int32_t h_last =
+              static_cast<int32_t>((end_u & 1) ? g >> 16 : g & 0xffffu) - bias + L * gap;
+          if (lane == 0) s.sink_score()[r] = h_last;
+          if (h_last > best) {
+            best = h_last;
+            best_row = r;
+            ties = 0;
+          } else if (h_last == best) {
+            ++ties;
+          }
+        }
+        record += row_bytes;
+      }
+    }
+  }
+  // (tracked under the live lanes' execution mask: uniform there)
+  *best_score = uniform(best);
+  *tied = uniform(ties) > 0;
+  return uniform(best_row);
+}
+
+__device__ __forceinline__ uint32_t from_prev_lane(uint32_t x) {
+  return static_cast<uint32_t>(
+      __builtin_amdgcn_update_dpp(0, static_cast<int>(x), 0x138, 0xf, 0xf, false));  // wave_shr:1
+}
+
+// Per-lane constants of the band rows: pair q holds strip columns
 // j0 + 2q (low half) and j0 + 2q + 1 (high half).
 template <int W>
 struct PackedStrip {
@@ -840,433 +1221,6 @@ __device__ __forceinline__ void packed_strip_init(PackedStrip<W>& ps, const uint
   ps.c4000 = 0x40004000u;
   asm volatile("" : "+v"(ps.c4000));
   ps.diff = pk_splat(mismatch - match);
-}
-
-// Predecessor row p (entry e) at the lane's strip as pairs of the row's
-// stored values G[p][j] = H[p][j] - j * gap: pp[q] = (G[p][j0 + 2q],
-// G[p][j0 + 2q + 1]); returns G[p][j0 - 1] in the low half. Row 0 is the
-// virtual start row (H = j * gap, so G = 0).
-template <int W>
-__device__ __forceinline__ uint32_t load_pairs(const int16_t* ring, int pitch, const Slot& s, int e,
-                                               int j0, int jq, int qs, int L, int32_t gap,
-                                               const PackedStrip<W>& ps, uint32_t* pp) {
-  const int p = e & kPredRowMask;
-  const int sl = static_cast<unsigned>(e) >> kPredRowBits;
-  if (p == 0) {
-#pragma unroll
-    for (int q = 0; q < W / 2; ++q) pp[q] = 0u;
-    return 0u;
-  } else if (sl < kSlotGlobal) {
-    const int16_t* row = ring + sl * pitch;
-#pragma unroll
-    for (int q = 0; q < W / 4; ++q) {
-      const uint2 v = *reinterpret_cast<const uint2*>(row + jq + q * qs);
-      pp[2 * q] = v.x;
-      pp[2 * q + 1] = v.y;
-    }
-    const uint32_t c0 = static_cast<uint16_t>(row[pitch - 1]);
-    const uint32_t prev = from_prev_lane(pp[W / 2 - 1]) >> 16;
-    return lane_id() == 0 ? c0 : prev;
-  } else {
-    const int32_t* row = s.H_row(p, pitch);
-    int32_t hv[W + 1];
-#pragma unroll
-    for (int u = 0; u <= W; ++u) {
-      const int j = j0 - 1 + u;
-      hv[u] = j <= L ? row[j] : 0;
-    }
-    wait_stores();
-#pragma unroll
-    for (int q = 0; q < W / 2; ++q) {
-      pp[q] = (static_cast<uint32_t>(hv[2 * q + 1]) & 0xffffu) |
-              (static_cast<uint32_t>(hv[2 * q + 2]) << 16);
-    }
-    return static_cast<uint32_t>(hv[0]);
-  }
-}
-
-// Scores and move codes of one packed row (registers only).
-template <int W>
-struct PackedOut {
-  uint32_t h[W / 2];
-  uint32_t cd[W / 2];
-  int32_t h0;  // column 0
-};
-
-template <int W, bool kMulti>
-__device__ __forceinline__ void packed_compute(const PackedStrip<W>& ps, const uint32_t* pp,
-                                               uint32_t hp0, const uint32_t* kk, uint32_t k0,
-                                               uint32_t b, uint32_t pay0, int lane, int32_t gap,
-                                               PackedOut<W>& o) {
-  constexpr int H2 = W / 2;
-  const uint32_t bb = b * 0x10001u;
-  // column 0 (hp0 + gap) heads lane 0's chain
-  o.h0 = pk_half(hp0 + static_cast<uint32_t>(gap), 0);
-  uint32_t carry = lane == 0 ? pk_splat(o.h0) : 0x80008000u;
-  uint32_t bd[H2], bv[H2], pre[H2];
-#pragma unroll
-  for (int q = 0; q < H2; ++q) {
-    // diagonal sources H[p][j - 1] of the pair
-    const uint32_t d = q == 0 ? ((pp[0] << 16) | (hp0 & 0xffffu))
-                              : __builtin_amdgcn_alignbit(pp[q], pp[q - 1], 16);
-    const uint32_t mis = pk_min_u(ps.base[q] ^ bb, ps.one);  // 1 where the bases differ
-    bd[q] = pk_mad(mis, ps.diff, pk_add(d, ps.match_gap));
-    bv[q] = pk_add(pp[q], ps.gap);
-    carry = pk_max_hi(pk_scan(pk_max(bd[q], bv[q])), carry);
-    pre[q] = carry;
-  }
-  const int32_t excl = wave_shift_right(wave_prefix_max(static_cast<int32_t>(carry) >> 16), -32768);
-#pragma unroll
-  for (int q = 0; q < H2; ++q) {
-    o.h[q] = pk_max_lo(pre[q], static_cast<uint32_t>(excl));
-    // diagonal first, then vertical, else horizontal, from 0/1 flags
-    // fd (not diagonal) and fv (not vertical)
-    const uint32_t fd = pk_min_u(pk_sub(o.h[q], bd[q]), ps.one);
-    const uint32_t fv = pk_min_u(pk_sub(o.h[q], bv[q]), ps.one);
-    if (kMulti) {
-      // codes of the first best predecessor: kCodeViaK | k
-      const uint32_t kd = q == 0 ? ((kk[0] << 16) | (k0 & 0xffffu))
-                                 : __builtin_amdgcn_alignbit(kk[q], kk[q - 1], 16);
-      const uint32_t dc = pk_add(kd, 0x20002000u);     // diagonal | kCodeViaK | k
-      const uint32_t vc = pk_add(kk[q], 0x60006000u);  // vertical | kCodeViaK | k
-      const uint32_t cv = pk_mad(fv, pk_sub(0x80008000u, vc), vc);
-      o.cd[q] = pk_mad(fd, pk_sub(cv, dc), dc);
-    } else {
-      // the move kind 2 fd + fv (both halves at once: no carries)
-      o.cd[q] = (fd << 1) | fv;
-    }
-    // computed here, not sunk into the store branch, so that a second row's
-    // scan can interleave with this row's codes
-    asm volatile("" : "+v"(o.cd[q]));
-  }
-}
-
-// Stores of one packed row (codes, the row's scores where later rows read
-// them) and H[row][L] as the return value.
-template <int W, bool kMulti>
-__device__ __forceinline__ int32_t packed_store(const PackedOut<W>& o, uint32_t k0, uint32_t pay0,
-                                                int lane, int j0, int jq, int qs, bool live, int L,
-                                                int32_t gap, int own, int pitch, int16_t* ring,
-                                                int32_t* Hg, uint16_t* Cr, int end_lane,
-                                                int end_u) {
-  constexpr int H2 = W / 2;
-  if (live) {
-    if (kMulti) {
-#pragma unroll
-      for (int q = 0; q < W / 4; ++q) {
-        *reinterpret_cast<uint2*>(Cr + (j0 - 1) + 4 * q) = make_uint2(o.cd[2 * q], o.cd[2 * q + 1]);
-      }
-    } else {
-      // move kinds, 2 bits per column: pair q's halves (columns 2q, 2q + 1
-      // of the strip) go to bits 4q and 4q + 2
-      auto pack8 = [&](int g) -> uint32_t {  // pairs 4g..4g+3: 16 bits
-        uint32_t x = o.cd[min(4 * g, H2 - 1)];
-#pragma unroll
-        for (int q = 1; q < 4; ++q) x |= o.cd[min(4 * g + q, H2 - 1)] << (4 * q);
-        return (x & 0xffffu) | (x >> 14);
-      };
-      uint8_t* K = reinterpret_cast<uint8_t*>(Cr) + (j0 - 1) / 4;
-      if constexpr (W == 4) {
-        const uint32_t x = o.cd[0] | (o.cd[1] << 4);
-        *K = static_cast<uint8_t>(x | (x >> 14));
-      } else if constexpr (W == 8) {
-        *reinterpret_cast<uint16_t*>(K) = static_cast<uint16_t>(pack8(0));
-      } else if constexpr (W == 12) {
-        const uint32_t v = pack8(0);
-        const uint32_t x = o.cd[4] | (o.cd[5] << 4);
-        K[0] = static_cast<uint8_t>(v);
-        K[1] = static_cast<uint8_t>(v >> 8);
-        K[2] = static_cast<uint8_t>(x | (x >> 14));
-      } else {
-        *reinterpret_cast<uint32_t*>(K) = pack8(0) | (pack8(1) << 16);
-      }
-    }
-    if (own < kSlotGlobal) {
-      int16_t* row = ring + own * pitch;
-#pragma unroll
-      for (int q = 0; q < W / 4; ++q) {
-        *reinterpret_cast<uint2*>(row + jq + q * qs) = make_uint2(o.h[2 * q], o.h[2 * q + 1]);
-      }
-    }
-  }
-  if (own == kSlotGlobal) {
-#pragma unroll
-    for (int u = 0; u < W; ++u) {
-      if (j0 + u <= L) Hg[j0 + u] = pk_half(o.h[u / 2], u & 1);
-    }
-  }
-  if (lane == 0) {
-    if (own < kSlotGlobal) ring[own * pitch + pitch - 1] = static_cast<int16_t>(o.h0);
-    if (own == kSlotGlobal) Hg[0] = o.h0;
-    if (kMulti) Cr[pitch - 1] = static_cast<uint16_t>(kCodeVert | kCodeViaK | (k0 & 0xffffu));
-  }
-  // (each pair opaque, so that the selection stays register selects rather
-  // than an indexed load from a stack copy of the row)
-  uint32_t lastp = o.h[0];
-#pragma unroll
-  for (int q = 1; q < H2; ++q) {
-    uint32_t v = o.h[q];
-    asm volatile("" : "+v"(v));
-    if (q == (end_u >> 1)) lastp = v;
-  }
-  return __builtin_amdgcn_readlane(pk_half(lastp, end_u & 1), end_lane) + L * gap;
-}
-
-// One DP row in packed pairs: the moves, codes, stores and end-column value
-// of finish_row, two columns per instruction. pp holds the predecessor
-// scores at the strip's columns and hp0 (low half) the one at column j0 - 1.
-// With one predecessor (kMulti false) every diagonal and vertical move names
-// it through pay0. With several, pp and hp0 hold the best predecessor score
-// of each column and kk, k0 the first predecessor k (in-edge order) that
-// reaches it: the diagonal into column j and the vertical into column j - 1
-// both take the first predecessor with the best H[p][j - 1], which is the
-// predecessor spoa's traceback prefers. Every value is kept as
-// G = H - j * gap (the rows in LDS or global memory too): a horizontal move
-// keeps G, a vertical one adds gap and a diagonal one adds s - gap, so the
-// horizontal chain is a plain prefix max, and every value of a live column
-// lies within max_abs * (V + 2L + 2) of zero; the caller takes this path only
-// when that fits 16 bits. Columns past L compute unused values (they flow
-// only into later columns). Returns H[row][L].
-template <int W, bool kMulti>
-__device__ __forceinline__ int32_t packed_row(const PackedStrip<W>& ps, const uint32_t* pp,
-                                              uint32_t hp0, const uint32_t* kk, uint32_t k0,
-                                              uint32_t b, uint32_t pay0, int lane,
-                                              int j0, int jq, int qs, bool live, int L,
-                                              int32_t gap, int own, int pitch, int16_t* ring,
-                                              int32_t* Hg, uint16_t* Cr, int end_lane,
-                                              int end_u) {
-  PackedOut<W> o;
-  packed_compute<W, kMulti>(ps, pp, hp0, kk, k0, b, pay0, lane, gap, o);
-  return packed_store<W, kMulti>(o, k0, pay0, lane, j0, jq, qs, live, L, gap, own, pitch, ring,
-                                 Hg, Cr, end_lane, end_u);
-}
-
-// DP rows of one layer with 16-bit scores, every row in one pass of the
-// wave: lane k owns columns 1 + kW .. (k + 1)W (W = 4, 8, 12, or 16 when
-// packed, so that 64W >= L), the layer bytes of its strip stay in
-// registers, and column 0 heads lane 0's horizontal chain. Same moves,
-// codes and end cell as
-// dp_layer. Requires in-degree <= 255, 64W + pad <= pitch and 16-bit scores
-// over the whole strip. With kPacked every row runs in packed 16-bit pairs
-// (packed_row; a row with several predecessors first folds them with a
-// packed max and first argmax), which needs max_abs * (V + 2L + 2) in 16
-// bits. Without it (W <= 12), rows with one predecessor take no argmax and
-// rows with several keep (score, 255 - k) in one integer so that one max
-// keeps the first predecessor with the best score (in-edge order, as spoa's
-// traceback prefers).
-template <int W, bool kPacked>
-__device__ __forceinline__ int dp_layer_strip(CParams& P, const Slot& s, uint8_t* lds, int V, int L,
-                              int* best_score, bool* tied) {
-  static_assert(W % 4 == 0 && W >= 4 && W <= (kPacked ? 16 : 12), "strip width");
-  const int lane = lane_id();
-  const int pitch = static_cast<int>(P.caps.cols);
-  // scores as uniform registers (a select between two parameter fields
-  // would otherwise become a per-lane load from the selected address)
-  const int32_t gap = uniform(P.gap);
-  const int32_t match = uniform(P.match);
-  const int32_t mismatch = uniform(P.mismatch);
-  int16_t* ring = reinterpret_cast<int16_t*>(lds);
-  const uint8_t* seq = lds + align_up(static_cast<uint64_t>(P.ring_rows) * pitch * 2, 16);
-  const int j0 = 1 + lane * W;
-  const bool live = j0 <= L;
-  const int jr = live ? j0 : 1;  // idle lanes read columns 0..W (in bounds)
-  // quad-major LDS rows (see from_prev_lane): this lane's first quad and the
-  // quad stride; idle lanes read lane 0's quads
-  const int n_live = (L + W - 1) / W;
-  const int jq = (live ? lane : 0) * 4;
-  const int qs = n_live * 4;
-  uint32_t sw[W / 4];            // layer bytes of the strip
-#pragma unroll
-  for (int q = 0; q < W / 4; ++q) sw[q] = *reinterpret_cast<const uint32_t*>(seq + (jr - 1) + 4 * q);
-  PackedStrip<W> ps;
-  if (kPacked) packed_strip_init<W>(ps, sw, j0, match, mismatch, gap);
-  const int end_lane = (L - 1) / W;
-  const int end_u = (L - 1) % W;
-  int32_t best = kNegInf;
-  int best_row = 0;
-  int ties = 0;
-  const int total_preds = uniform(s.pred_off()[V]);
-  // sink rows: record the end-column score and keep the best (in row order)
-  auto account = [&](int32_t h, int row, int m) {
-    if ((m & kRowMetaSink) != 0) {
-      if (lane == 0) {
-        s.sink_score()[row] = h;
-      }
-      if (h > best) {
-        best = h;
-        best_row = row;
-        ties = 0;
-      } else if (h == best) {
-        ++ties;
-      }
-    }
-  };
-  for (int r0 = 1; r0 <= V; r0 += kWave) {
-    const int rk = r0 + lane;
-    int off_v = 0, end_v = 0, meta_v = 0;
-    if (rk <= V) {
-      off_v = s.pred_off()[rk - 1];
-      end_v = s.pred_off()[rk];
-      meta_v = s.row_meta()[rk - 1];
-    }
-    const int base = __builtin_amdgcn_readlane(off_v, 0);
-    const int pr0 = base + lane < total_preds ? s.pred_rows()[base + lane] : 0;
-    const int pr1 = base + kWave + lane < total_preds ? s.pred_rows()[base + kWave + lane] : 0;
-    // (up to four entries per row of the chunk without a reload)
-    const int pr2 =
-        base + 2 * kWave + lane < total_preds ? s.pred_rows()[base + 2 * kWave + lane] : 0;
-    const int pr3 =
-        base + 3 * kWave + lane < total_preds ? s.pred_rows()[base + 3 * kWave + lane] : 0;
-    // complete the chunk's loads here: otherwise the row loop would wait for
-    // them (and for every code store issued before them) on each row
-    wait_stores();
-    const int chunk = min(kWave, V - r0 + 1);
-    for (int rr = 0; rr < chunk; ++rr) {
-      const int r = r0 + rr;
-      const int off = __builtin_amdgcn_readlane(off_v, rr);
-      const int np = __builtin_amdgcn_readlane(end_v, rr) - off;
-      const int meta = __builtin_amdgcn_readlane(meta_v, rr);
-      auto pred_of = [&](int o, int k) -> int {
-        const int idx = o + k - base;
-        if (idx < kWave) return __builtin_amdgcn_readlane(pr0, idx);
-        if (idx < 2 * kWave) return __builtin_amdgcn_readlane(pr1, idx - kWave);
-        if (idx < 3 * kWave) return __builtin_amdgcn_readlane(pr2, idx - 2 * kWave);
-        if (idx < 4 * kWave) return __builtin_amdgcn_readlane(pr3, idx - 3 * kWave);
-        const int e = uniform(s.pred_rows()[o + k]);
-        wait_stores();
-        return e;
-      };
-      auto pred_at = [&](int k) -> int { return pred_of(off, k); };
-      const uint32_t b = static_cast<uint32_t>(meta & 0xff);
-      const int own = (meta >> kRowMetaSlotShift) & 31;
-      int32_t* Hg = s.H_row(r, meta, pitch);
-      uint16_t* Cr = s.code() + static_cast<int64_t>(r) * pitch;
-      // match score of strip column u against the row's base
-      auto sc = [&](int u) -> int32_t {
-        return ((sw[u / 4] >> (8 * (u % 4))) & 0xffu) == b ? match : mismatch;
-      };
-      int32_t bd[W], bv[W];
-      int32_t h_last = 0;
-      // the row the common tail below accounts for (the second of a pair)
-      int tail_row = r, tail_meta = meta, tail_own = own;
-      if (kPacked && np == 1) {
-        const int e = pred_at(0);
-        const uint32_t delta = static_cast<uint32_t>(r - (e & kPredRowMask));
-        const uint32_t pay0 = delta <= kCodePayload ? delta : kCodeViaK;
-        // The next row as well when it has one predecessor other than this
-        // row and neither row keeps its scores in global memory: the rows
-        // are independent, so both loads go out before either row's
-        // arithmetic and the two rows' instructions interleave. (This row's
-        // LDS slot holds no row the next one reads: a slot is reused only
-        // after the last reader of its row.)
-        bool paired = false;
-        if (W <= 12 && rr + 1 < chunk && own != kSlotGlobal) {  // (16 would spill)
-          const int off2 = __builtin_amdgcn_readlane(off_v, rr + 1);
-          const int np2 = __builtin_amdgcn_readlane(end_v, rr + 1) - off2;
-          const int meta2 = __builtin_amdgcn_readlane(meta_v, rr + 1);
-          const int own2 = (meta2 >> kRowMetaSlotShift) & 31;
-          if (np2 == 1 && own2 != kSlotGlobal) {
-            const int e2 = pred_of(off2, 0);
-            if ((e2 & kPredRowMask) != r) {
-              paired = true;
-              const uint32_t delta2 = static_cast<uint32_t>(r + 1 - (e2 & kPredRowMask));
-              const uint32_t pay2 = delta2 <= kCodePayload ? delta2 : kCodeViaK;
-              uint32_t pa[W / 2], pb[W / 2];
-              const uint32_t ha0 = load_pairs<W>(ring, pitch, s, e, j0, jq, qs, L, gap, ps, pa);
-              const uint32_t hb0 = load_pairs<W>(ring, pitch, s, e2, j0, jq, qs, L, gap, ps, pb);
-              PackedOut<W> oa, ob;
-              packed_compute<W, false>(ps, pa, ha0, pa, 0u, b, pay0, lane, gap, oa);
-              packed_compute<W, false>(ps, pb, hb0, pb, 0u, static_cast<uint32_t>(meta2 & 0xff),
-                                       pay2, lane, gap, ob);
-              const int32_t h_a = packed_store<W, false>(oa, 0u, pay0, lane, j0, jq, qs, live, L, gap,
-                                                         own, pitch, ring, Hg, Cr, end_lane,
-                                                         end_u);
-              h_last = packed_store<W, false>(ob, 0u, pay2, lane, j0, jq, qs, live, L, gap, own2, pitch,
-                                              ring, s.H_row(r + 1, meta2, pitch),
-                                              s.code() + static_cast<int64_t>(r + 1) * pitch,
-                                              end_lane, end_u);
-              account(h_a, r, meta);
-              tail_row = r + 1;
-              tail_meta = meta2;
-              tail_own = own2;
-              ++rr;
-            }
-          }
-        }
-        if (!paired) {
-          uint32_t pp[W / 2];
-          const uint32_t hp0 = load_pairs<W>(ring, pitch, s, e, j0, jq, qs, L, gap, ps, pp);
-          h_last = packed_row<W, false>(ps, pp, hp0, pp, 0u, b, pay0, lane, j0, jq, qs, live, L, gap,
-                                        own, pitch, ring, Hg, Cr, end_lane, end_u);
-        }
-      } else if (kPacked) {
-        // best predecessor score of every column and the first predecessor
-        // reaching it (a later one replaces it only when strictly better)
-        uint32_t mx[W / 2], kx[W / 2];
-        uint32_t m0 = load_pairs<W>(ring, pitch, s, pred_at(0), j0, jq, qs, L, gap, ps, mx);
-        uint32_t k0 = 0;
-#pragma unroll
-        for (int q = 0; q < W / 2; ++q) kx[q] = 0;
-        for (int k = 1; k < np; ++k) {
-          uint32_t pp[W / 2];
-          const uint32_t hk = load_pairs<W>(ring, pitch, s, pred_at(k), j0, jq, qs, L, gap, ps, pp);
-          const uint32_t ks = static_cast<uint32_t>(k) * 0x10001u;
-#pragma unroll
-          for (int q = 0; q < W / 2; ++q) {
-            const uint32_t m = pk_max(mx[q], pp[q]);
-            kx[q] = pk_mad(pk_min_u(pk_sub(m, mx[q]), ps.one), pk_sub(ks, kx[q]), kx[q]);
-            mx[q] = m;
-          }
-          const uint32_t m = pk_max(m0, hk);
-          k0 = pk_mad(pk_min_u(pk_sub(m, m0), ps.one), pk_sub(ks, k0), k0);
-          m0 = m;
-        }
-        h_last = packed_row<W, true>(ps, mx, m0, kx, k0, b, 0u, lane, j0, jq, qs, live, L, gap, own, pitch,
-                                     ring, Hg, Cr, end_lane, end_u);
-      } else if (np == 1) {
-        // move-code payload of the single predecessor: its row delta
-        const uint32_t delta = static_cast<uint32_t>(r - (pred_at(0) & kPredRowMask));
-        const uint32_t pay0 = delta <= kCodePayload ? delta : kCodeViaK;
-        int32_t hp[W + 1];
-        load_strip<W>(ring, pitch, s, pred_at(0), j0, jq, qs, L, gap, hp);
-#pragma unroll
-        for (int u = 0; u < W; ++u) {
-          bd[u] = hp[u] + sc(u);
-          bv[u] = hp[u + 1] + gap;
-        }
-        h_last = finish_row<W, false>(bd, bv, hp[0] + gap, pay0, lane, j0, jq, qs, live, L, gap, own,
-                                      pitch, ring, Hg, Cr, end_lane, end_u);
-      } else {
-        int32_t c0k = kNegKey;
-#pragma unroll
-        for (int u = 0; u < W; ++u) {
-          bd[u] = kNegKey;
-          bv[u] = kNegKey;
-        }
-        for (int k = 0; k < np; ++k) {
-          int32_t hp[W + 1];
-          load_strip<W>(ring, pitch, s, pred_at(k), j0, jq, qs, L, gap, hp);
-          const int32_t tag = 255 - k;
-#pragma unroll
-          for (int u = 0; u < W; ++u) {
-            bd[u] = max(bd[u], (hp[u] + sc(u)) * 256 | tag);
-            bv[u] = max(bv[u], (hp[u + 1] + gap) * 256 | tag);
-          }
-          c0k = max(c0k, (hp[0] + gap) * 256 | tag);
-        }
-        h_last = finish_row<W, true>(bd, bv, c0k, 0u, lane, j0, jq, qs, live, L, gap, own, pitch, ring,
-                                     Hg, Cr, end_lane, end_u);
-      }
-      account(h_last, tail_row, tail_meta);
-      if (tail_own == kSlotGlobal) {
-        wait_stores();
-      }
-      wave_fence();
-    }
-  }
-  *best_score = best;
-  *tied = ties > 0;
-  return best_row;
 }
 
 // ---- banded rows: the opt-in approximation of racon -b ----
@@ -1536,13 +1490,11 @@ __device__ __forceinline__ T* uniform_ptr(T* p) {
 }
 
 enum DpKind : int {
-  kDpStrip4,
-  kDpStrip8,
-  kDpStrip12,
-  kDpPacked4,
-  kDpPacked8,
-  kDpPacked12,
-  kDpPacked16,
+  kDpRows4,
+  kDpRows8,
+  kDpRows12,
+  kDpRows16,
+  kDpRows20,
   kDpGeneric16,
   kDpGeneric32,
   kDpBand4
@@ -1552,38 +1504,34 @@ enum DpKind : int {
 // allocation of their own instead of sharing one with the rest of the window
 // loop. Arguments arrive in vector registers and are made uniform again on
 // entry. Returns the end-cell row, its score and whether sinks tied.
-typedef __attribute__((address_space(3))) uint8_t LByte;
-
 template <int kKind>
 __device__ __noinline__ uint64_t dp_layer_call(CParams* params, GByte* base, CLayout* layout,
-                                               uint32_t lds_addr, int V, int L) {
+                                               uint32_t lds_addr, int V, int L, int bias) {
   CParams& P = *uniform_ptr(params);
   Slot s = carve(uniform_ptr(base), *uniform_ptr(layout));
   V = uniform(V);
   L = uniform(L);
+  bias = uniform(bias);
   // the wave's LDS as a local-memory pointer from the caller (no lookup of
   // the dynamic LDS offset inside the loops)
-  uint8_t* lds = (uint8_t*)(LByte*)(size_t)__builtin_amdgcn_readfirstlane(lds_addr);
+  lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);
+  [[maybe_unused]] uint8_t* lds = (uint8_t*)(LByte*)(size_t)lds_addr;
   int best_score = 0;
   bool tied = false;
   int row;
-  if (kKind == kDpStrip4) {
-    row = dp_layer_strip<4, false>(P, s, lds, V, L, &best_score, &tied);
-  } else if (kKind == kDpStrip8) {
-    row = dp_layer_strip<8, false>(P, s, lds, V, L, &best_score, &tied);
-  } else if (kKind == kDpStrip12) {
-    row = dp_layer_strip<12, false>(P, s, lds, V, L, &best_score, &tied);
-  } else if (kKind == kDpPacked4) {
-    row = dp_layer_strip<4, true>(P, s, lds, V, L, &best_score, &tied);
-  } else if (kKind == kDpPacked8) {
-    row = dp_layer_strip<8, true>(P, s, lds, V, L, &best_score, &tied);
-  } else if (kKind == kDpPacked12) {
-    row = dp_layer_strip<12, true>(P, s, lds, V, L, &best_score, &tied);
-  } else if (kKind == kDpPacked16) {
-    row = dp_layer_strip<16, true>(P, s, lds, V, L, &best_score, &tied);
-  } else if (kKind == kDpBand4) {
+  if constexpr (kKind == kDpRows4) {
+    row = dp_rows<4>(P, s, lds_addr, V, L, bias, &best_score, &tied);
+  } else if constexpr (kKind == kDpRows8) {
+    row = dp_rows<8>(P, s, lds_addr, V, L, bias, &best_score, &tied);
+  } else if constexpr (kKind == kDpRows12) {
+    row = dp_rows<12>(P, s, lds_addr, V, L, bias, &best_score, &tied);
+  } else if constexpr (kKind == kDpRows16) {
+    row = dp_rows<16>(P, s, lds_addr, V, L, bias, &best_score, &tied);
+  } else if constexpr (kKind == kDpRows20) {
+    row = dp_rows<20>(P, s, lds_addr, V, L, bias, &best_score, &tied);
+  } else if constexpr (kKind == kDpBand4) {
     row = dp_layer_band(P, s, lds, V, L, &best_score, &tied);
-  } else if (kKind == kDpGeneric16) {
+  } else if constexpr (kKind == kDpGeneric16) {
     row = dp_layer<int16_t>(P, s, lds, V, L, &best_score, &tied);
   } else {
     row = dp_layer<int32_t>(P, s, lds, V, L, &best_score, &tied);
@@ -2055,7 +2003,7 @@ __device__ __noinline__ int build_rows(GByte* slot_base, CLayout* layout, int V,
   int32_t* row_meta = s.row_meta();
   int32_t* pred_off = s.pred_off();
   int32_t* pred_rows = s.pred_rows();
-  uint64_t* row_pred4 = s.row_pred4();
+  uint4* row_rec = s.row_rec();
   auto included = [&](int v) { return kFull || in_sub[v] != 0; };
   // predecessor entry of DP row pr: the row and the slot it lives in
   auto pred_entry = [&](int pr) {
@@ -2073,7 +2021,7 @@ __device__ __noinline__ int build_rows(GByte* slot_base, CLayout* layout, int V,
   int pool1 = lane + kWave < hpool ? 0 : 0x7fffffff;
   bool pool_full = false;
   for (int r0 = 0; r0 < V; r0 += kU * kWave) {
-    int v[kU], ei[kU], eo[kU], np[kU], oc[kU], lu[kU], meta[kU], off[kU];
+    int v[kU], ei[kU], eo[kU], np[kU], oc[kU], lu[kU], meta[kU], off[kU], slot[kU];
     int pr[kU][kP];
 #pragma unroll
     for (int i = 0; i < kU; ++i) {
@@ -2185,6 +2133,7 @@ __device__ __noinline__ int build_rows(GByte* slot_base, CLayout* layout, int V,
         pred_off[r] = off[i];
         if (slots_in_lds) lslot[r] = static_cast<uint8_t>(my_slot);
       }
+      slot[i] = my_slot;
       run += __builtin_amdgcn_readlane(x, kWave - 1);
     }
     // predecessor entries (their slots are all assigned by now: predecessor
@@ -2194,6 +2143,16 @@ __device__ __noinline__ int build_rows(GByte* slot_base, CLayout* layout, int V,
       if (v[i] < 0) continue;
       const int r = r0 + i * kWave + lane;
       uint64_t deltas = 0;  // row deltas of the first four predecessors (0: none or too far)
+      // the row descriptor of dp_rows: stays in the general form (no
+      // predecessor count) unless every condition below holds
+      const int letter = meta[i] & 0xff;
+      const int code = ((letter >> 1) ^ (letter >> 2)) & 3;
+      uint32_t desc = (meta[i] & kRowMetaSink) != 0 ? kRecSink : 0u;
+      bool fast = np[i] >= 1 && np[i] <= static_cast<int>(kRecMaxPreds) && slot[i] != kSlotGlobal &&
+                  static_cast<int>((0x54474341u >> (8 * code)) & 0xffu) == letter;
+      uint32_t fields = static_cast<uint32_t>(np[i]) | static_cast<uint32_t>(code << 3) |
+                        static_cast<uint32_t>(slot[i]) << kRecOwnShift;
+      if (np[i] == 1 && pr[i][0] == r) fields |= kRecChain;
       if (np[i] == 0) {
         pred_rows[off[i]] = 0;
         deltas = static_cast<uint64_t>(r + 1 <= 0xffff ? r + 1 : 0);
@@ -2201,9 +2160,13 @@ __device__ __noinline__ int build_rows(GByte* slot_base, CLayout* layout, int V,
 #pragma unroll
         for (int j = 0; j < kP; ++j) {
           if (j < np[i]) {
-            pred_rows[off[i] + j] = pred_entry(pr[i][j]);
+            const int entry = pred_entry(pr[i][j]);
+            const uint32_t sl = static_cast<uint32_t>(entry) >> kPredRowBits;
+            fast = fast && sl < static_cast<uint32_t>(kSlotGlobal);
+            if (j < static_cast<int>(kRecMaxPreds)) fields |= sl << (kRecPredShift + 5 * j);
+            pred_rows[off[i] + j] = entry;
             const int d = r + 1 - pr[i][j];
-            if (d <= 0xffff) deltas |= static_cast<uint64_t>(d) << (16 * j);
+            if (j < 4 && d <= 0xffff) deltas |= static_cast<uint64_t>(d) << (16 * j);
           }
         }
       } else {
@@ -2220,7 +2183,9 @@ __device__ __noinline__ int build_rows(GByte* slot_base, CLayout* layout, int V,
           }
         }
       }
-      row_pred4[r] = deltas;
+      if (fast) desc |= fields;
+      row_rec[r] = make_uint4(desc, static_cast<uint32_t>(v[i]), static_cast<uint32_t>(deltas),
+                              static_cast<uint32_t>(deltas >> 32));
     }
   }
   if (lane == 0) {
@@ -2229,8 +2194,6 @@ __device__ __noinline__ int build_rows(GByte* slot_base, CLayout* layout, int V,
   if (pool_full) return -1;
   return __builtin_amdgcn_readlane(wave_prefix_max(max_np), kWave - 1);
 }
-
-typedef __attribute__((address_space(3))) uint32_t LWord;
 
 // Included nodes of a layer that does not span the window (spoa
 // Graph::subgraph's walk): the nodes >= begin that reach `end` backwards
@@ -2609,14 +2572,17 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
     }
     // layer bytes and weights into the slot
     uint8_t* lds_seq = lds + align_up(static_cast<uint64_t>(P.ring_rows) * pitch * 2, 16);
+    bool plain = true;  // A, C, G and T only
     for (int j = lane; j < L; j += kWave) {
       const uint8_t c = arena[Lr.seq_off + j];
       s.seq()[j] = c;
       lds_seq[j] = c;
+      plain &= c == 'A' || c == 'C' || c == 'G' || c == 'T';
       s.qual()[j] = Lr.qual_off == kNoQuality
                       ? 1
                       : static_cast<int>(arena[Lr.qual_off + j]) - 33;
     }
+    const bool layer_plain = __all(plain);
     const bool full = Lr.begin < W.offset && Lr.end > W.backbone_len - W.offset;
     if (static_cast<int>(Lr.end) >= s.n_nodes || Lr.begin > Lr.end) {
       R.status = kPoaBadInput;
@@ -2709,11 +2675,13 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
     // score width: 16-bit ring rows when every score of the layer fits
     const int32_t max_abs = max(max(abs(P.match), abs(P.mismatch)), abs(P.gap));
     const bool narrow = static_cast<int64_t>(max_abs) * (V + L + 2) < 32000;
+    // the packed one-pass rows (dp_rows) hold the layer
+    int bias = 0;
+    const bool rows16 = L >= 1 && L < 20 * kWave &&
+                        rows_fit_16(P.match, P.mismatch, P.gap, V, L, &bias);
     // (a pass for very long layers may keep no rows in LDS at all)
-    const int n_slots = min(kMaxLdsSlots, narrow ? static_cast<int>(P.ring_rows)
+    const int n_slots = min(kMaxLdsSlots, narrow || rows16 ? static_cast<int>(P.ring_rows)
                                                  : static_cast<int>(P.ring_rows) / 2);
-
-    bool strip_ok = false;  // the one-pass DP applies (dp_layer_strip)
 
     // predecessor rows, sink flags, slots
     uint32_t rows_lds = static_cast<uint32_t>((size_t)(LByte*)lds);
@@ -2727,7 +2695,6 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
       R.status = kPoaRowOverflow;  // the pooled global rows ran out: rerun exactly
       return;
     }
-    strip_ok = narrow && L >= 1 && max_abs <= 4096 && max_np <= 255;
     if (max_np > static_cast<int>(kCodePayload) + 1) {
       // a move code holds the in-edge index in 13 bits
       R.status = kPoaInDegree;
@@ -2746,30 +2713,29 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
     // opaque to the optimizer: otherwise the callee would rebuild the address
     // from the dynamic LDS symbol (a table load) inside its loops
     asm volatile("" : "+v"(lds_addr));
-    // packed pairs keep H - j * gap in 16 bits
-    const bool packed = strip_ok && static_cast<int64_t>(max_abs) * (V + 2 * L + 2) < 32000;
-    // racon -b: band rows for layers longer than the band (approximation)
-    const bool banded = packed && P.band != 0 && L > kBand;
+    // racon -b: band rows for layers longer than the band (approximation);
+    // their pairs keep H - j * gap in signed 16 bits
+    const bool banded = P.band != 0 && L > kBand && max_abs <= 4096 && max_np <= 255 &&
+                        static_cast<int64_t>(max_abs) * (V + 2 * L + 2) < 32000;
+    // columns per lane of the packed rows
+    const int row_w = L < 4 * kWave ? 4 : L < 8 * kWave ? 8 : L < 12 * kWave ? 12
+                      : L < 16 * kWave ? 16 : 20;
     if (banded) {
-      dp = dp_layer_call<kDpBand4>(pp, s.p, ly, lds_addr, V, L);
-    } else if (packed && L <= 4 * kWave) {
-      dp = dp_layer_call<kDpPacked4>(pp, s.p, ly, lds_addr, V, L);
-    } else if (packed && L <= 8 * kWave) {
-      dp = dp_layer_call<kDpPacked8>(pp, s.p, ly, lds_addr, V, L);
-    } else if (packed && L <= 12 * kWave) {
-      dp = dp_layer_call<kDpPacked12>(pp, s.p, ly, lds_addr, V, L);
-    } else if (packed && L <= 16 * kWave) {
-      dp = dp_layer_call<kDpPacked16>(pp, s.p, ly, lds_addr, V, L);
-    } else if (strip_ok && L <= 4 * kWave) {
-      dp = dp_layer_call<kDpStrip4>(pp, s.p, ly, lds_addr, V, L);
-    } else if (strip_ok && L <= 8 * kWave) {
-      dp = dp_layer_call<kDpStrip8>(pp, s.p, ly, lds_addr, V, L);
-    } else if (strip_ok && L <= 12 * kWave) {
-      dp = dp_layer_call<kDpStrip12>(pp, s.p, ly, lds_addr, V, L);
+      dp = dp_layer_call<kDpBand4>(pp, s.p, ly, lds_addr, V, L, 0);
+    } else if (rows16 && row_w == 4) {
+      dp = dp_layer_call<kDpRows4>(pp, s.p, ly, lds_addr, V, L, bias);
+    } else if (rows16 && row_w == 8) {
+      dp = dp_layer_call<kDpRows8>(pp, s.p, ly, lds_addr, V, L, bias);
+    } else if (rows16 && row_w == 12) {
+      dp = dp_layer_call<kDpRows12>(pp, s.p, ly, lds_addr, V, L, bias);
+    } else if (rows16 && row_w == 16) {
+      dp = dp_layer_call<kDpRows16>(pp, s.p, ly, lds_addr, V, L, bias);
+    } else if (rows16) {
+      dp = dp_layer_call<kDpRows20>(pp, s.p, ly, lds_addr, V, L, bias);
     } else if (narrow) {
-      dp = dp_layer_call<kDpGeneric16>(pp, s.p, ly, lds_addr, V, L);
+      dp = dp_layer_call<kDpGeneric16>(pp, s.p, ly, lds_addr, V, L, 0);
     } else {
-      dp = dp_layer_call<kDpGeneric32>(pp, s.p, ly, lds_addr, V, L);
+      dp = dp_layer_call<kDpGeneric32>(pp, s.p, ly, lds_addr, V, L, 0);
     }
     int best_row = uniform(static_cast<int>(static_cast<uint32_t>(dp) & 0x7fffffffu));
     best_score = uniform(static_cast<int>(dp >> 32));
@@ -2826,13 +2792,15 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
     // j0 - 1 - t) and stored together.
     {
       const uint16_t* code = s.code();
-      const int32_t* sub_order = s.sub_order();
       const int32_t* pred_off = s.pred_off();
       const int32_t* pred_rows = s.pred_rows();
-      const uint64_t* row_pred4 = s.row_pred4();
+      const uint4* row_rec = s.row_rec();
       const int32_t* row_meta = s.row_meta();
-      // the packed DP and the band rows keep move kinds for one-predecessor rows
-      const bool kinds = banded || (packed && L <= 16 * kWave);
+      // the packed rows keep move records, the band rows move kinds for rows
+      // with one predecessor
+      const bool records = rows16 && !banded;
+      const int record_half = row_record_bytes(row_w) / 2;
+      const int row_inv = 65536 / row_w + 1;
       int32_t* pos_node = s.path();
       constexpr uint32_t kNextExit = 0xff;  // successor: the decoder takes the move
       constexpr uint32_t kDiagBit = 0x100;
@@ -2854,24 +2822,55 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
         const int cj = j0 - 2 * (lane & 3);
         const uint16_t* crow = code + static_cast<int64_t>(rc) * pitch;
         uint32_t c0, c1;
-        if (kinds && (row_meta[rc - 1] & kRowMetaSingle) != 0) {
-          // a one-predecessor row of the packed DP: its 2-bit move kinds,
-          // turned into the codes of moves to in-edge 0
-          const uint8_t* krow = reinterpret_cast<const uint8_t*>(crow);
-          auto kind_code = [&](int j) -> uint32_t {
-            if (j <= 0) return kCodeVert | kCodeViaK;
-            const uint32_t k = (static_cast<uint32_t>(krow[(j - 1) >> 2]) >> (2 * ((j - 1) & 3))) & 3u;
-            return k == kKindHorz ? kCodeHorz
-                                  : ((k == kKindVert ? kCodeVert : kCodeDiag) | kCodeViaK);
+        uint4 rec;  // descriptor, graph node, first four predecessor row deltas
+        if (records) {
+          // the row's record and both halves of its move record in one round
+          // trip: kinds of columns cj and cj - 1, predecessor indices of
+          // cj, cj - 1 and cj - 2
+          const uint8_t* mrow = reinterpret_cast<const uint8_t*>(crow);
+          const RecordBit b0 = record_bit(max(cj, 0), row_w, row_inv);
+          const RecordBit b1 = record_bit(max(cj - 1, 0), row_w, row_inv);
+          const RecordBit b2 = record_bit(max(cj - 2, 0), row_w, row_inv);
+          rec = row_rec[rc - 1];
+          const uint32_t m0 = mrow[b0.byte], m1 = mrow[b1.byte];
+          const uint32_t x0 = mrow[b0.byte + record_half], x1 = mrow[b1.byte + record_half];
+          const uint32_t x2 = mrow[b2.byte + record_half];
+          const uint32_t k0 = (x0 >> b0.bit) & 3u, k1 = (x1 >> b1.bit) & 3u;
+          const uint32_t k2 = (x2 >> b2.bit) & 3u;
+          auto move_code = [&](uint32_t kind, uint32_t above, uint32_t left) -> uint32_t {
+            return (kind & 2u) != 0   ? (kCodeDiag | kCodeViaK | left)
+                   : (kind & 1u) != 0 ? (kCodeVert | kCodeViaK | above)
+                                      : static_cast<uint32_t>(kCodeHorz);
           };
-          c0 = kind_code(cj);
-          c1 = kind_code(cj - 1);
+          c0 = move_code((m0 >> b0.bit) & 3u, k0, k1);
+          c1 = move_code((m1 >> b1.bit) & 3u, k1, k2);
+          if (!layer_plain || (rec.x & kRecPreds) == 0) {
+            // a row of the general form: 16-bit codes
+            c0 = crow[max(cj, 0)];
+            c1 = crow[max(cj - 1, 0)];
+          }
         } else {
-          c0 = crow[code_index(max(cj, 0), pitch)];
-          c1 = crow[code_index(max(cj - 1, 0), pitch)];
+          rec = row_rec[rc - 1];
+          if (banded && (row_meta[rc - 1] & kRowMetaSingle) != 0) {
+            // a one-predecessor band row: its 2-bit move kinds, turned into
+            // the codes of moves to in-edge 0
+            const uint8_t* krow = reinterpret_cast<const uint8_t*>(crow);
+            auto kind_code = [&](int j) -> uint32_t {
+              if (j <= 0) return kCodeVert | kCodeViaK;
+              const uint32_t k =
+                  (static_cast<uint32_t>(krow[(j - 1) >> 2]) >> (2 * ((j - 1) & 3))) & 3u;
+              return k == kKindHorz ? kCodeHorz
+                                    : ((k == kKindVert ? kCodeVert : kCodeDiag) | kCodeViaK);
+            };
+            c0 = kind_code(cj);
+            c1 = kind_code(cj - 1);
+          } else {
+            c0 = crow[code_index(max(cj, 0), pitch)];
+            c1 = crow[code_index(max(cj - 1, 0), pitch)];
+          }
         }
-        const uint64_t d4 = row_pred4[rc - 1];  // first four predecessor row deltas of the row
-        const int nrow = sub_order[rc - 1];     // graph node of the row
+        const uint64_t d4 = static_cast<uint64_t>(rec.w) << 32 | rec.z;
+        const int nrow = static_cast<int>(rec.y);  // graph node of the row
         const uint32_t cw = ri >= 1 ? ((cj >= 0 ? c0 : 0u) | ((cj >= 1 ? c1 : 0u) << 16)) : 0u;
         wait_stores();  // the block is in registers before the walk starts
         // successor of the lane's cell (di_l, dj) as di * 8 + dj, with the
@@ -3280,7 +3279,7 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(RH_POA_WAVES_PER_EU))) void RH_POA_SYM(poa_batch_kernel)(
     const PoaParams* __restrict__ params) {
   CParams& P = *(CParams*)params;
-  extern __shared__ uint8_t lds[];
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   GByte* slot_mem = global(P.scratch) + static_cast<uint64_t>(blockIdx.x) * P.slot_bytes;
   __shared__ uint32_t next;
   while (true) {
@@ -3324,7 +3323,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(RH_POA_WAVES
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(RH_POA_WAVES_PER_EU))) void RH_POA_SYM(poa_single_kernel)(
     const PoaParams* __restrict__ params, uint32_t q) {
   CParams& P = *(CParams*)params;
-  extern __shared__ uint8_t lds[];
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const uint32_t w = global(P.order)[q];
   Slot s = carve(global(P.scratch), P.layout);
   __shared__ PoaResult res;
@@ -3347,7 +3346,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(RH_POA_WAVES
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(RH_POA_WAVES_PER_EU))) void RH_POA_SYM(poa_static_kernel)(
     const PoaParams* __restrict__ params, uint32_t first) {
   CParams& P = *(CParams*)params;
-  extern __shared__ uint8_t lds[];
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const uint32_t w = global(P.order)[first + blockIdx.x];
   Slot s = carve(global(P.scratch) + static_cast<uint64_t>(blockIdx.x) * P.slot_bytes, P.layout);
   __shared__ PoaResult res;

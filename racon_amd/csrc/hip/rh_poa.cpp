@@ -46,20 +46,34 @@ const char* last_error() { return g_error.c_str(); }
 
 namespace {
 
-// DP rows kept in LDS (16-bit scores): as many as fit while 16 waves share a
-// CU's 160 KiB (12 or 8 waves for long layers), at most 8; a tuned value
-// overrides it.
-uint32_t ring_rows_for(uint32_t cols, uint32_t tuned) {
+// DP rows kept in LDS (16-bit scores) when `waves` waves share a CU's
+// 160 KiB: as many as fit, at most 16 (8 at the full 16 waves, fewer waves
+// for long layers whose rows would be under four); a tuned value overrides
+// it. A row that finds no LDS slot goes through global memory and costs
+// several times an LDS row, so a batch that cannot fill the CUs with 16 waves
+// takes the deeper ring that its fewer waves leave room for: 1,037 windows of
+// 1,000 bp (5 waves per CU) took 1,427 ms with the 4 rows of 16 waves per CU
+// and 520 ms with 12 or more; 800 windows of short reads 191 and 186 ms with
+// 8 and 16.
+uint32_t ring_rows_for(uint32_t cols, uint32_t tuned, uint32_t waves) {
   if (tuned != 0) {
     return std::max<uint32_t>(2, std::min<uint32_t>(16, tuned));
   }
   const uint64_t lds_per_cu = 160u * 1024u;
-  for (uint32_t waves : {16u, 12u, 8u}) {
-    const uint64_t per_wave = lds_per_cu / waves;
-    const uint64_t fixed = align_up(cols, 16);
+  const uint64_t fixed = align_up(cols, 16);
+  if (waves < 16) {
+    // (LDS is handed out in 1,280-byte steps, and the kernel holds a few
+    // hundred bytes of its own)
+    const uint64_t per_wave = lds_per_cu / std::max(1u, waves) / 1280 * 1280;
+    const uint64_t taken = fixed + 512;
+    const uint64_t rows = per_wave > taken ? (per_wave - taken) / (2ull * cols) : 0;
+    if (rows >= 4) return static_cast<uint32_t>(std::min<uint64_t>(16, rows));
+  }
+  for (uint32_t w : {16u, 12u, 8u}) {
+    const uint64_t per_wave = lds_per_cu / w;
     if (per_wave <= fixed) continue;
     const uint64_t rows = (per_wave - fixed) / (2ull * cols);
-    if (rows >= 4 || waves == 8u) {
+    if (rows >= 4 || w == 8u) {
       return static_cast<uint32_t>(std::max<uint64_t>(2, std::min<uint64_t>(8, rows)));
     }
   }
@@ -332,7 +346,8 @@ void PoaLane::release() {
 }
 
 bool plan_pass(const PoaWindow* host, const std::vector<uint32_t>& ws, uint32_t row_cap,
-               uint32_t lds_limit, uint32_t tune_ring, bool wide, PassPlan* plan) {
+               uint32_t lds_limit, uint32_t tune_ring, uint32_t waves, bool wide,
+               PassPlan* plan) {
   PoaSlotCaps caps{};
   uint32_t max_nodes = 1, max_edges = 1, max_cols = 1;
   for (uint32_t w : ws) {
@@ -354,7 +369,7 @@ bool plan_pass(const PoaWindow* host, const std::vector<uint32_t>& ws, uint32_t 
   caps.hrows = row_cap == 0 ? 0 : std::min<uint32_t>(caps.rows, kPoaHPoolRows);
   caps.aligned = wide ? kMaxAlignedWide : kMaxAligned;
   caps.stack = 2 * (max_edges + (caps.aligned + 1) * max_nodes) + 64;
-  uint32_t ring = ring_rows_for(caps.cols, tune_ring);
+  uint32_t ring = ring_rows_for(caps.cols, tune_ring, waves);
   while (ring > 0 && poa_lds_bytes(caps.cols, ring) > lds_limit) --ring;
   if (ring == 1) ring = 0;  // one 16-bit row is no slot in 32-bit mode; keep none
   if (poa_lds_bytes(caps.cols, ring) > lds_limit) {
@@ -407,13 +422,21 @@ int32_t plan_bins(PoaLane& lane, const PoaWindow* host, const std::vector<uint32
   for (uint32_t w : ws) {
     bins[layer_bin(host[w])].push_back(w);
   }
+  int cus = 0;
+  RH_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, lane.device),
+               RH_ERR_DEVICE);
   for (int k = 0; k < 2; ++k) {
     std::vector<uint32_t>& bin = bins[k];
     if (bin.empty()) continue;
+    // waves that share a CU: this pass on every lane of the device at once
+    const uint64_t resident = mode == RH_POA_PLAIN ? 1 : bin.size();
+    const uint64_t per_cu = (resident * std::max<uint32_t>(1, c.slot_share) + std::max(1, cus) - 1) /
+                            std::max(1, cus);
+    const uint32_t waves = static_cast<uint32_t>(std::min<uint64_t>(16, per_cu));
     if (mode == RH_POA_STATIC) std::sort(bin.begin(), bin.end());
     PassPlan plan{};
     const uint32_t ring = c.bin_ring[k] != 0 ? c.bin_ring[k] : c.tune_ring;
-    if (!plan_pass(host, bin, row_cap, lane.lds_limit, ring, wide, &plan)) {
+    if (!plan_pass(host, bin, row_cap, lane.lds_limit, ring, waves, wide, &plan)) {
       refused->insert(refused->end(), bin.begin(), bin.end());
       continue;
     }

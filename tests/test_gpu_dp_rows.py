@@ -1,0 +1,102 @@
+"""The packed DP rows at the edges of their forms, against the CPU oracle:
+layer lengths around 64 W columns for every strip width W (and past the last
+one, where the tiled rows take over), scores whose range just fits or just
+exceeds 16 bits, layers with letters other than A, C, G and T, rings of
+2 to 16 LDS rows (rows that find no slot go through global memory), and
+windows with several predecessors per node.
+"""
+import sys
+
+import numpy as np
+import pytest
+
+from racon_amd import _lib
+from racon_amd._lib import Layer, Window
+from synth import mutate, oracle_args, random_quality, random_seq
+
+sys.path.insert(0, _lib.PKG_DIR + "/../oracle")
+import oracle_py  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+
+def window(rng, length, depth, error=0.12, exact=()):
+    """A window of `length` bases; the layers named in `exact` are cut or
+    padded to that many bases."""
+    backbone = random_seq(rng, length)
+    truth = mutate(rng, backbone, 0.03)
+    layers = []
+    for k in range(depth):
+        begin, end = 0, length - 1
+        if k % 5 == 4:
+            begin, end = length // 5, length - 1 - length // 7
+        seq = mutate(rng, truth[begin:end + 1], error)
+        if k < len(exact):
+            begin, end = 0, length - 1
+            seq = (mutate(rng, truth, error) + random_seq(rng, exact[k]))[:exact[k]]
+        layers.append(Layer(seq, random_quality(rng, len(seq)), begin, end))
+    return Window(backbone, b"!" * length, layers)
+
+
+def check(windows, scores=(3, -5, -4), ring=0):
+    b = _lib.PoaBatch(*scores, trim=True)
+    if ring:
+        b.set_tuning(0, 0, ring)
+    b.upload(windows)
+    b.run(_lib.RH_POA_BATCHED)
+    out, status = b.download()
+    b.close()
+    for i, w in enumerate(windows):
+        cons, ost, _, _ = oracle_py.window_consensus(*oracle_args(w), True, *scores)
+        assert status[i] == ost, f"window {i} status"
+        assert out[i] == cons, f"window {i} consensus"
+
+
+@pytest.mark.parametrize("columns", [1, 4, 256, 512, 768, 1024, 1280])
+def test_layer_lengths_around_a_strip_edge(columns):
+    rng = np.random.default_rng(columns)
+    exact = [max(1, columns + d) for d in (-2, -1, 0, 1, 2)]
+    check([window(rng, max(30, columns), 8, exact=exact) for _ in range(2)])
+
+
+@pytest.mark.parametrize("scores", [(1, -1, -1), (5, -4, -8), (30, -20, -25), (127, -127, -20),
+                                    (1, -128, -128), (3, -5, 0)])
+def test_score_ranges_around_16_bits(scores):
+    rng = np.random.default_rng(17)
+    check([window(rng, n, 10) for n in (40, 250, 480, 700)], scores)
+
+
+@pytest.mark.parametrize("ring", [2, 3, 5, 16])
+def test_rows_without_an_lds_slot(ring):
+    rng = np.random.default_rng(23)
+    check([window(rng, n, 24, error=0.2) for n in (120, 505, 900)], ring=ring)
+
+
+def test_letters_other_than_acgt():
+    rng = np.random.default_rng(29)
+    wins = [window(rng, 300, 12) for _ in range(4)]
+    for w in wins[:3]:
+        for k in (1, 4, 7):
+            seq = bytearray(w.layers[k].sequence)
+            for at in rng.integers(0, len(seq), size=5):
+                seq[at] = ord("N")
+            w.layers[k].sequence = bytes(seq)
+    backbone = bytearray(wins[3].backbone)
+    backbone[10:14] = b"NNNN"
+    wins[3].backbone = bytes(backbone)
+    check(wins)
+
+
+def test_many_predecessors():
+    """Long random deletions give nodes with far more than four in-edges."""
+    rng = np.random.default_rng(31)
+    wins = []
+    for _ in range(3):
+        backbone = random_seq(rng, 400)
+        layers = []
+        for k in range(40):
+            cut = int(rng.integers(0, 150))
+            seq = mutate(rng, backbone[:200 - cut] + backbone[200:], 0.03)
+            layers.append(Layer(seq, None, 0, 399))
+        wins.append(Window(backbone, b"!" * 400, layers))
+    check(wins)
