@@ -43,15 +43,21 @@ enum : int32_t {
 // Leaf size rule of the path search: a subproblem is traced back directly
 // when (2 * 8 + 4) * ceil(|q| / 64) * |t| < 1 MiB, else split at |t| / 2.
 constexpr uint64_t kLeafBytes = 1024 * 1024;
-constexpr uint32_t kAlignStackDepth = 128;
+constexpr uint32_t kAlignTeamWaves = 8;  // waves of a team workgroup
+
+// One subproblem of the path recursion (score < 0: not known yet).
+struct AlignTask {
+  int32_t q0, ql, t0, tl, score;
+};
 
 struct AlignSlotLayout {
   uint64_t col_left;   // int32 [q cap]
   uint64_t col_right;  // int32 [q cap]
-  uint64_t carry;      // int8  [t cap + 64]
-  uint64_t store_p;    // uint64 [store words]
-  uint64_t store_m;    // uint64 [store words]
-  uint64_t store_s;    // int32  [store words]
+  uint64_t carry;      // int8  [t cap + 128] per wave
+  uint64_t carry_bytes;
+  uint64_t store;      // 16 B [store words] per wave
+  uint64_t planes;     // 32 B per 64 query rows
+  uint64_t tasks;      // AlignTask [2 x task cap]
   uint64_t ops_tmp;    // uint8 [q cap + t cap]
   uint64_t total;
 };
@@ -59,12 +65,13 @@ struct AlignSlotLayout {
 struct AlignSlotCaps {
   uint32_t q;            // longest query
   uint32_t t;            // longest target
-  uint64_t store_words;  // stored (column, block) entries for a leaf
+  uint64_t store_words;  // stored (column, block) entries of a wave's leaves
+  uint32_t tasks;        // subproblems of one recursion level
 };
 
 inline uint64_t align_up_a(uint64_t x, uint64_t a) { return (x + a - 1) / a * a; }
 
-inline AlignSlotLayout align_slot_layout(const AlignSlotCaps& c) {
+inline AlignSlotLayout align_slot_layout(const AlignSlotCaps& c, uint32_t waves = 1) {
   AlignSlotLayout l{};
   uint64_t o = 0;
   auto take = [&](uint64_t bytes) {
@@ -74,25 +81,50 @@ inline AlignSlotLayout align_slot_layout(const AlignSlotCaps& c) {
   };
   l.col_left = take(4ull * (c.q + 64));
   l.col_right = take(4ull * (c.q + 64));
-  l.carry = take(uint64_t(c.t) + 128);
-  l.store_p = take(8ull * c.store_words);
-  l.store_m = take(8ull * c.store_words);
-  l.store_s = take(4ull * c.store_words);
+  l.carry_bytes = align_up_a(uint64_t(c.t) + 128, 64);
+  l.carry = take(l.carry_bytes * waves);
+  l.store = take(16ull * c.store_words * waves);
+  l.planes = take(32ull * ((uint64_t(c.q) + 63) / 64 + 3));
+  l.tasks = take(2ull * c.tasks * sizeof(AlignTask));
   l.ops_tmp = take(uint64_t(c.q) + c.t + 64);
   l.total = o;
   return l;
 }
 
 // Slot capacities for pairs of at most max_q query and max_t target bytes:
-// the score columns and carries, and the stored columns of the largest leaf
-// (under kLeafBytes at 20 bytes per stored word) plus one block row's slack.
+// the score columns and carries, the stored columns of the largest leaf
+// (fewer than kLeafBytes / 20 blocks x columns) plus one block row's slack,
+// and the subproblems of one level: those that split again hold at least
+// kLeafBytes / 20 blocks x columns each, so n of them at tl = t / 2^level
+// columns need n <= q t / (64 kLeafBytes / 20) / 2^level, and there are at
+// most 2^level (all of them split while tl alone reaches kLeafBytes / 20).
 inline AlignSlotCaps align_caps_for(uint32_t max_q, uint32_t max_t) {
   AlignSlotCaps caps{};
   caps.q = max_q < 64 ? 64 : max_q;
   caps.t = max_t < 64 ? 64 : max_t;
   const uint64_t max_blocks = (caps.q + 63) / 64 + 1;
   caps.store_words = kLeafBytes / 20 + 64 * (max_blocks + 2);
+  const uint64_t blocks_cols = (max_blocks * caps.t) / (kLeafBytes / 20) + 1;
+  uint64_t most = 1;
+  while (most * most < blocks_cols) most *= 2;
+  caps.tasks = static_cast<uint32_t>(4 * most + 64 + 4 * (caps.t / (kLeafBytes / 20) + 1));
   return caps;
+}
+
+// Slot bytes that the allocation-free entry point has always asked for, and
+// so refuses sizes by; at least align_slot_layout(c).total.
+inline uint64_t align_slot_bound(const AlignSlotCaps& c) {
+  const auto up = [](uint64_t x) { return align_up_a(x, 256); };
+  return 2 * up(4ull * (c.q + 64)) + up(uint64_t(c.t) + 128) + 2 * up(8ull * c.store_words) +
+         up(4ull * c.store_words) + up(uint64_t(c.q) + c.t + 64);
+}
+
+// Waves per pair of a batch: a team of eight when pairs are long enough that
+// their runs outgrow one wave's lanes (about 10 kbp at a band of a fifth of the
+// length) and too few to give every SIMD its waves one pair each.
+inline uint32_t align_waves(uint64_t pairs, uint32_t max_q, uint32_t max_t, uint32_t cus) {
+  const uint32_t longest = max_q > max_t ? max_q : max_t;
+  return longest > 10000 && pairs <= 2ull * cus ? kAlignTeamWaves : 1;
 }
 
 struct AlignParams {
@@ -108,7 +140,7 @@ struct AlignParams {
   AlignSlotCaps caps;
   AlignSlotLayout layout;
   uint32_t band0;  // first band guess (distance bound) of a whole pair; 0: automatic
-  uint32_t pad;
+  uint32_t waves;  // waves per pair: 1 or kAlignTeamWaves
 };
 
 }  // namespace rh

@@ -15,7 +15,7 @@
 
 namespace rh {
 hipError_t launch_align_batch(const AlignParams& params, uint32_t grid, hipStream_t stream);
-hipError_t align_occupancy(int* blocks_per_cu);
+hipError_t align_occupancy(int* blocks_per_cu, uint32_t waves);
 hipError_t launch_breaking_points(const AlignPair* pairs, const AlignResult* results,
                                   const uint8_t* ops, const BreakSpan* spans, uint32_t n,
                                   uint32_t window_length, uint32_t* points, uint32_t* counts,
@@ -221,13 +221,15 @@ int32_t rh_align_run(rh_align_batch* b) {
     return RH_OK;
   }
   const rh::AlignSlotCaps caps = rh::align_caps_for(b->max_q, b->max_t);
-  const rh::AlignSlotLayout layout = rh::align_slot_layout(caps);
-  const uint64_t slot_bytes = rh::align_up_a(layout.total, 4096);
-
-  int per_cu = 0, cus = 0;
-  RH_HIP_CHECK(rh::align_occupancy(&per_cu), RH_ERR_DEVICE);
+  int cus = 0;
   RH_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device),
                RH_ERR_DEVICE);
+  const uint32_t waves = rh::align_waves(n, b->max_q, b->max_t, std::max(1, cus));
+  const rh::AlignSlotLayout layout = rh::align_slot_layout(caps, waves);
+  const uint64_t slot_bytes = rh::align_up_a(layout.total, 4096);
+
+  int per_cu = 0;
+  RH_HIP_CHECK(rh::align_occupancy(&per_cu, waves), RH_ERR_DEVICE);
   size_t free_b = 0, total_b = 0;
   RH_HIP_CHECK(hipMemGetInfo(&free_b, &total_b), RH_ERR_DEVICE);
   uint64_t slots = static_cast<uint64_t>(std::max(1, per_cu)) * std::max(1, cus);
@@ -251,6 +253,7 @@ int32_t rh_align_run(rh_align_batch* b) {
   p.caps = caps;
   p.layout = layout;
   p.band0 = b->band0;
+  p.waves = waves;
 
   RH_HIP_CHECK(hipEventRecord(b->ev0, b->stream), RH_ERR_DEVICE);
   RH_HIP_CHECK(rh::launch_align_batch(p, static_cast<uint32_t>(slots), b->stream),

@@ -18,7 +18,7 @@
 namespace rh {
 hipError_t launch_align_batch_cleared(const AlignParams& params, uint32_t grid,
                                       hipStream_t stream);
-hipError_t align_occupancy(int* blocks_per_cu);
+hipError_t align_occupancy(int* blocks_per_cu, uint32_t waves);
 }  // namespace rh
 
 // The scratch of every rh_align_run_noalloc call on a device. Held by each
@@ -85,15 +85,16 @@ extern "C" int32_t rh_align_run_noalloc(int32_t device, void* stream, uint32_t n
   const uint64_t slot_bytes = rh::align_up_a(layout.total, 256);
   const uint64_t head_bytes = 256;
   const uint64_t room = RH_NOALLOC_SCRATCH_BYTES - head_bytes;
-  if (slot_bytes > room) {
+  const uint64_t bound = rh::align_up_a(rh::align_slot_bound(caps), 256);
+  if (bound > room || slot_bytes > room) {
     rh::set_error("rh_align_run_noalloc: pairs of " + std::to_string(max_query_length) + " x " +
                   std::to_string(max_target_length) + " bytes need a " +
-                  std::to_string(slot_bytes) + "-byte slot, more than the " +
+                  std::to_string(bound) + "-byte slot, more than the " +
                   std::to_string(room) + " bytes of scratch");
     return RH_ERR_ARGUMENT;
   }
   int per_cu = 0, cus = 0;
-  RH_HIP_CHECK(rh::align_occupancy(&per_cu), RH_ERR_DEVICE);
+  RH_HIP_CHECK(rh::align_occupancy(&per_cu, 1), RH_ERR_DEVICE);
   RH_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device),
                RH_ERR_DEVICE);
   uint64_t slots = room / slot_bytes;
@@ -112,6 +113,7 @@ extern "C" int32_t rh_align_run_noalloc(int32_t device, void* stream, uint32_t n
   p.slot_bytes = slot_bytes;
   p.caps = caps;
   p.layout = layout;
+  p.waves = 1;
   RH_HIP_CHECK(rh::launch_align_batch_cleared(p, static_cast<uint32_t>(slots),
                                               static_cast<hipStream_t>(stream)),
                RH_ERR_KERNEL);
