@@ -175,6 +175,16 @@ struct Slot {
   __device__ int32_t* lpath() const { return (int32_t*)(p + L->lpath); }
   __device__ int32_t* sink_score() const { return (int32_t*)(p + L->sink_score); }
   __device__ int32_t* tie_mark() const { return (int32_t*)(p + L->tie_mark); }
+  // per node: base | in-edge count << 8, and the tails of the first eight
+  // in-edges (two quads)
+  __device__ uint32_t* node_info() const { return (uint32_t*)(p + L->node_info); }
+  __device__ int4* node_in() const { return (int4*)(p + L->node_in); }
+  // the in-edge that node_info has counted `info >> 8` of before
+  __device__ void add_in(int node, uint32_t info, int tail) const {
+    const uint32_t n = info >> 8;
+    if (n < 8) ((int32_t*)(p + L->node_in))[8 * node + n] = tail;
+    node_info()[node] = info + 256u;
+  }
   __device__ uint4* row_rec() const { return (uint4*)(p + L->row_rec); }
 
   int32_t n_nodes;
@@ -210,6 +220,7 @@ __device__ __forceinline__ int add_node(Slot& s, CCaps& caps, uint8_t base) {
   }
   const int v = s.n_nodes++;
   s.base()[v] = base;
+  s.node_info()[v] = base;
   s.in_head()[v] = -1;
   s.out_head()[v] = -1;
   s.in_tail()[v] = -1;
@@ -251,6 +262,7 @@ __device__ __forceinline__ void add_edge(Slot& s, CCaps& caps, int tail, int hea
     s.e_next_in()[s.in_tail()[head]] = e;
   }
   s.in_tail()[head] = e;
+  s.add_in(head, s.node_info()[head], tail);
   touch(s, tail, s.n_seqs);
   touch(s, head, s.n_seqs);
 }
@@ -1096,6 +1108,10 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
             if (p == 0) {
 #pragma unroll
               for (int q = 0; q < H2; ++q) pp[q] = pk_splat(bias);
+            } else if (sl == kSlotNone) {
+              // the row before, kept in registers only
+#pragma unroll
+              for (int q = 0; q < H2; ++q) pp[q] = cur[q];
             } else if (sl < kSlotGlobal) {
               lds_row_load<W>(strip + static_cast<uint32_t>(sl) * row_bytes, pp);
             } else {
@@ -1790,6 +1806,7 @@ __device__ __noinline__ InsertResult insert_parallel(GByte* slot_base, CLayout* 
         const int id = nv[i];
         s.anchor()[id - before] = v[i] != -1 ? bound[i] : prev_bound;
         base[id] = lseq[p];
+        s.node_info()[id] = lseq[p];
         s.in_head()[id] = -1;
         s.out_head()[id] = -1;
         s.in_tail()[id] = -1;
@@ -1881,12 +1898,14 @@ __device__ __noinline__ InsertResult insert_parallel(GByte* slot_base, CLayout* 
       }
     }
     int ot[kU], it[kU];
+    uint32_t info[kU];
 #pragma unroll
     for (int i = 0; i < kU; ++i) {
       const int p = p0 + i * kWave + lane;
       const bool need = p < L && found[i] == -1;
       ot[i] = need ? out_tail[tail[i]] : -1;
       it[i] = need ? in_tail[head[i]] : -1;
+      info[i] = need ? s.node_info()[head[i]] : 0u;
       if (found[i] != -1) e_weight[found[i]] = e_weight[found[i]] + w[i];
     }
 #pragma unroll
@@ -1917,6 +1936,7 @@ __device__ __noinline__ InsertResult insert_parallel(GByte* slot_base, CLayout* 
           e_next_in[it[i]] = ne;
         }
         in_tail[head[i]] = ne;
+        s.add_in(head[i], info[i], tail[i]);
       }
       n_edges += __popcll(m);
     }
@@ -1968,61 +1988,66 @@ __device__ __forceinline__ int32_t wave_prefix_sum(int32_t x) {
 // in-edge order (row 0, the virtual start, for rows without one), sink flags,
 // and an LDS slot for every row that a later row reads: the lowest slot whose
 // previous row is no longer needed (lane k < n_slots holds the last row that
-// reads slot k). With kFull every node is in the layer's subgraph and the
-// membership checks are skipped. Returns the largest predecessor count, or
-// -1 when a row needs a global score row and the slot's pool has none free.
-// Each lane takes kU rows per round (64 kU rows) and walks their edge lists
-// in lockstep, one edge of every list per step, so that the loads of the
-// kU lists are in flight together; the walk keeps the first kP predecessor
-// rows of each row, so only rows with more walk their in-edges again. The
-// slot of every row is also kept in LDS (one byte per row, in the DP ring,
-// which is idle here) for the predecessor entries, which then need no
-// reload of the row table just written. Out of line, like the DP, for a
-// register allocation of its own.
-template <bool kFull>
+// reads slot k). row_of is 0 for nodes outside the layer's subgraph. Returns
+// the largest predecessor count, or -1 when a row needs a global score row
+// and the slot's pool has none free. Out of line, like the DP, for a register
+// allocation of its own.
+//
+// Bound by the round trips to the graph's arrays (a slot's graph does not
+// stay in the caches of a full device) and by the serial slot assignment. The
+// first pass takes kU rows per lane per round in three round trips: the rows'
+// nodes, their first eight in-edges (kept inline per node) and the in-edges'
+// rows; it leaves each row's predecessor rows in its record, and the last
+// reader of every row in LDS with an atomic maximum, so no out-edge list is
+// walked. The second pass goes over 64 rows at a time, with the next rows
+// already loaded: slots one row after the other (ten instructions each), then
+// records and lists from the slots kept in LDS. With `records` (dp_rows) a row
+// whose only reader is the next row, which reads nothing else, takes no slot
+// (the DP still holds it in registers), and only rows of the general form get
+// a predecessor list. Walking both edge lists of every row instead took
+// 187 us a layer in a full batch of 500 bp windows at 52 layers and 79 us
+// alone; this takes 146 and 67.
 __device__ __noinline__ int build_rows(GByte* slot_base, CLayout* layout, int V, int n_slots,
-                                       uint32_t lds_addr, int lds_bytes) {
-  constexpr int kU = 3;  // rows per lane per round
-  constexpr int kP = 6;  // predecessor rows kept in registers (99.9% of rows have <= 6)
+                                       uint32_t lds_addr, int lds_bytes, int records) {
+  constexpr int kU = 4;       // rows per lane per round of the first pass
+  constexpr int kInline = 8;  // in-edges kept per node
   const Slot s = carve(uniform_ptr(slot_base), *uniform_ptr(layout));
   V = uniform(V);
   n_slots = uniform(n_slots);
-  const bool slots_in_lds = V <= uniform(lds_bytes);
-  LByte* lslot = (LByte*)(size_t)__builtin_amdgcn_readfirstlane(lds_addr);
+  lds_bytes = uniform(lds_bytes);
+  records = uniform(records);
+  lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);
   const int lane = lane_id();
+  // word r: last reader of row r + 1, then (second pass) its slot
+  LWord* word = (LWord*)(size_t)lds_addr;
+  const bool words = 4 * static_cast<int64_t>(V) <= lds_bytes;
+  LByte* lslot = (LByte*)(size_t)lds_addr;  // without room for words: slots in bytes
+  const bool bytes = V <= lds_bytes;
+  const bool packed = V < 0x10000;  // predecessor rows fit 16 bits
   const int32_t* sub_order = s.sub_order();
+  const int32_t* row_of = s.row_of();
+  const uint32_t* node_info = s.node_info();
+  const int4* node_in = s.node_in();
   const int32_t* in_head = s.in_head();
-  const int32_t* out_head = s.out_head();
   const int32_t* e_next_in = s.e_next_in();
-  const int32_t* e_next_out = s.e_next_out();
   const int32_t* e_tail = s.e_tail();
-  const int32_t* e_head = s.e_head();
-  const uint8_t* in_sub = s.in_sub();
-  const uint8_t* base = s.base();
-  int32_t* row_of = s.row_of();
   int32_t* row_meta = s.row_meta();
   int32_t* pred_off = s.pred_off();
   int32_t* pred_rows = s.pred_rows();
   uint4* row_rec = s.row_rec();
-  auto included = [&](int v) { return kFull || in_sub[v] != 0; };
-  // predecessor entry of DP row pr: the row and the slot it lives in
-  auto pred_entry = [&](int pr) {
-    const int sl = slots_in_lds ? static_cast<int>(lslot[pr - 1])
-                                : (row_meta[pr - 1] >> kRowMetaSlotShift) & 31;
-    return pr | (sl << kPredRowBits);
+  if (words) {
+    for (int r = lane; r < V; r += kWave) word[r] = 0u;
+    wave_fence();
+  }
+  auto read_by = [&](int p, int row) {
+    if (words) __hip_atomic_fetch_max(&word[p - 1], static_cast<uint32_t>(row), __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_WAVEFRONT);
   };
-  int run = 0;
   int max_np = 0;
-  int busy = lane < n_slots ? 0 : 0x7fffffff;
-  // pooled global score rows: lane k holds the last reader of entry k
-  // (pool0) and of entry 64 + k (pool1); entries past the pool never free
-  const int hpool = uniform(static_cast<int>(s.L->hpool));
-  int pool0 = lane < hpool ? 0 : 0x7fffffff;
-  int pool1 = lane + kWave < hpool ? 0 : 0x7fffffff;
-  bool pool_full = false;
   for (int r0 = 0; r0 < V; r0 += kU * kWave) {
-    int v[kU], ei[kU], eo[kU], np[kU], oc[kU], lu[kU], meta[kU], off[kU], slot[kU];
-    int pr[kU][kP];
+    int v[kU], np[kU];
+    uint32_t info[kU], at[kU][kInline / 2];
+    int4 in[kU];
 #pragma unroll
     for (int i = 0; i < kU; ++i) {
       const int r = r0 + i * kWave + lane;
@@ -2030,161 +2055,232 @@ __device__ __noinline__ int build_rows(GByte* slot_base, CLayout* layout, int V,
     }
 #pragma unroll
     for (int i = 0; i < kU; ++i) {
-      ei[i] = v[i] >= 0 ? in_head[v[i]] : -1;
-      eo[i] = v[i] >= 0 ? out_head[v[i]] : -1;
-      meta[i] = v[i] >= 0 ? static_cast<int>(base[v[i]]) : 0;
-      np[i] = 0;
-      oc[i] = 0;
-      lu[i] = 0;
-#pragma unroll
-      for (int j = 0; j < kP; ++j) pr[i][j] = 0;
-    }
-    for (;;) {
-      bool act = false;
-#pragma unroll
-      for (int i = 0; i < kU; ++i) act = act || ei[i] != -1 || eo[i] != -1;
-      if (__ballot(act) == 0) break;
-      int t[kU], h[kU], ni[kU], no[kU];
-#pragma unroll
-      for (int i = 0; i < kU; ++i) {
-        t[i] = -1;
-        ni[i] = -1;
-        h[i] = -1;
-        no[i] = -1;
-        if (ei[i] != -1) {
-          t[i] = e_tail[ei[i]];
-          ni[i] = e_next_in[ei[i]];
-        }
-        if (eo[i] != -1) {
-          h[i] = e_head[eo[i]];
-          no[i] = e_next_out[eo[i]];
-        }
-      }
-      int rt[kU], rh[kU];
-#pragma unroll
-      for (int i = 0; i < kU; ++i) {
-        rt[i] = t[i] != -1 && included(t[i]) ? row_of[t[i]] : 0;
-        rh[i] = h[i] != -1 && included(h[i]) ? row_of[h[i]] : 0;
-      }
-#pragma unroll
-      for (int i = 0; i < kU; ++i) {
-        if (rt[i] > 0) {
-#pragma unroll
-          for (int j = 0; j < kP; ++j) pr[i][j] = np[i] == j ? rt[i] : pr[i][j];
-          ++np[i];
-        }
-        if (rh[i] > 0) {
-          ++oc[i];
-          lu[i] = max(lu[i], rh[i]);
-        }
-        ei[i] = ni[i];
-        eo[i] = no[i];
-      }
+      info[i] = v[i] >= 0 ? node_info[v[i]] : 0u;
+      in[i] = v[i] >= 0 ? node_in[2 * v[i]] : make_int4(0, 0, 0, 0);
     }
 #pragma unroll
     for (int i = 0; i < kU; ++i) {
-      if (v[i] >= 0) meta[i] |= (oc[i] == 0 ? kRowMetaSink : 0) | (np[i] <= 1 ? kRowMetaSingle : 0);
-      max_np = max(max_np, v[i] >= 0 ? max(np[i], 1) : 0);  // row 0 stands in for none
+      const int n = static_cast<int>(info[i] >> 8);
+      const int t[4] = {in[i].x, in[i].y, in[i].z, in[i].w};
+      int row[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) row[j] = j < n ? row_of[t[j]] : 0;
+      in[i] = make_int4(row[0], row[1], row[2], row[3]);
     }
 #pragma unroll
     for (int i = 0; i < kU; ++i) {
-      const int c0 = r0 + i * kWave;
-      if (c0 >= V) break;
-      int my_slot = kSlotNone;
-      int my_pool = 0;
-      const int n_chunk = uniform(min(kWave, V - c0));
-      for (int rr = 0; rr < n_chunk; ++rr) {
-        const int l = __builtin_amdgcn_readlane(lu[i], rr);
-        if (l > 0) {
-          const int row = c0 + rr + 1;
-          const unsigned long long free_mask = __ballot(busy < row);
-          // the lowest free slot, else the global matrix (then the write
-          // goes to lane 63, which holds no slot and stays never free)
-          const bool none = free_mask == 0;
-          const int sl = none ? kSlotGlobal : __ffsll(static_cast<long long>(free_mask)) - 1;
-          busy = lane_write(none ? 0x7fffffff : l, none ? kWave - 1 : sl, busy);
-          my_slot = lane_write(sl, rr, my_slot);
-          if (none && hpool != 0) {
-            // the lowest free pool entry (lane k of pool0 holds entry k, of
-            // pool1 entry 64 + k); none free: the window reruns exactly
-            const unsigned long long g0 = __ballot(pool0 < row);
-            const unsigned long long g1 = __ballot(pool1 < row);
-            int g = 0;
-            if (g0 != 0) {
-              g = __ffsll(static_cast<long long>(g0)) - 1;
-              pool0 = lane_write(l, g, pool0);
-            } else if (g1 != 0) {
-              const int t = __ffsll(static_cast<long long>(g1)) - 1;
-              pool1 = lane_write(l, t, pool1);
-              g = kWave + t;
-            } else {
-              pool_full = true;
-            }
-            my_pool = lane_write(g, rr, my_pool);
-          }
-        }
-      }
-      const int r = c0 + lane;
-      const int cnt = v[i] >= 0 ? max(np[i], 1) : 0;
-      const int x = wave_prefix_sum(cnt);
-      off[i] = run + x - cnt;
-      if (r < V) {
-        row_meta[r] = meta[i] | (my_slot << kRowMetaSlotShift) | (my_pool << kRowMetaGShift);
-        pred_off[r] = off[i];
-        if (slots_in_lds) lslot[r] = static_cast<uint8_t>(my_slot);
-      }
-      slot[i] = my_slot;
-      run += __builtin_amdgcn_readlane(x, kWave - 1);
-    }
-    // predecessor entries (their slots are all assigned by now: predecessor
-    // rows come first)
-#pragma unroll
-    for (int i = 0; i < kU; ++i) {
-      if (v[i] < 0) continue;
       const int r = r0 + i * kWave + lane;
-      uint64_t deltas = 0;  // row deltas of the first four predecessors (0: none or too far)
-      // the row descriptor of dp_rows: stays in the general form (no
-      // predecessor count) unless every condition below holds
-      const int letter = meta[i] & 0xff;
-      const int code = ((letter >> 1) ^ (letter >> 2)) & 3;
-      uint32_t desc = (meta[i] & kRowMetaSink) != 0 ? kRecSink : 0u;
-      bool fast = np[i] >= 1 && np[i] <= static_cast<int>(kRecMaxPreds) && slot[i] != kSlotGlobal &&
-                  static_cast<int>((0x54474341u >> (8 * code)) & 0xffu) == letter;
-      uint32_t fields = static_cast<uint32_t>(np[i]) | static_cast<uint32_t>(code << 3) |
-                        static_cast<uint32_t>(slot[i]) << kRecOwnShift;
-      if (np[i] == 1 && pr[i][0] == r) fields |= kRecChain;
-      if (np[i] == 0) {
-        pred_rows[off[i]] = 0;
-        deltas = static_cast<uint64_t>(r + 1 <= 0xffff ? r + 1 : 0);
-      } else if (np[i] <= kP) {
+      np[i] = 0;
 #pragma unroll
-        for (int j = 0; j < kP; ++j) {
-          if (j < np[i]) {
-            const int entry = pred_entry(pr[i][j]);
-            const uint32_t sl = static_cast<uint32_t>(entry) >> kPredRowBits;
-            fast = fast && sl < static_cast<uint32_t>(kSlotGlobal);
-            if (j < static_cast<int>(kRecMaxPreds)) fields |= sl << (kRecPredShift + 5 * j);
-            pred_rows[off[i] + j] = entry;
-            const int d = r + 1 - pr[i][j];
-            if (j < 4 && d <= 0xffff) deltas |= static_cast<uint64_t>(d) << (16 * j);
+      for (int j = 0; j < kInline / 2; ++j) at[i][j] = 0u;
+      // the next predecessor of the row, in in-edge order
+      auto add = [&](int p) {
+        if (p <= 0) return;
+        read_by(p, r + 1);
+#pragma unroll
+        for (int j = 0; j < kInline / 2; ++j) {
+          at[i][j] |= (np[i] >> 1) == j ? static_cast<uint32_t>(p) << (16 * (np[i] & 1)) : 0u;
+        }
+        ++np[i];
+      };
+      add(in[i].x);
+      add(in[i].y);
+      add(in[i].z);
+      add(in[i].w);
+      const int n = static_cast<int>(info[i] >> 8);
+      if (__any(n > 4)) {
+        if (n > 4) {
+          const int4 t = node_in[2 * v[i] + 1];
+          const int a = row_of[t.x], b = n > 5 ? row_of[t.y] : 0;
+          const int c = n > 6 ? row_of[t.z] : 0, d = n > 7 ? row_of[t.w] : 0;
+          add(a);
+          add(b);
+          add(c);
+          add(d);
+        }
+        if (n > kInline) {
+          int k = 0;
+          for (int e = in_head[v[i]]; e != -1; e = e_next_in[e], ++k) {
+            if (k >= kInline) add(row_of[e_tail[e]]);
           }
         }
-      } else {
-        int o = off[i];
+      }
+      if (v[i] >= 0) {
+        row_meta[r] = static_cast<int32_t>((info[i] & 0xffu) | static_cast<uint32_t>(min(np[i], 255)) << 8);
+        row_rec[r] = make_uint4(at[i][0], at[i][1], at[i][2], at[i][3]);
+        max_np = max(max_np, max(np[i], 1));  // row 0 stands in for none
+      }
+    }
+  }
+  wave_sync();
+  int busy = lane < n_slots ? 0 : 0x7fffffff;
+  // pooled global score rows: lane k holds the last reader of entry k
+  // (pool0) and of entry 64 + k (pool1); entries past the pool never free
+  const int hpool = uniform(static_cast<int>(s.L->hpool));
+  int pool0 = lane < hpool ? 0 : 0x7fffffff;
+  int pool1 = lane + kWave < hpool ? 0 : 0x7fffffff;
+  bool pool_full = false;
+  int run = 0;
+  uint4 rec_next = make_uint4(0u, 0u, 0u, 0u);
+  int meta_next = 0, after_next = 0, node_next = 0;
+  auto fetch = [&](int r) {
+    if (r < V) {
+      rec_next = row_rec[r];
+      meta_next = row_meta[r];
+      node_next = sub_order[r];
+    }
+    after_next = r + 1 < V ? row_meta[r + 1] : 0;
+  };
+  fetch(lane);
+  for (int c0 = 0; c0 < V; c0 += kWave) {
+    const int r = c0 + lane;
+    const bool in = r < V;
+    const uint4 x = rec_next;
+    const int meta0 = meta_next, after = after_next, node = node_next;
+    // (the next rows' first-pass records: this chunk's writes stop before)
+    fetch(r + kWave);
+    const int letter = meta0 & 0xff;
+    const int np = (meta0 >> 8) & 0xff;
+    int last = 0;
+    if (words) {
+      last = in ? static_cast<int>(word[r]) : 0;
+    } else if (in) {
+      // no room for the last readers: from the out-edges
+      for (int e = s.out_head()[node]; e != -1; e = s.e_next_out()[e]) {
+        last = max(last, row_of[s.e_head()[e]]);
+      }
+    }
+    const bool chained = records != 0 && last == r + 2 && ((after >> 8) & 0xff) == 1;
+    int my_slot = kSlotNone;
+    int my_pool = 0;
+    for (unsigned long long need = __ballot(in && last != 0 && !chained); need != 0;
+         need &= need - 1) {
+      const int rr = __ffsll(static_cast<long long>(need)) - 1;
+      const int l = __builtin_amdgcn_readlane(last, rr);
+      const int row = c0 + rr + 1;
+      const unsigned long long free_mask = __ballot(busy < row);
+      if (free_mask != 0) {
+        const int sl = __ffsll(static_cast<long long>(free_mask)) - 1;
+        busy = lane_write(l, sl, busy);
+        my_slot = lane_write(sl, rr, my_slot);
+        continue;
+      }
+      // no LDS slot: the global matrix
+      my_slot = lane_write(kSlotGlobal, rr, my_slot);
+      if (hpool != 0) {
+        // the lowest free pool entry (lane k of pool0 holds entry k, of
+        // pool1 entry 64 + k); none free: the window reruns exactly
+        const unsigned long long g0 = __ballot(pool0 < row);
+        const unsigned long long g1 = __ballot(pool1 < row);
+        int g = 0;
+        if (g0 != 0) {
+          g = __ffsll(static_cast<long long>(g0)) - 1;
+          pool0 = lane_write(l, g, pool0);
+        } else if (g1 != 0) {
+          const int t = __ffsll(static_cast<long long>(g1)) - 1;
+          pool1 = lane_write(l, t, pool1);
+          g = kWave + t;
+        } else {
+          pool_full = true;
+        }
+        my_pool = lane_write(g, rr, my_pool);
+      }
+    }
+    const bool sink = last == 0;
+    if (in) {
+      row_meta[r] = letter | (sink ? kRowMetaSink : 0) | (np <= 1 ? kRowMetaSingle : 0) |
+                    (my_slot << kRowMetaSlotShift) | (my_pool << kRowMetaGShift);
+      if (words) {
+        word[r] = static_cast<uint32_t>(my_slot);
+      } else if (bytes) {
+        lslot[r] = static_cast<uint8_t>(my_slot);
+      }
+    }
+    if (!words && !bytes) {
+      wave_sync();  // slots are read from the row table
+    } else {
+      wave_fence();
+    }
+    auto slot_of = [&](int p) -> int {
+      if (words) return static_cast<int>(word[p - 1]);
+      if (bytes) return static_cast<int>(lslot[p - 1]);
+      return (row_meta[p - 1] >> kRowMetaSlotShift) & 31;
+    };
+    // the row's descriptor, unless it takes the general form
+    const int code = ((letter >> 1) ^ (letter >> 2)) & 3;
+    bool fast = packed && np >= 1 && np <= static_cast<int>(kRecMaxPreds) && my_slot != kSlotGlobal &&
+                static_cast<int>((0x54474341u >> (8 * code)) & 0xffu) == letter;
+    uint32_t fields = static_cast<uint32_t>(np) | static_cast<uint32_t>(code << 3) |
+                      static_cast<uint32_t>(my_slot) << kRecOwnShift;
+    uint64_t deltas = 0;  // row deltas of the first four predecessors (0: none or too far)
+    int p[kInline], sl[kInline];
+    if (in) {
+      const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+      for (int j = 0; j < kInline; ++j) {
+        p[j] = static_cast<int>((w[j / 2] >> (16 * (j & 1))) & 0xffffu);
+        sl[j] = 0;
+      }
+#pragma unroll
+      for (int j = 0; j < static_cast<int>(kRecMaxPreds); ++j) {
+        if (j < np && packed) {
+          sl[j] = slot_of(p[j]);
+          // (a chained predecessor is the row before: the descriptor's flag
+          // or, in the general form, kSlotNone)
+          fast = fast && (sl[j] < kSlotGlobal || (sl[j] == kSlotNone && np == 1));
+          fields |= static_cast<uint32_t>(sl[j] & 31) << (kRecPredShift + 5 * j);
+          deltas |= static_cast<uint64_t>(static_cast<uint32_t>(r + 1 - p[j])) << (16 * j);
+        }
+      }
+      if (np == 1 && packed && p[0] == r) fields |= kRecChain;
+    }
+    const bool lists = in && !(records != 0 && fast);
+    int cnt = lists ? max(np, 1) : 0;
+    const bool walk = lists && (!packed || np > kInline);
+    if (__any(walk)) {
+      if (walk) {
+        // (the count was capped in the row's record)
+        cnt = 0;
+        for (int e = in_head[node]; e != -1; e = e_next_in[e]) cnt += row_of[e_tail[e]] > 0;
+        cnt = max(cnt, 1);
+      }
+    }
+    const int sum = wave_prefix_sum(cnt);
+    const int off = run + sum - cnt;
+    run += __builtin_amdgcn_readlane(sum, kWave - 1);
+    if (in) pred_off[r] = off;
+    if (__any(lists)) {
+      if (lists && !walk) {
+        if (np == 0) {
+          pred_rows[off] = 0;
+          deltas = static_cast<uint64_t>(r + 1 <= 0xffff ? r + 1 : 0);
+        }
+#pragma unroll
+        for (int j = 0; j < kInline; ++j) {
+          if (j < np) pred_rows[off + j] = p[j] | (slot_of(p[j]) << kPredRowBits);
+        }
+      } else if (walk) {
+        int o = off;
         int k = 0;
-        for (int e = in_head[v[i]]; e != -1; e = e_next_in[e]) {
-          const int u = e_tail[e];
-          if (included(u)) {
-            const int p = row_of[u];
-            pred_rows[o++] = pred_entry(p);
-            const int d = r + 1 - p;
+        deltas = 0;
+        for (int e = in_head[node]; e != -1; e = e_next_in[e]) {
+          const int q = row_of[e_tail[e]];
+          if (q > 0) {
+            pred_rows[o++] = q | (slot_of(q) << kPredRowBits);
+            const int d = r + 1 - q;
             if (k < 4 && d <= 0xffff) deltas |= static_cast<uint64_t>(d) << (16 * k);
             ++k;
           }
         }
+        if (k == 0) {
+          pred_rows[off] = 0;
+          deltas = static_cast<uint64_t>(r + 1 <= 0xffff ? r + 1 : 0);
+        }
       }
-      if (fast) desc |= fields;
-      row_rec[r] = make_uint4(desc, static_cast<uint32_t>(v[i]), static_cast<uint32_t>(deltas),
+    }
+    if (in) {
+      const uint32_t desc = (sink ? kRecSink : 0u) | (fast ? fields : 0u);
+      row_rec[r] = make_uint4(desc, static_cast<uint32_t>(node), static_cast<uint32_t>(deltas),
                               static_cast<uint32_t>(deltas >> 32));
     }
   }
@@ -2198,112 +2294,169 @@ __device__ __noinline__ int build_rows(GByte* slot_base, CLayout* layout, int V,
 // Included nodes of a layer that does not span the window (spoa
 // Graph::subgraph's walk): the nodes >= begin that reach `end` backwards
 // along in-edges and aligned sets through nodes >= begin. The set is a
-// reachability closure and the stack bound (every in-edge and aligned entry
-// once, plus one) is within stack_cap, so the order of the walk changes
-// nothing: here every lane pops one stack entry per round, a visit bit in
-// LDS (claimed with an atomic OR) lets each node expand once, and the stack
-// sits in LDS above the bits, continuing into the slot's global stack.
-// Writes in_sub[0..nn). Returns 0, kPoaNodeOverflow, or 1 when the LDS
-// (lds_bytes at lds_addr) cannot hold the bits and 64 stack entries.
-__device__ __noinline__ int include_walk(GByte* slot_base, CLayout* layout, uint32_t lds_addr,
-                                         int lds_bytes, int begin, int end, int nn,
-                                         int stack_cap) {
+// reachability closure, so the order in which it is found changes nothing:
+// here it is found by rank, 64 ranks at a time from `end`'s down. In-edges lead
+// to lower ranks and aligned sets lie side by side, so a chunk's nodes are
+// decided by chunks above it and by each other. A chunk takes three round
+// trips to memory (its nodes; their in-edges and aligned sets; the ranks of
+// those), then closes over itself in registers: each node's readers inside the
+// chunk as a 64-bit mask, and one ballot per edge of the longest chain. Edges
+// that leave the chunk set the rank's bit in LDS; when one leads up to a chunk
+// that is done (an aligned set across a chunk border), that chunk is taken
+// again with its new nodes. Every pass over a chunk marks at least one new
+// node done, so the walk ends.
+//
+// On 800 windows of 150 bp reads a layer takes 23 us; a walk from `end` with a
+// round trip per edge of the path through the graph took 121.
+//
+// Writes in_sub[0..nn) for every rank's node. Returns 0, or 1 when the LDS
+// (lds_bytes at lds_addr) cannot hold the bits.
+__device__ __noinline__ int include_ranks(GByte* slot_base, CLayout* layout, uint32_t lds_addr,
+                                          int lds_bytes, int begin, int end, int nn) {
+  constexpr int kInline = 8;
+  constexpr int kA = static_cast<int>(kAligned);
+  constexpr int kT = kInline + kA;  // targets of a node kept in registers
   const Slot s = carve(uniform_ptr(slot_base), *uniform_ptr(layout));
-  lds_addr = uniform(static_cast<int>(lds_addr));
+  lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);
   lds_bytes = uniform(lds_bytes);
   begin = uniform(begin);
   end = uniform(end);
   nn = uniform(nn);
-  stack_cap = uniform(stack_cap);
   const int lane = lane_id();
-  const int n_words = (nn + 31) >> 5;
-  const int bits_bytes = static_cast<int>(align_up(static_cast<uint64_t>(n_words) * 4, 16));
-  const int lcap = (lds_bytes - bits_bytes) / 4;
-  if (lcap < kWave) return 1;
-  LWord* bits = (LWord*)(size_t)lds_addr;
-  LWord* lstack = (LWord*)(size_t)(lds_addr + bits_bytes);
-  int32_t* gstack = s.stack();
-  const int32_t* in_head = s.in_head();
-  const int32_t* e_next_in = s.e_next_in();
-  const int32_t* e_tail = s.e_tail();
+  const int chunks = (nn + kWave - 1) / kWave;
+  // per chunk 64 reached bits and 64 done bits, then the chunk's reader masks
+  typedef __attribute__((address_space(3))) unsigned long long LMask;
+  if (16 * chunks + 8 * kWave > lds_bytes) return 1;
+  LMask* reached = (LMask*)(size_t)lds_addr;
+  LMask* done = reached + chunks;
+  LMask* readers = done + chunks;
+  for (int c = lane; c < 2 * chunks; c += kWave) reached[c] = 0ull;
+  const int32_t* rank_to_node = s.rank_to_node();
+  const int32_t* node_rank = s.node_rank();
+  const uint32_t* node_info = s.node_info();
+  const int32_t* node_in = (const int32_t*)s.node_in();
+  const uint8_t* n_aligned = s.n_aligned();
   const int32_t* aligned = s.aligned();
-  const uint8_t* n_aligned_of = s.n_aligned();
-  for (int w = lane; w < n_words; w += kWave) bits[w] = 0u;
-  auto st_load = [&](int i) -> int {
-    return i < lcap ? static_cast<int>(lstack[i]) : gstack[i];
+  auto set_bit = [&](int rank) {
+    return __hip_atomic_fetch_or(&reached[rank >> 6], 1ull << (rank & 63), __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_WAVEFRONT);
   };
-  auto st_store = [&](int i, int x) {
-    if (i < lcap) {
-      lstack[i] = static_cast<uint32_t>(x);
-    } else {
-      gstack[i] = x;
-    }
-  };
-  auto unseen = [&](int u) {
-    return u >= begin && ((bits[u >> 5] >> (u & 31)) & 1u) == 0u;
-  };
-  const uint64_t below = (1ull << lane) - 1ull;
-  if (lane == 0) st_store(0, end);
-  int top = 1;
+  const int rank_end = uniform(node_rank[end]);
   wave_fence();
-  // candidates of one round, pushed in lane order; false on overflow
-  auto push = [&](bool c, int x) -> bool {
-    const uint64_t m = __ballot(c);
-    const int cnt = __popcll(m);
-    if (top + cnt > stack_cap) return false;
-    if (c) st_store(top + __popcll(m & below), x);
-    top += cnt;
-    return true;
-  };
-  // every claim sets a bit that stays set, so more than nn claims cannot
-  // happen; the count bounds the rounds even so (rounds without a claim only
-  // pop)
-  int claims = 0;
-  while (top > 0) {
-    const int nb = min(top, kWave);
-    const int first = top - nb;
-    int v = -1;
-    if (lane < nb) v = st_load(first + lane);
-    top = first;
-    bool mine = false;
-    if (v >= begin) {
-      const uint32_t m = 1u << (v & 31);
-      mine = (__atomic_fetch_or(&bits[v >> 5], m, __ATOMIC_RELAXED) & m) == 0u;
+  if (lane == 0 && end >= begin) set_bit(rank_end);
+  wave_fence();
+  int c = rank_end >> 6;
+  int low = c;  // lowest chunk with a reached node so far
+  while (c >= low) {
+    const unsigned long long before = reached[c], was_done = done[c];
+    const uint64_t r_lo = uniform(static_cast<int>(before)) & 0xffffffffu;
+    const uint64_t r_hi = uniform(static_cast<int>(before >> 32)) & 0xffffffffu;
+    unsigned long long now = r_hi << 32 | r_lo;
+    const uint64_t d_lo = uniform(static_cast<int>(was_done)) & 0xffffffffu;
+    const uint64_t d_hi = uniform(static_cast<int>(was_done >> 32)) & 0xffffffffu;
+    const unsigned long long old = d_hi << 32 | d_lo;
+    if (now == old) {
+      --c;
+      continue;
     }
-    claims += __popcll(__ballot(mine));
-    if (claims > nn) return kPoaNodeOverflow;
-    int e = -1;
-    int na = 0;
-    int al[kAligned];
-    if (mine) {
-      e = in_head[v];
-      na = n_aligned_of[v];
+    const int base = c * kWave;
+    const int v = base + lane < nn ? rank_to_node[base + lane] : -1;
+    // targets: in-edge tails, then the aligned set (-1: none or below begin)
+    int t[kT];
+    int n_in = 0, n_al = 0;
+    if (v >= 0) {
+      n_in = static_cast<int>(node_info[v] >> 8);
+      n_al = n_aligned[v];
+    }
+    const int max_in = min(kInline, uniform(__builtin_amdgcn_readlane(wave_prefix_max(n_in), kWave - 1)));
+    const int max_al = uniform(__builtin_amdgcn_readlane(wave_prefix_max(n_al), kWave - 1));
 #pragma unroll
-      for (int k = 0; k < static_cast<int>(kAligned); ++k) al[k] = aligned[v * kAligned + k];
-    }
-    wave_fence();  // the claims before the visit-bit reads below
-    const int max_na = uniform(__builtin_amdgcn_readlane(wave_prefix_max(na), kWave - 1));
-#pragma unroll
-    for (int k = 0; k < static_cast<int>(kAligned); ++k) {
-      if (k >= max_na) break;
-      const bool c = k < na && unseen(al[k]);
-      if (!push(c, al[k])) return kPoaNodeOverflow;
-    }
-    while (__ballot(e != -1) != 0) {
-      int t = -1;
-      int nx = -1;
-      if (e != -1) {
-        t = e_tail[e];
-        nx = e_next_in[e];
+    for (int j = 0; j < kT; ++j) {
+      const bool edge = j < kInline;
+      const int k = edge ? j : j - kInline;
+      t[j] = -1;
+      if (k < (edge ? max_in : max_al)) {
+        if (k < (edge ? n_in : n_al)) t[j] = edge ? node_in[kInline * v + k] : aligned[v * kA + k];
       }
-      if (!push(e != -1 && unseen(t), t)) return kPoaNodeOverflow;
-      e = nx;
+    }
+#pragma unroll
+    for (int j = 0; j < kT; ++j) {
+      const bool edge = j < kInline;
+      const int k = edge ? j : j - kInline;
+      if (k < (edge ? max_in : max_al)) t[j] = t[j] >= begin ? node_rank[t[j]] : -1;
+    }
+    readers[lane] = 0ull;
+    wave_fence();
+    const unsigned long long mine = 1ull << lane;
+    auto inside = [&](int rank) { return rank >= base && rank < base + kWave; };
+    auto add_reader = [&](int rank) {
+      __hip_atomic_fetch_or(&readers[rank - base], mine, __ATOMIC_RELAXED,
+                            __HIP_MEMORY_SCOPE_WAVEFRONT);
+    };
+#pragma unroll
+    for (int j = 0; j < kT; ++j) {
+      const bool edge = j < kInline;
+      const int k = edge ? j : j - kInline;
+      if (k < (edge ? max_in : max_al)) {
+        if (t[j] >= 0 && inside(t[j])) add_reader(t[j]);
+      }
+    }
+    // in-edges past the inline ones
+    auto more = [&](auto&& f) {
+      if (n_in > kInline) {
+        int k = 0;
+        for (int e = s.in_head()[v]; e != -1; e = s.e_next_in()[e], ++k) {
+          const int u = s.e_tail()[e];
+          if (k >= kInline && u >= begin) f(node_rank[u]);
+        }
+      }
+    };
+    more([&](int rank) {
+      if (inside(rank)) add_reader(rank);
+    });
+    wave_fence();
+    const unsigned long long by = readers[lane];
+    for (;;) {
+      const unsigned long long grown = now | __ballot((by & now) != 0);
+      if (grown == now) break;
+      now = grown;
+    }
+    // edges out of the chunk, from its new nodes
+    int up = -1;
+    int down = c;
+    if (((now & ~old) & mine) != 0) {
+      auto leave = [&](int rank) {
+        if (inside(rank)) return;
+        const unsigned long long seen = set_bit(rank);
+        if (rank < base) {
+          down = min(down, rank >> 6);
+        } else if (((seen >> (rank & 63)) & 1ull) == 0) {
+          up = max(up, rank >> 6);
+        }
+      };
+#pragma unroll
+      for (int j = 0; j < kT; ++j) {
+        const bool edge = j < kInline;
+        const int k = edge ? j : j - kInline;
+        if (k < (edge ? max_in : max_al)) {
+          if (t[j] >= 0) leave(t[j]);
+        }
+      }
+      more(leave);
+    }
+    if (lane == 0) {
+      reached[c] = now;
+      done[c] = now;
     }
     wave_fence();
+    low = min(low, uniform(-__builtin_amdgcn_readlane(wave_prefix_max(-down), kWave - 1)));
+    up = uniform(__builtin_amdgcn_readlane(wave_prefix_max(up), kWave - 1));
+    c = up >= 0 ? up : c - 1;
   }
   uint8_t* in_sub = s.in_sub();
-  for (int v = lane; v < nn; v += kWave) {
-    in_sub[v] = static_cast<uint8_t>((bits[v >> 5] >> (v & 31)) & 1u);
+  for (int r0 = 0; r0 < nn; r0 += kWave) {
+    const int r = r0 + lane;
+    if (r < nn) in_sub[rank_to_node[r]] = static_cast<uint8_t>((reached[r0 >> 6] >> lane) & 1ull);
   }
   return 0;
 }
@@ -2533,6 +2686,8 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
   }
   for (int i = lane; i < n; i += kWave) {
     s.base()[i] = bb[i];
+    s.node_info()[i] = bb[i] | (i > 0 ? 256u : 0u);
+    s.node_in()[2 * i] = make_int4(i - 1, 0, 0, 0);
     s.in_head()[i] = i > 0 ? i - 1 : -1;
     s.in_tail()[i] = i > 0 ? i - 1 : -1;
     s.out_head()[i] = i + 1 < n ? i : -1;
@@ -2595,13 +2750,8 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
     if (!full) {
       uint32_t walk_lds = static_cast<uint32_t>((size_t)(LByte*)lds);
       asm volatile("" : "+v"(walk_lds));
-      walk_rc = uniform(include_walk(s.p, s.L, walk_lds, static_cast<int>(P.ring_rows) * pitch * 2,
-                                     static_cast<int>(Lr.begin), static_cast<int>(Lr.end), nn,
-                                     static_cast<int>(caps.stack)));
-      if (walk_rc < 0) {
-        R.status = walk_rc;
-        return;
-      }
+      walk_rc = uniform(include_ranks(s.p, s.L, walk_lds, static_cast<int>(P.ring_rows) * pitch * 2,
+                                      static_cast<int>(Lr.begin), static_cast<int>(Lr.end), nn));
     }
     if (walk_rc != 0) {
       for (int v = lane; v < nn; v += kWave) {
@@ -2660,6 +2810,8 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
           const int at = V + __popcll(mask & ((1ull << lane) - 1ull));
           s.sub_order()[at] = v;
           s.row_of()[v] = at + 1;
+        } else if (r < nn) {
+          s.row_of()[v] = 0;
         }
         V += __popcll(mask);
       }
@@ -2688,8 +2840,8 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
     asm volatile("" : "+v"(rows_lds));
     const int ring_bytes = static_cast<int>(P.ring_rows) * pitch * 2;
     const int max_np =
-        uniform(full ? build_rows<true>(s.p, s.L, V, n_slots, rows_lds, ring_bytes)
-                     : build_rows<false>(s.p, s.L, V, n_slots, rows_lds, ring_bytes));
+        uniform(build_rows(s.p, s.L, V, n_slots, rows_lds, ring_bytes,
+                           rows16 && P.band == 0 && layer_plain ? 1 : 0));
     wave_sync();
     if (max_np < 0) {
       R.status = kPoaRowOverflow;  // the pooled global rows ran out: rerun exactly

@@ -107,7 +107,7 @@ struct PoaSlotLayout {
       last_label, e_tail, e_head, e_weight, e_next_in, e_next_out, rank_to_node,
       node_rank, mark, lead, stack, in_sub, row_of, sub_order, pred_off, pred_rows,
       row_meta, H, code, scores, preds, path, seq, qual, anchor, lpath,
-      sink_score, tie_mark, row_rec, total;
+      sink_score, tie_mark, row_rec, node_info, node_in, total;
   uint64_t hpool;  // caps.hrows
 };
 
@@ -159,6 +159,8 @@ inline PoaSlotLayout poa_slot_layout(const PoaSlotCaps& c) {
   l.sink_score = take(4 * (n + 1));
   l.tie_mark = take(4 * n);
   l.row_rec = take(16 * uint64_t(c.rows));
+  l.node_info = take(4 * n);
+  l.node_in = take(32 * n);
   l.total = o;
   l.hpool = c.hrows;
   return l;
