@@ -2461,6 +2461,175 @@ __device__ __noinline__ int include_ranks(GByte* slot_base, CLayout* layout, uin
   return 0;
 }
 
+// Traceback over the move records of dp_rows (W <= 16), from the end cell
+// (row, L) up to the virtual start row; the graph node of the diagonal move
+// into column p + 1, or -1 for a horizontal one, goes to path()[p] (s.path).
+// Returns the column reached in row 0, or -1 when a move leads outside.
+//
+// A tile is 64 rows, one per lane, and the columns of the last few strip
+// records at and before the current one: one round trip brings every row's
+// record (descriptor, node, predecessor deltas) and 16 or 32 bytes of moves.
+// The lanes put their fields in column order, the current column on top, so
+// that a column step is one shift of the tile and the walk reads its row's
+// move with v_readlane: about 35 instructions a move, most of them scalar. (Tiles of 16 rows x 8
+// columns with successor indices per cell took 66 round trips a layer of 490
+// columns instead of 20, 106 us alone and 216 us in a full batch.) Rows of the
+// general form are decoded one move at a time.
+template <int W>
+__device__ __noinline__ int trace_rows(GByte* slot_base, CLayout* layout, int pitch, int L, int row,
+                                       int plain) {
+  static_assert(W == 4 || W == 8 || W == 12 || W == 16, "strip width");
+  const Slot s = carve(uniform_ptr(slot_base), *uniform_ptr(layout));
+  pitch = uniform(pitch);
+  plain = uniform(plain);
+  const int lane = lane_id();
+  constexpr int kRecord = W == 4 ? 2 : W == 8 ? 4 : 8;  // bytes
+  constexpr int kRecords = 16 / kRecord;                // records of a tile
+  const GByte* codes = (const GByte*)s.code();
+  const uint4* row_rec = s.row_rec();
+  int32_t* pos_node = s.path();
+  int i = uniform(row), j = uniform(L);
+  while (i > 0) {
+    const int i0 = i, j0 = j;
+    const int ri = i0 - lane;
+    const int rc = max(ri, 1);
+    const GByte* mrow = codes + static_cast<int64_t>(rc) * pitch * 2;
+    const int q = j0 / W;
+    const int first = max(0, q - (kRecords - 1));  // first record of the tile
+    U32x4 w;
+    __builtin_memcpy(&w, (const uint8_t*)(mrow + first * kRecord), 16);
+    const uint4 rec = row_rec[rc - 1];
+    // fields of columns first * W .. in ascending order (two bits each, the
+    // bits of a field swapped: 1 diagonal, 2 vertical; predecessor indices 1
+    // and 2 trade places)
+    uint64_t kinds, preds;
+    {
+      const uint32_t r[4] = {__builtin_bitreverse32(w.x), __builtin_bitreverse32(w.y),
+                             __builtin_bitreverse32(w.z), __builtin_bitreverse32(w.w)};
+      if constexpr (W == 4) {
+        // bytes of r: record 2m + 1's indices, its kinds, record 2m's
+        // indices, its kinds; columns 1, 3, 0, 2 from the low bits up
+        uint32_t y[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+          y[m] = ((r[m] >> 4) & 0x03030303u) | ((r[m] & 0x03030303u) << 2) |
+                 ((r[m] >> 2) & 0x30303030u) | ((r[m] & 0x0c0c0c0cu) << 4);
+        }
+        const auto pick = [&](uint32_t a, uint32_t b, uint32_t sel) {
+          return __builtin_amdgcn_perm(b, a, sel);
+        };
+        kinds = static_cast<uint64_t>(pick(y[2], y[3], 0x05070103u)) << 32 | pick(y[0], y[1], 0x05070103u);
+        preds = static_cast<uint64_t>(pick(y[2], y[3], 0x04060002u)) << 32 | pick(y[0], y[1], 0x04060002u);
+      } else if constexpr (W == 8) {
+        // bytes of r: indices of the odd columns, of the even ones, kinds of
+        // the odd columns, of the even ones
+        const auto spread = [](uint32_t x) {  // even bytes' fields to every second field
+          x = (x | x << 4) & 0x0f0f0f0fu;
+          x = (x | x << 2) & 0x33333333u;
+          return (x | x >> 14) & 0xffffu;
+        };
+        uint32_t k[4], p[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+          k[m] = spread(__builtin_amdgcn_perm(0u, r[m], 0x0c020c03u));
+          p[m] = spread(__builtin_amdgcn_perm(0u, r[m], 0x0c000c01u));
+        }
+        kinds = static_cast<uint64_t>(k[2] | k[3] << 16) << 32 | (k[0] | k[1] << 16);
+        preds = static_cast<uint64_t>(p[2] | p[3] << 16) << 32 | (p[0] | p[1] << 16);
+      } else {
+        // words: kinds, indices per record; after the reversal the odd
+        // columns' fields are the low half, the even ones' the high half
+        const auto spread = [](uint32_t x) {  // 16 bits of fields to every second field
+          x = (x | x << 8) & 0x00ff00ffu;
+          x = (x | x << 4) & 0x0f0f0f0fu;
+          return (x | x << 2) & 0x33333333u;
+        };
+        const auto order = [&](uint32_t x) {
+          const uint32_t even = W == 16 ? x >> 16 : x >> 20;
+          const uint32_t odd = W == 16 ? x & 0xffffu : (x >> 4) & 0xfffu;
+          return spread(even) | spread(odd) << 2;
+        };
+        kinds = static_cast<uint64_t>(order(r[2])) << (2 * W) | order(r[0]);
+        preds = static_cast<uint64_t>(order(r[3])) << (2 * W) | order(r[1]);
+      }
+    }
+    // the current column's field on top
+    const int at = j0 - first * W;
+    kinds <<= 62 - 2 * at;
+    preds <<= 62 - 2 * at;
+    // lanes that end the walk inside the tile: rows of the general form and
+    // rows past the start (their node's sign bit set)
+    const bool stop = ri < 1 || plain == 0 || (rec.x & kRecPreds) == 0;
+    const int node_v = static_cast<int>(rec.y | (stop ? 0x80000000u : 0u));
+    // columns the tile can step: a diagonal also reads the column before
+    const int columns = first == 0 ? j0 + 1 : at;
+    int out = -1;  // lane t: the node of position j0 - 1 - t
+    int l = 0, t = 0;
+    int stopped = 0;
+    // (no branch on the kind of move: every move reads the same lanes and
+    // selects in scalar registers; a vertical move's -1 in lane t is written
+    // over by the move that leaves the column)
+    for (;;) {
+      const int node = __builtin_amdgcn_readlane(node_v, l);
+      if (node < 0) {
+        stopped = 1;
+        break;
+      }
+      uint32_t kx = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(kinds >> 32), l));
+      uint32_t px = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(preds >> 32), l));
+      uint32_t da = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(rec.z), l));
+      uint32_t db = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(rec.w), l));
+      // (opaque, so that the tests below stay on one word)
+      asm volatile("" : "+s"(kx));
+      const uint32_t kind = kx >> 30;
+      const uint32_t k = px >> ((kind & 1u) != 0 ? 28 : 30);  // (low two bits; 1 and 2 swapped)
+      const uint32_t pair = (k & 1u) != 0 ? db : da;
+      uint32_t delta = max((pair >> ((k & 2u) << 3)) & 0xffffu, 1u);
+      delta = kind != 0 ? delta : 0u;
+      uint32_t step = kind != 2u ? 1u : 0u;
+      out = lane_write((kind & 1u) != 0 ? node : -1, t, out);
+      l += static_cast<int>(delta);
+      t += static_cast<int>(step);
+      kinds <<= 2 * step;
+      preds <<= 2 * step;
+      if (((kWave - 1 - l) | (columns - 1 - t)) < 0) break;
+    }
+    i = i0 - l;
+    j = j0 - t;
+    if (lane < t && j0 - 1 - lane >= 0) pos_node[j0 - 1 - lane] = out;
+    if (i < 0 || j < 0) return -1;
+    if (i > 0 && stopped != 0) {
+      // one move of a row of the general form, from its 16-bit code
+      const int c = uniform(static_cast<int>(s.code()[static_cast<int64_t>(i) * pitch + j]));
+      const int kind = c & 0xc000;
+      if (kind == 0xc000 || (kind != kCodeVert && j == 0)) return -1;
+      if (kind != kCodeVert) {
+        if (lane == 0) {
+          pos_node[j - 1] = kind == kCodeDiag ? uniform(static_cast<int>(row_rec[i - 1].y)) : -1;
+        }
+        --j;
+      }
+      if (kind != kCodeHorz) {
+        const int k = c & static_cast<int>(kCodePayload);
+        int delta = 0;
+        if (k < 4) {
+          const uint4 x = row_rec[i - 1];
+          const uint32_t pair = k < 2 ? x.z : x.w;
+          delta = uniform(static_cast<int>((pair >> (16 * (k & 1))) & 0xffffu));
+        }
+        if (delta == 0) {
+          const int p = uniform(s.pred_rows()[uniform(s.pred_off()[i - 1]) + k]) & kPredRowMask;
+          delta = i - p;
+        }
+        if (delta <= 0) return -1;
+        i -= delta;
+        if (i < 0) return -1;
+      }
+    }
+  }
+  return j;
+}
+
 // End cell among tied sinks: spoa takes the first tied sink in its DFS order
 // of the (sub)graph (roots in id order; a node's predecessors first; a lead
 // node pushes its aligned set and emits it after itself, in aligned-list
@@ -2942,7 +3111,20 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
     // the predecessor lists) is taken by the full single-step decoder. The
     // block's positions are collected in one register (lane t: position
     // j0 - 1 - t) and stored together.
-    {
+    if (rows16 && !banded && row_w <= 16) {
+      const int plain = layer_plain ? 1 : 0;
+      const int left = uniform(
+          row_w == 4    ? trace_rows<4>(s.p, s.L, pitch, L, best_row, plain)
+          : row_w == 8  ? trace_rows<8>(s.p, s.L, pitch, L, best_row, plain)
+          : row_w == 12 ? trace_rows<12>(s.p, s.L, pitch, L, best_row, plain)
+                        : trace_rows<16>(s.p, s.L, pitch, L, best_row, plain));
+      if (left < 0) {
+        R.status = kPoaBadInput;
+        return;
+      }
+      // from the virtual start row only horizontal moves remain
+      for (int p = lane; p < left; p += kWave) s.path()[p] = -1;
+    } else{
       const uint16_t* code = s.code();
       const int32_t* pred_off = s.pred_off();
       const int32_t* pred_rows = s.pred_rows();
