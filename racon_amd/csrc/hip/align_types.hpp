@@ -119,14 +119,6 @@ inline uint64_t align_slot_bound(const AlignSlotCaps& c) {
          up(4ull * c.store_words) + up(uint64_t(c.q) + c.t + 64);
 }
 
-// Waves per pair of a batch: a team of eight when pairs are long enough that
-// their runs outgrow one wave's lanes (about 10 kbp at a band of a fifth of the
-// length) and too few to give every SIMD its waves one pair each.
-inline uint32_t align_waves(uint64_t pairs, uint32_t max_q, uint32_t max_t, uint32_t cus) {
-  const uint32_t longest = max_q > max_t ? max_q : max_t;
-  return longest > 10000 && pairs <= 2ull * cus ? kAlignTeamWaves : 1;
-}
-
 struct AlignParams {
   const AlignPair* pairs;
   const uint8_t* arena;

@@ -21,6 +21,36 @@ hipError_t launch_breaking_points(const AlignPair* pairs, const AlignResult* res
                                   uint32_t window_length, uint32_t* points, uint32_t* counts,
                                   hipStream_t stream);
 
+// Steps a pair takes on one wave, about: each level of the recursion runs over
+// the target once, its runs side by side while they fit the 64 lanes (up to
+// about 9 kbp at a band of a fifth of the length), the top level's halves one
+// after the other up to 19 kbp, and strips of 4,096 rows beyond.
+double single_wave_steps(const AlignPair& p) {
+  const double n = std::max(p.q_len, p.t_len);
+  if (n <= 9000) return 1.3 * n;
+  if (n <= 19000) return 2.2 * n;
+  return n * (2.2 + n / 20480);
+}
+
+// Pairs at the head of the cost order that run in teams of kAlignTeamWaves
+// waves: those that outgrow one wave's lanes and would, on one wave, outlast
+// the mean wave of the batch. They set the batch's time otherwise: of 12,000
+// pairs of 8 +- 4 kbp the mean wave was done after 11 ms and the last one
+// after 36; with the longest 500 or so in teams the batch takes 16 to 20 ms.
+uint32_t align_team_pairs(const std::vector<AlignPair>& pairs, const std::vector<uint32_t>& order,
+                          uint64_t waves) {
+  double total = 0;
+  for (const AlignPair& p : pairs) total += single_wave_steps(p);
+  uint32_t n = 0;
+  while (n < order.size()) {
+    const AlignPair& p = pairs[order[n]];
+    if (std::max(p.q_len, p.t_len) <= 10000) break;
+    if (single_wave_steps(p) * static_cast<double>(waves) <= total) break;
+    ++n;
+  }
+  return n;
+}
+
 // Windows of window_length target bases that the span [t_begin, t_end)
 // crosses: one per multiple of W inside (t_begin, t_end), plus the last.
 uint64_t span_windows(uint32_t window_length, const rh_break_span& s) {
@@ -42,8 +72,9 @@ struct rh_align_batch {
   uint32_t max_q = 0, max_t = 0;
   rh::DeviceBuffer d_arena, d_pairs, d_ops, d_results, d_order, d_queue, d_scratch;
   rh::DeviceBuffer d_spans, d_points, d_counts;  // breaking points
-  hipStream_t stream = nullptr;
-  hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  rh::DeviceBuffer d_team;  // slots of the teams
+  hipStream_t stream = nullptr, team_stream = nullptr;
+  hipEvent_t ev0 = nullptr, ev1 = nullptr, ev_team = nullptr;
   bool uploaded = false, ran = false;
   // the last rh_align_breaking_points call's points, still on the device
   bool points_ready = false;
@@ -88,10 +119,11 @@ int32_t rh_align_create(int32_t device, rh_align_batch** batch) {
   RH_HIP_CHECK(hipSetDevice(device), RH_ERR_DEVICE);
   rh_align_batch* b = new rh_align_batch();
   b->device = device;
-  if (hipStreamCreate(&b->stream) != hipSuccess || hipEventCreate(&b->ev0) != hipSuccess ||
-      hipEventCreate(&b->ev1) != hipSuccess) {
+  if (hipStreamCreate(&b->stream) != hipSuccess || hipStreamCreate(&b->team_stream) != hipSuccess ||
+      hipEventCreate(&b->ev0) != hipSuccess || hipEventCreate(&b->ev1) != hipSuccess ||
+      hipEventCreateWithFlags(&b->ev_team, hipEventDisableTiming) != hipSuccess) {
     rh::set_error("rh_align_create: stream/event creation failed");
-    delete b;
+    rh_align_destroy(b);
     return RH_ERR_DEVICE;
   }
   *batch = b;
@@ -104,6 +136,8 @@ void rh_align_destroy(rh_align_batch* b) {
   }
   (void)hipSetDevice(b->device);
   if (b->stream != nullptr) (void)hipStreamSynchronize(b->stream);
+  if (b->team_stream != nullptr) (void)hipStreamSynchronize(b->team_stream);
+  b->d_team.release();
   b->d_arena.release();
   b->d_pairs.release();
   b->d_ops.release();
@@ -116,7 +150,9 @@ void rh_align_destroy(rh_align_batch* b) {
   b->d_scratch.release();
   if (b->ev0 != nullptr) (void)hipEventDestroy(b->ev0);
   if (b->ev1 != nullptr) (void)hipEventDestroy(b->ev1);
+  if (b->ev_team != nullptr) (void)hipEventDestroy(b->ev_team);
   if (b->stream != nullptr) (void)hipStreamDestroy(b->stream);
+  if (b->team_stream != nullptr) (void)hipStreamDestroy(b->team_stream);
   delete b;
 }
 
@@ -220,50 +256,82 @@ int32_t rh_align_run(rh_align_batch* b) {
     b->points_ready = false;
     return RH_OK;
   }
-  const rh::AlignSlotCaps caps = rh::align_caps_for(b->max_q, b->max_t);
   int cus = 0;
   RH_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device),
                RH_ERR_DEVICE);
-  const uint32_t waves = rh::align_waves(n, b->max_q, b->max_t, std::max(1, cus));
-  const rh::AlignSlotLayout layout = rh::align_slot_layout(caps, waves);
-  const uint64_t slot_bytes = rh::align_up_a(layout.total, 4096);
-
-  int per_cu = 0;
-  RH_HIP_CHECK(rh::align_occupancy(&per_cu, waves), RH_ERR_DEVICE);
   size_t free_b = 0, total_b = 0;
   RH_HIP_CHECK(hipMemGetInfo(&free_b, &total_b), RH_ERR_DEVICE);
-  uint64_t slots = static_cast<uint64_t>(std::max(1, per_cu)) * std::max(1, cus);
-  slots = std::min<uint64_t>(slots, std::max<uint64_t>(
-                                        1, (free_b + b->d_scratch.bytes) * 6 / 10 / slot_bytes));
-  slots = std::min<uint64_t>(slots, n);
-  RH_HIP_CHECK(b->d_scratch.reserve(slots * slot_bytes), RH_ERR_MEMORY);
-  RH_HIP_CHECK(b->d_queue.reserve(sizeof(uint32_t)), RH_ERR_MEMORY);
-  RH_HIP_CHECK(hipMemsetAsync(b->d_queue.ptr, 0, sizeof(uint32_t), b->stream), RH_ERR_DEVICE);
-
-  rh::AlignParams p{};
-  p.pairs = b->d_pairs.as<rh::AlignPair>();
-  p.arena = b->d_arena.as<uint8_t>();
-  p.ops = b->d_ops.as<uint8_t>();
-  p.results = b->d_results.as<rh::AlignResult>();
-  p.order = b->d_order.as<uint32_t>();
-  p.n_order = n;
-  p.queue_head = b->d_queue.as<uint32_t>();
-  p.scratch = b->d_scratch.as<uint8_t>();
-  p.slot_bytes = slot_bytes;
-  p.caps = caps;
-  p.layout = layout;
-  p.band0 = b->band0;
-  p.waves = waves;
-
+  // the long pairs at the head of the cost order run in teams on a stream of
+  // their own, beside the rest
+  int waves_per_cu = 0;
+  RH_HIP_CHECK(rh::align_occupancy(&waves_per_cu, 1), RH_ERR_DEVICE);
+  const uint32_t teams = rh::align_team_pairs(
+      b->pairs, b->order, static_cast<uint64_t>(std::max(1, waves_per_cu)) * std::max(1, cus));
+  struct Part {
+    uint32_t first, n, waves;
+    uint64_t slots, slot_bytes;
+    rh::AlignSlotCaps caps;
+    rh::AlignSlotLayout layout;
+    rh::DeviceBuffer* scratch;
+    hipStream_t stream;
+  };
+  std::vector<Part> parts;
+  if (teams > 0) parts.push_back(Part{0, teams, rh::kAlignTeamWaves, 0, 0, {}, {}, &b->d_team, b->team_stream});
+  if (teams < n) parts.push_back(Part{teams, n - teams, 1, 0, 0, {}, {}, &b->d_scratch, b->stream});
+  // (the slots of both parts within 60% of the free memory)
+  const uint64_t budget =
+      (free_b + b->d_scratch.bytes + b->d_team.bytes) * 6 / 10 / parts.size();
+  for (Part& part : parts) {
+    uint32_t max_q = 0, max_t = 0;
+    for (uint32_t k = part.first; k < part.first + part.n; ++k) {
+      max_q = std::max(max_q, b->pairs[b->order[k]].q_len);
+      max_t = std::max(max_t, b->pairs[b->order[k]].t_len);
+    }
+    part.caps = rh::align_caps_for(max_q, max_t);
+    part.layout = rh::align_slot_layout(part.caps, part.waves);
+    part.slot_bytes = rh::align_up_a(part.layout.total, 4096);
+    int per_cu = 0;
+    RH_HIP_CHECK(rh::align_occupancy(&per_cu, part.waves), RH_ERR_DEVICE);
+    uint64_t slots = static_cast<uint64_t>(std::max(1, per_cu)) * std::max(1, cus);
+    slots = std::min<uint64_t>(slots, std::max<uint64_t>(1, budget / part.slot_bytes));
+    part.slots = std::min<uint64_t>(slots, part.n);
+    RH_HIP_CHECK(part.scratch->reserve(part.slots * part.slot_bytes), RH_ERR_MEMORY);
+  }
+  RH_HIP_CHECK(b->d_queue.reserve(2 * sizeof(uint32_t)), RH_ERR_MEMORY);
+  RH_HIP_CHECK(hipMemsetAsync(b->d_queue.ptr, 0, 2 * sizeof(uint32_t), b->stream), RH_ERR_DEVICE);
   RH_HIP_CHECK(hipEventRecord(b->ev0, b->stream), RH_ERR_DEVICE);
-  RH_HIP_CHECK(rh::launch_align_batch(p, static_cast<uint32_t>(slots), b->stream),
-               RH_ERR_KERNEL);
+  for (size_t k = 0; k < parts.size(); ++k) {
+    const Part& part = parts[k];
+    rh::AlignParams p{};
+    p.pairs = b->d_pairs.as<rh::AlignPair>();
+    p.arena = b->d_arena.as<uint8_t>();
+    p.ops = b->d_ops.as<uint8_t>();
+    p.results = b->d_results.as<rh::AlignResult>();
+    p.order = b->d_order.as<uint32_t>() + part.first;
+    p.n_order = part.n;
+    p.queue_head = b->d_queue.as<uint32_t>() + k;
+    p.scratch = part.scratch->as<uint8_t>();
+    p.slot_bytes = part.slot_bytes;
+    p.caps = part.caps;
+    p.layout = part.layout;
+    p.band0 = b->band0;
+    p.waves = part.waves;
+    if (part.stream != b->stream) {
+      RH_HIP_CHECK(hipStreamWaitEvent(part.stream, b->ev0, 0), RH_ERR_DEVICE);
+    }
+    RH_HIP_CHECK(rh::launch_align_batch(p, static_cast<uint32_t>(part.slots), part.stream),
+                 RH_ERR_KERNEL);
+    if (part.stream != b->stream) {
+      RH_HIP_CHECK(hipEventRecord(b->ev_team, part.stream), RH_ERR_DEVICE);
+    }
+  }
+  if (teams > 0) RH_HIP_CHECK(hipStreamWaitEvent(b->stream, b->ev_team, 0), RH_ERR_DEVICE);
   RH_HIP_CHECK(hipEventRecord(b->ev1, b->stream), RH_ERR_DEVICE);
   RH_HIP_CHECK(hipEventSynchronize(b->ev1), RH_ERR_KERNEL);
   float ms = 0;
   RH_HIP_CHECK(hipEventElapsedTime(&ms, b->ev0, b->ev1), RH_ERR_DEVICE);
   b->stats.kernel_ms = ms;
-  b->stats.launches = 1;
+  b->stats.launches = static_cast<uint32_t>(parts.size());
   RH_HIP_CHECK(rh::copy_sync(b->results.data(), b->d_results.ptr, n * sizeof(rh::AlignResult),
                              hipMemcpyDeviceToHost, b->stream),
                RH_ERR_DEVICE);
