@@ -86,12 +86,6 @@ constexpr uint16_t kCodeVert = 0x4000;
 constexpr uint16_t kCodeHorz = 0x8000;
 constexpr uint16_t kCodeViaK = 0x2000;
 constexpr uint32_t kCodePayload = 0x1fff;
-// Band rows with one predecessor store only the move of each cell, as a 2-bit kind 2 fd + fv from the flags fd (not diagonal) and fv
-// (not vertical): 0 or 1 diagonal, 2 vertical, 3 horizontal (column j at
-// bits 2 (j - 1) % 8 of byte (j - 1) / 4 of the row's code memory). The
-// predecessor is implied, and column 0 is always vertical.
-constexpr uint32_t kKindVert = 2;
-constexpr uint32_t kKindHorz = 3;
 // Bits 16..22 of a row's meta word: the row's entry in the slot's pool of
 // global score rows (a row that found no LDS slot, in a pass with a pool).
 constexpr int kRowMetaGShift = 16;
@@ -387,8 +381,6 @@ __device__ __forceinline__ void wave_fence() {
 __device__ __forceinline__ void wait_stores() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
 constexpr int kRowMetaSink = 0x100;
-// The row has one predecessor (or only the virtual start row).
-constexpr int kRowMetaSingle = 0x200;
 // Bits 10..14 of a row's meta word: where the row's scores live while later
 // rows need them. Slots 0..kMaxLdsSlots-1 are LDS rows; kSlotGlobal rows go
 // through the slot's global H matrix; kSlotNone rows are read by no later row.
@@ -674,22 +666,16 @@ __device__ __forceinline__ int dp_layer(CParams& P, const Slot& s, uint8_t* lds,
 
 // ---- packed 16-bit pairs: two DP columns per 32-bit register ----
 
-typedef short __attribute__((ext_vector_type(2))) I16x2;
 typedef unsigned short __attribute__((ext_vector_type(2))) U16x2;
 
 __device__ __forceinline__ U16x2 as_u16x2(uint32_t x) { return __builtin_bit_cast(U16x2, x); }
-__device__ __forceinline__ I16x2 as_i16x2(uint32_t x) { return __builtin_bit_cast(I16x2, x); }
 __device__ __forceinline__ uint32_t pk_bits(U16x2 x) { return __builtin_bit_cast(uint32_t, x); }
-__device__ __forceinline__ uint32_t pk_bits(I16x2 x) { return __builtin_bit_cast(uint32_t, x); }
-// per-half wrapping add / subtract, signed max, unsigned min, multiply-add
+// per-half wrapping add / subtract, unsigned min, multiply-add
 __device__ __forceinline__ uint32_t pk_add(uint32_t a, uint32_t b) {
   return pk_bits(as_u16x2(a) + as_u16x2(b));
 }
 __device__ __forceinline__ uint32_t pk_sub(uint32_t a, uint32_t b) {
   return pk_bits(as_u16x2(a) - as_u16x2(b));
-}
-__device__ __forceinline__ uint32_t pk_max(uint32_t a, uint32_t b) {
-  return pk_bits(__builtin_elementwise_max(as_i16x2(a), as_i16x2(b)));
 }
 __device__ __forceinline__ uint32_t pk_min_u(uint32_t a, uint32_t b) {
   return pk_bits(__builtin_elementwise_min(as_u16x2(a), as_u16x2(b)));
@@ -697,21 +683,8 @@ __device__ __forceinline__ uint32_t pk_min_u(uint32_t a, uint32_t b) {
 __device__ __forceinline__ uint32_t pk_mad(uint32_t a, uint32_t b, uint32_t c) {
   return pk_bits(as_u16x2(a) * as_u16x2(b) + as_u16x2(c));
 }
-// max of a with the low (resp. high) half of b in both halves
-__device__ __forceinline__ uint32_t pk_max_lo(uint32_t a, uint32_t b) {
-  const I16x2 v = as_i16x2(b);
-  return pk_bits(__builtin_elementwise_max(as_i16x2(a), __builtin_shufflevector(v, v, 0, 0)));
-}
-__device__ __forceinline__ uint32_t pk_max_hi(uint32_t a, uint32_t b) {
-  const I16x2 v = as_i16x2(b);
-  return pk_bits(__builtin_elementwise_max(as_i16x2(a), __builtin_shufflevector(v, v, 1, 1)));
-}
-// (lo, max(lo, hi)): inclusive prefix max inside the pair
-__device__ __forceinline__ uint32_t pk_scan(uint32_t a) {
-  const I16x2 v = as_i16x2(a);
-  return pk_bits(__builtin_elementwise_max(v, __builtin_shufflevector(v, v, 0, 0)));
-}
-// the same for unsigned halves
+// unsigned max; of a with the high half of b; inclusive prefix max inside the
+// pair; saturating subtract
 __device__ __forceinline__ uint32_t pk_max_u(uint32_t a, uint32_t b) {
   return pk_bits(__builtin_elementwise_max(as_u16x2(a), as_u16x2(b)));
 }
@@ -728,9 +701,6 @@ __device__ __forceinline__ uint32_t pk_sub_sat(uint32_t a, uint32_t b) {
 }
 __device__ __forceinline__ uint32_t pk_splat(int32_t v) {
   return (static_cast<uint32_t>(v) & 0xffffu) * 0x10001u;
-}
-__device__ __forceinline__ int32_t pk_half(uint32_t x, int hi) {
-  return hi ? static_cast<int32_t>(x) >> 16 : static_cast<int32_t>(static_cast<int16_t>(x & 0xffffu));
 }
 
 // ---- packed DP rows (dp_rows) ----
@@ -1206,39 +1176,6 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
   return uniform(best_row);
 }
 
-__device__ __forceinline__ uint32_t from_prev_lane(uint32_t x) {
-  return static_cast<uint32_t>(
-      __builtin_amdgcn_update_dpp(0, static_cast<int>(x), 0x138, 0xf, 0xf, false));  // wave_shr:1
-}
-
-// Per-lane constants of the band rows: pair q holds strip columns
-// j0 + 2q (low half) and j0 + 2q + 1 (high half).
-template <int W>
-struct PackedStrip {
-  uint32_t base[W / 2];  // layer bytes of the pair, one per half
-  uint32_t match_gap;    // match - gap and gap in both halves
-  uint32_t gap;
-  uint32_t one;          // 1 in both halves, opaque to the optimizer (a
-  uint32_t c4000;        // visible 1 turns min(x, 1) into compares and selects)
-  uint32_t diff;         // mismatch - match in both halves
-};
-
-template <int W>
-__device__ __forceinline__ void packed_strip_init(PackedStrip<W>& ps, const uint32_t* sw, int j0,
-                                                  int32_t match, int32_t mismatch, int32_t gap) {
-#pragma unroll
-  for (int q = 0; q < W / 2; ++q) {
-    ps.base[q] = __builtin_amdgcn_perm(sw[q / 2], sw[q / 2], (q & 1) ? 0x0c030c02u : 0x0c010c00u);
-  }
-  ps.match_gap = pk_splat(match - gap);
-  ps.gap = pk_splat(gap);
-  ps.one = 0x00010001u;
-  asm volatile("" : "+s"(ps.one));
-  ps.c4000 = 0x40004000u;
-  asm volatile("" : "+v"(ps.c4000));
-  ps.diff = pk_splat(mismatch - match);
-}
-
 // ---- banded rows: the opt-in approximation of racon -b ----
 //
 // Each DP row r (1..V) computes only 256 columns, 4 per lane: columns
@@ -1247,11 +1184,25 @@ __device__ __forceinline__ void packed_strip_init(PackedStrip<W>& ps, const uint
 // lo never decreases with r, so a predecessor p < r holds row r's lane k in
 // its lane k + (lo(r) - lo(p)) / 4. Values outside a row's band read as
 // kBandNeg; a window whose traceback would leave the band is rerun unbanded
-// (kPoaBandMiss). Used for layers longer than 256 only, and only in the
-// packed 16-bit form (kBandNeg sits below every value that form holds).
+// (kPoaBandMiss). Used for layers longer than 256 only, and only while scores
+// fit signed 16 bits (kBandNeg sits below every value they hold).
+//
+// The rows work as dp_rows' with 4 columns per lane (unsigned halves, the
+// bias is 32768): one descriptor per row, scores by byte permute, move
+// records. An LDS row holds column lo's value (column 0's when lo is 0, else
+// kBandNeg) in front of the lanes' strips, so the value left of the first
+// lane is one read whatever the shift. Records are kept by column as if column
+// j were j + 3, so that a lane's four columns are one record; a row with
+// several predecessors also keeps the index chosen at column lo, which the
+// diagonal into its first column takes. Rows of one wave alone are bound by
+// their instructions: 611 windows of 1,000 bp at 30 layers take 61 ms, where
+// band rows with a predecessor list per row, letters reloaded per row and a
+// traceback in blocks of 16 rows took about 90.
 constexpr int kBandW = 4;
 constexpr int kBand = kWave * kBandW;  // 256 columns
-constexpr int32_t kBandNeg = -32768 + 64;
+constexpr uint32_t kBandNeg = 64;      // -32768 + 64, with the bias
+constexpr uint32_t kBandBias = 0x8000;
+constexpr int kBandColumn = 3;         // record column of column j: j + 3
 
 __device__ __forceinline__ int band_lo(int r, int V, int L) {
   // (single-precision r * (L / V): monotone in r, the same in the DP and the
@@ -1262,222 +1213,300 @@ __device__ __forceinline__ int band_lo(int r, int V, int L) {
   return min(max(c, 0) & ~3, top);
 }
 
-// Whether cell (i, j) lies in row i's band (row 0, the virtual start row,
-// holds every column).
-__device__ __forceinline__ bool in_band(int i, int j, int V, int L) {
-  if (i <= 0) return true;
-  const int lo = band_lo(i, V, L);
-  return (j > lo && j <= lo + kBand) || (j == 0 && lo == 0);
-}
-
-// Predecessor row p (entry e) at the lanes of a band row whose band starts
-// after column lo: pp[q] = (G[p][j0 + 2q], G[p][j0 + 2q + 1]) with
-// j0 = lo + 1 + 4 lane, kBandNeg outside p's band; returns G[p][j0 - 1] in
-// the low half.
-__device__ __forceinline__ uint32_t load_band(const int16_t* ring, int pitch, const Slot& s, int e,
-                                              int lo, int V, int L, int lane, uint32_t* pp) {
-  const int p = e & kPredRowMask;
-  const int sl = static_cast<unsigned>(e) >> kPredRowBits;
-  const uint32_t neg = pk_splat(kBandNeg);
-  if (p == 0) {  // the virtual start row: G = 0 everywhere
-    pp[0] = pp[1] = 0u;
-    return 0u;
+// Predecessor row in the LDS row at `row` (its data after 8 bytes), seen
+// `shift` lanes further right; *left: the value left of the first lane.
+__device__ __forceinline__ void band_load(uint32_t row, int lane, int shift, uint32_t* pp,
+                                          uint32_t* left) {
+  constexpr uint32_t neg = kBandNeg * 0x10001u;
+  if (shift > kWave) {
+    pp[0] = pp[1] = neg;
+    *left = kBandNeg;
+    return;
   }
-  const int lo_p = band_lo(p, V, L);
-  const int shift = max(lo - lo_p, 0) >> 2;  // p < r: lo_p <= lo
   const int src = lane + shift;
-  if (sl < kSlotGlobal) {
-    const int16_t* row = ring + sl * pitch;
-    const bool in = src < kWave;
-    const uint2 v = *reinterpret_cast<const uint2*>(row + 4 * (in ? src : 0));
-    pp[0] = in ? v.x : neg;
-    pp[1] = in ? v.y : neg;
-    // column lo of p: the last one of p's lane shift - 1, or p's column 0
-    uint32_t c0 = neg;
-    if (shift > 0 && shift <= kWave) {
-      c0 = static_cast<uint16_t>(row[4 * (shift - 1) + 3]);
-    } else if (shift == 0 && lo == 0) {
-      c0 = static_cast<uint16_t>(row[pitch - 1]);
-    }
-    const uint32_t prev = from_prev_lane(pp[1]) >> 16;
-    return lane == 0 ? c0 : prev;
-  }
-  // a row kept in the slot's global matrix (int32, absolute columns)
-  const int32_t* row = s.H_row(p, pitch);
-  int32_t hv[kBandW + 1];
-#pragma unroll
-  for (int u = 0; u <= kBandW; ++u) {
-    const int j = lo + 4 * lane + u;
-    const bool valid = (j > lo_p && j <= lo_p + kBand && j <= L) || (j == 0 && lo_p == 0);
-    hv[u] = valid ? row[j] : kBandNeg;
-  }
-  wait_stores();
-  pp[0] = (static_cast<uint32_t>(hv[1]) & 0xffffu) | (static_cast<uint32_t>(hv[2]) << 16);
-  pp[1] = (static_cast<uint32_t>(hv[3]) & 0xffffu) | (static_cast<uint32_t>(hv[4]) << 16);
-  return static_cast<uint32_t>(hv[0]) & 0xffffu;
+  const U32x2 v = *(const LPair*)(size_t)(row + 8 + 8 * static_cast<uint32_t>(min(src, kWave - 1)));
+  typedef __attribute__((address_space(3))) uint16_t LHalf;
+  *left = *(const LHalf*)(size_t)(row + 8 * static_cast<uint32_t>(shift) + 6);
+  pp[0] = src < kWave ? v.x : neg;
+  pp[1] = src < kWave ? v.y : neg;
 }
 
-// One band row: packed_compute with the lane-0 chain starting from column 0
-// only when the band starts there, values kept at or above kBandNeg, then
-// the stores of packed_store at the band's columns. Returns H[row][L], or
-// kNegInf when column L is outside the band.
-template <bool kMulti>
-__device__ __forceinline__ int32_t band_row(const PackedStrip<kBandW>& ps, const uint32_t* pp,
-                                            uint32_t hp0, const uint32_t* kk, uint32_t k0,
-                                            uint32_t b, uint32_t pay0, int lane, int lo, int L,
-                                            int32_t gap, int own, int pitch, int16_t* ring,
-                                            int32_t* Hg, uint16_t* Cr) {
-  constexpr int H2 = kBandW / 2;
-  const uint32_t bb = b * 0x10001u;
-  const uint32_t neg = pk_splat(kBandNeg);
-  const int32_t h0 = pk_half(hp0 + static_cast<uint32_t>(gap), 0);  // column 0 when lo == 0
-  uint32_t carry = lane == 0 ? (lo == 0 ? pk_splat(h0) : neg) : 0x80008000u;
-  uint32_t bd[H2], bv[H2], pre[H2], h[H2], cd[H2];
+// The rest of a band row: moves, chain, scores (cur), from the best
+// predecessor scores pp and the value left of the first lane.
+__device__ __forceinline__ void band_scores(const uint32_t* pp, uint32_t left, const uint32_t* sub,
+                                            uint32_t gap_pair, int lane, int lo, uint32_t& excl,
+                                            uint32_t* cur, uint32_t* cur_left, uint32_t* bd,
+                                            uint32_t* bv) {
+  constexpr uint32_t neg = kBandNeg * 0x10001u;
+  const uint32_t prev = shift_into(left << 16, pp[1]);
+  // column 0 heads the chain of a band that starts there
+  const uint32_t h0 = lo == 0 ? (left + gap_pair) & 0xffffu : kBandNeg;
+  uint32_t carry = lane == 0 ? h0 << 16 : 0u;
+  uint32_t pre[2];
 #pragma unroll
-  for (int q = 0; q < H2; ++q) {
-    const uint32_t d = q == 0 ? ((pp[0] << 16) | (hp0 & 0xffffu))
-                              : __builtin_amdgcn_alignbit(pp[q], pp[q - 1], 16);
-    const uint32_t mis = pk_min_u(ps.base[q] ^ bb, ps.one);
-    bd[q] = pk_mad(mis, ps.diff, pk_add(d, ps.match_gap));
-    bv[q] = pk_add(pp[q], ps.gap);
-    carry = pk_max_hi(pk_scan(pk_max(bd[q], bv[q])), carry);
+  for (int q = 0; q < 2; ++q) {
+    const uint32_t d = __builtin_amdgcn_alignbit(pp[q], q == 0 ? prev : pp[0], 16);
+    bd[q] = pk_add(d, sub[q]);
+    bv[q] = pk_add(pp[q], gap_pair);
+    carry = pk_max_hi_u(pk_scan_u(pk_max_u(bd[q], bv[q])), carry);
     pre[q] = carry;
   }
-  const int32_t excl = wave_shift_right(wave_prefix_max(static_cast<int32_t>(carry) >> 16), -32768);
+  excl = shift_into(excl, wave_prefix_max_u(carry));
 #pragma unroll
-  for (int q = 0; q < H2; ++q) {
-    h[q] = pk_max(pk_max_lo(pre[q], static_cast<uint32_t>(excl)), neg);
-    const uint32_t fd = pk_min_u(pk_sub(h[q], bd[q]), ps.one);
-    const uint32_t fv = pk_min_u(pk_sub(h[q], bv[q]), ps.one);
-    if (kMulti) {
-      const uint32_t kd = q == 0 ? ((kk[0] << 16) | (k0 & 0xffffu))
-                                 : __builtin_amdgcn_alignbit(kk[q], kk[q - 1], 16);
-      const uint32_t dc = pk_add(kd, 0x20002000u);     // diagonal | kCodeViaK | k
-      const uint32_t vc = pk_add(kk[q], 0x60006000u);  // vertical | kCodeViaK | k
-      const uint32_t cv = pk_mad(fv, pk_sub(0x80008000u, vc), vc);
-      cd[q] = pk_mad(fd, pk_sub(cv, dc), dc);
-    } else {
-      cd[q] = (fd << 1) | fv;  // the move kind, as in packed_compute
-    }
-  }
-  const int j0 = lo + 1 + kBandW * lane;
-  if (kMulti) {
-    *reinterpret_cast<uint2*>(Cr + (j0 - 1)) = make_uint2(cd[0], cd[1]);
-  } else {
-    // 2-bit kinds of the lane's 4 columns: byte (j0 - 1) / 4 of the row
-    const uint32_t x = cd[0] | (cd[1] << 4);
-    reinterpret_cast<uint8_t*>(Cr)[(j0 - 1) >> 2] = static_cast<uint8_t>(x | (x >> 14));
-  }
-  if (own < kSlotGlobal) {
-    *reinterpret_cast<uint2*>(ring + own * pitch + 4 * lane) = make_uint2(h[0], h[1]);
-  } else if (own == kSlotGlobal) {
-#pragma unroll
-    for (int u = 0; u < kBandW; ++u) {
-      if (j0 + u <= L) Hg[j0 + u] = pk_half(h[u / 2], u & 1);
-    }
-  }
-  if (lane == 0) {
-    const int16_t c0 = static_cast<int16_t>(lo == 0 ? h0 : kBandNeg);
-    if (own < kSlotGlobal) ring[own * pitch + pitch - 1] = c0;
-    if (own == kSlotGlobal) Hg[0] = c0;
-    if (kMulti && lo == 0) {
-      Cr[pitch - 1] = static_cast<uint16_t>(kCodeVert | kCodeViaK | (k0 & 0xffffu));
-    }
-  }
-  const int e = L - 1 - lo;  // column L in the band: lane e / 4, column e % 4
-  if (e < 0 || e >= kBand) return kNegInf;
-  const int eu = e % kBandW;
-  uint32_t v = eu < 2 ? h[0] : h[1];
-  return __builtin_amdgcn_readlane(pk_half(v, eu & 1), e / kBandW) + L * gap;
+  for (int q = 0; q < 2; ++q) cur[q] = pk_max_u(pk_max_hi_u(pre[q], excl), neg);
+  *cur_left = h0;
 }
 
-// DP rows of one layer in band rows (layers longer than 256, packed form).
-// Same codes, sink scores and end cell as dp_layer_strip inside the bands.
-__device__ __forceinline__ int dp_layer_band(CParams& P, const Slot& s, uint8_t* lds, int V, int L,
-                                             int* best_score, bool* tied) {
+// DP rows of one layer in band rows (layers longer than 256, 16-bit form).
+__device__ __forceinline__ int dp_band(CParams& P, const Slot& s, uint32_t lds, int V, int L,
+                                       int* best_score, bool* tied) {
   const int lane = lane_id();
   const int pitch = static_cast<int>(P.caps.cols);
   const int32_t gap = uniform(P.gap);
   const int32_t match = uniform(P.match);
   const int32_t mismatch = uniform(P.mismatch);
-  int16_t* ring = reinterpret_cast<int16_t*>(lds);
-  const uint8_t* seq = lds + align_up(static_cast<uint64_t>(P.ring_rows) * pitch * 2, 16);
-  PackedStrip<kBandW> ps;
-  {
-    uint32_t sw0 = 0;
-    packed_strip_init<kBandW>(ps, &sw0, 1, match, mismatch, gap);
+  const uint32_t row_bytes = static_cast<uint32_t>(pitch) * 2;
+  const uint32_t seq_at =
+      lds + static_cast<uint32_t>(align_up(static_cast<uint64_t>(P.ring_rows) * row_bytes, 16));
+  const LByte* seq = (const LByte*)(size_t)seq_at;
+  typedef __attribute__((address_space(3))) uint16_t LHalf;
+  typedef __attribute__((address_space(1))) uint16_t GHalf;
+  const uint32_t gap_pair = pk_splat(gap);
+  const uint32_t miss = static_cast<uint32_t>(mismatch - gap) & 0xffffu;
+  const uint32_t flip = (static_cast<uint32_t>(match - gap) & 0xffffu) ^ miss;
+  const uint64_t table0 = static_cast<uint64_t>((miss >> 8) * 0x01010101u) << 32 |
+                          (miss & 0xffu) * 0x01010101u;
+  const uint64_t table1 = static_cast<uint64_t>(flip >> 8) << 32 | (flip & 0xffu);
+  uint32_t one = 0x00010001u;  // (opaque, as in dp_rows)
+  asm volatile("" : "+s"(one));
+  bool plain = true;
+  for (int j = lane; j < L; j += kWave) {
+    const int c = seq[j];
+    plain &= static_cast<int>((0x54474341u >> (8 * (((c >> 1) ^ (c >> 2)) & 3))) & 0xffu) == c;
   }
+  const bool layer_plain = __all(plain);
+  uint32_t excl = 0;  // lane 0: nothing to its left
   int32_t best = kNegInf;
   int best_row = 0;
   int ties = 0;
   const int total_preds = uniform(s.pred_off()[V]);
+  uint32_t cur[2] = {0u, 0u}, cur_left = 0u;  // the row before
+  uint32_t sel[2] = {0u, 0u};
+  int sel_lo = -1;
+  GByte* const codes = (GByte*)s.code();
   for (int r0 = 1; r0 <= V; r0 += kWave) {
     const int rk = r0 + lane;
-    int off_v = 0, end_v = 0, meta_v = 0;
+    uint32_t desc_v = 0, shift_v = 0;
+    const int lo_v = band_lo(min(rk, V), V, L);
     if (rk <= V) {
-      off_v = s.pred_off()[rk - 1];
-      end_v = s.pred_off()[rk];
-      meta_v = s.row_meta()[rk - 1];
+      const uint4 rec = s.row_rec()[rk - 1];
+      desc_v = rec.x;
+      const uint32_t d[4] = {rec.z & 0xffffu, rec.z >> 16, rec.w & 0xffffu, rec.w >> 16};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int by = (lo_v - band_lo(rk - static_cast<int>(d[k]), V, L)) >> 2;
+        shift_v |= static_cast<uint32_t>(min(max(by, 0), kWave + 1)) << (8 * k);
+      }
     }
-    const int base = __builtin_amdgcn_readlane(off_v, 0);
-    const int pr0 = base + lane < total_preds ? s.pred_rows()[base + lane] : 0;
-    const int pr1 = base + kWave + lane < total_preds ? s.pred_rows()[base + kWave + lane] : 0;
-    wait_stores();
-    const int chunk = min(kWave, V - r0 + 1);
+    if (!layer_plain) desc_v &= ~(kRecPreds | kRecChain);
+    const int chunk = uniform(min(kWave, V - r0 + 1));
+    int off_v = 0, end_v = 0, meta_v = 0, base = 0, pr0 = 0, pr1 = 0;
+    if (__any(rk <= V && (desc_v & kRecPreds) == 0)) {
+      if (rk <= V) {
+        off_v = s.pred_off()[rk - 1];
+        end_v = s.pred_off()[rk];
+        meta_v = s.row_meta()[rk - 1];
+      }
+      base = __builtin_amdgcn_readlane(off_v, 0);
+      pr0 = base + lane < total_preds ? s.pred_rows()[base + lane] : 0;
+      pr1 = base + kWave + lane < total_preds ? s.pred_rows()[base + kWave + lane] : 0;
+    }
+    wait_stores();  // (the chunk's loads, as in dp_rows)
+    GByte* record = codes + static_cast<int64_t>(r0) * row_bytes;
     for (int rr = 0; rr < chunk; ++rr) {
       const int r = r0 + rr;
-      const int off = __builtin_amdgcn_readlane(off_v, rr);
-      const int np = __builtin_amdgcn_readlane(end_v, rr) - off;
-      const int meta = __builtin_amdgcn_readlane(meta_v, rr);
-      auto pred_at = [&](int k) -> int {
-        const int idx = off + k - base;
-        if (idx < kWave) return __builtin_amdgcn_readlane(pr0, idx);
-        if (idx < 2 * kWave) return __builtin_amdgcn_readlane(pr1, idx - kWave);
-        const int e = uniform(s.pred_rows()[off + k]);
-        wait_stores();
-        return e;
-      };
-      const int lo = uniform(band_lo(r, V, L));
-      // the row's layer bytes: columns lo + 1 + 4 lane .. + 3 (lo + 4 lane
-      // + 3 <= L + 2 < pitch: inside the layer's LDS bytes and padding)
-      const uint32_t sw = *reinterpret_cast<const uint32_t*>(seq + lo + kBandW * lane);
-      ps.base[0] = __builtin_amdgcn_perm(sw, sw, 0x0c010c00u);
-      ps.base[1] = __builtin_amdgcn_perm(sw, sw, 0x0c030c02u);
-      const uint32_t b = static_cast<uint32_t>(meta & 0xff);
-      const int own = (meta >> kRowMetaSlotShift) & 31;
-      int32_t* Hg = s.H_row(r, meta, pitch);
-      uint16_t* Cr = s.code() + static_cast<int64_t>(r) * pitch;
-      int32_t h_last;
-      if (np == 1) {
-        const int e = pred_at(0);
-        const uint32_t delta = static_cast<uint32_t>(r - (e & kPredRowMask));
-        const uint32_t pay0 = delta <= kCodePayload ? delta : kCodeViaK;
-        uint32_t pp[2];
-        const uint32_t hp0 = load_band(ring, pitch, s, e, lo, V, L, lane, pp);
-        h_last = band_row<false>(ps, pp, hp0, pp, 0u, b, pay0, lane, lo, L, gap, own, pitch, ring,
-                                 Hg, Cr);
+      const uint32_t d = static_cast<uint32_t>(
+          __builtin_amdgcn_readlane(static_cast<int>(desc_v), rr));
+      const int lo = __builtin_amdgcn_readlane(lo_v, rr);
+      const uint32_t np = d & kRecPreds;
+      uint32_t bd[2], bv[2], sub[2];
+      if (np != 0) {
+        const uint32_t shifts = static_cast<uint32_t>(
+            __builtin_amdgcn_readlane(static_cast<int>(shift_v), rr));
+        if (lo != sel_lo) {
+          // letters of columns lo + 1 + 4 lane .. (bytes past the layer are
+          // never read back)
+          const uint32_t w = *(const LWord*)(size_t)(seq_at + static_cast<uint32_t>(lo + kBandW * lane));
+          const uint32_t c = ((w >> 1) ^ (w >> 2)) & 0x03030303u;
+          sel[0] = __builtin_amdgcn_perm(0u, c, 0x01010000u) + 0x04000400u;
+          sel[1] = __builtin_amdgcn_perm(0u, c, 0x03030202u) + 0x04000400u;
+          sel_lo = lo;
+        }
+        const uint64_t table = table0 ^ (table1 << (d & kRecBase));
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          sub[q] = __builtin_amdgcn_perm(static_cast<uint32_t>(table >> 32),
+                                         static_cast<uint32_t>(table), sel[q]);
+        }
+        const auto row_at = [&](int k) {
+          return lds + ((d >> (kRecPredShift + 5 * k)) & 31u) * row_bytes;
+        };
+        uint32_t mx[2], left;
+        uint32_t ack = 0, k_left = 0;
+        if ((d & kRecChain) != 0 && (shifts & 0xffu) == 0) {
+          mx[0] = cur[0];
+          mx[1] = cur[1];
+          left = cur_left;
+        } else {
+          band_load(row_at(0), lane, static_cast<int>(shifts & 0xffu), mx, &left);
+        }
+        if (np > 1) {
+          uint32_t kx[2] = {0u, 0u};
+#pragma unroll
+          for (int k = 1; k < static_cast<int>(kRecMaxPreds); ++k) {
+            if (k < static_cast<int>(np)) {
+              uint32_t pp[2], l1;
+              band_load(row_at(k), lane, static_cast<int>((shifts >> (8 * k)) & 0xffu), pp, &l1);
+#pragma unroll
+              for (int q = 0; q < 2; ++q) {
+                const uint32_t g = pk_min_u(pk_sub_sat(pp[q], mx[q]), one);
+                kx[q] = pk_max_u(kx[q], pk_mad(g, static_cast<uint32_t>(k) * 0x10001u, 0u));
+                mx[q] = pk_max_u(mx[q], pp[q]);
+              }
+              k_left = l1 > left ? static_cast<uint32_t>(k) : k_left;
+              left = max(left, l1);
+            }
+          }
+          ack = (kx[0] << 2) | kx[1];
+        }
+        band_scores(mx, left, sub, gap_pair, lane, lo, excl, cur, &cur_left, bd, bv);
+        const uint32_t own = (d >> kRecOwnShift) & 31u;
+        if (own != static_cast<uint32_t>(kSlotNone)) {
+          const uint32_t at = lds + own * row_bytes;
+          *(LPair*)(size_t)(at + 8 + 8 * static_cast<uint32_t>(lane)) = U32x2{cur[0], cur[1]};
+          if (lane == 0) *(LHalf*)(size_t)(at + 6) = static_cast<uint16_t>(cur_left);
+        }
+        uint32_t acc[1];
+        row_kinds<kBandW>(cur, bd, bv, acc);
+        GByte* at = record + ((lo >> 2) + 1 + lane) * 2;
+        const uint32_t a = (acc[0] | (acc[0] >> 12)) & 0xffu;
+        const uint32_t k = (ack | (ack >> 12)) & 0xffu;
+        *(GHalf*)at = static_cast<uint16_t>(a | (k << 8));
+        if (np > 1 && lane == 0) record[(lo >> 2) * 2 + 1] = static_cast<uint8_t>(k_left << 4);
       } else {
-        uint32_t mx[2], kx[2] = {0u, 0u};
-        uint32_t m0 = load_band(ring, pitch, s, pred_at(0), lo, V, L, lane, mx);
-        uint32_t k0 = 0;
-        for (int k = 1; k < np; ++k) {
-          uint32_t pp[2];
-          const uint32_t hk = load_band(ring, pitch, s, pred_at(k), lo, V, L, lane, pp);
+        // the general form, as in dp_rows
+        const int off = __builtin_amdgcn_readlane(off_v, rr);
+        const int n_preds = __builtin_amdgcn_readlane(end_v, rr) - off;
+        const int meta = __builtin_amdgcn_readlane(meta_v, rr);
+        const int own = (meta >> kRowMetaSlotShift) & 31;
+        const int j0 = lo + 1 + kBandW * lane;
+        uint32_t mx[2] = {0u, 0u}, kx[2] = {0u, 0u}, left = 0u, k_left = 0u;
+        for (int k = 0; k < n_preds; ++k) {
+          const int idx = off + k - base;
+          int e;
+          if (idx < kWave) {
+            e = __builtin_amdgcn_readlane(pr0, idx);
+          } else if (idx < 2 * kWave) {
+            e = __builtin_amdgcn_readlane(pr1, idx - kWave);
+          } else {
+            e = uniform(s.pred_rows()[off + k]);
+          }
+          const int p = e & kPredRowMask;
+          const int sl = static_cast<int>(static_cast<unsigned>(e) >> kPredRowBits);
+          uint32_t pp[2], l1;
+          if (p == 0) {
+            pp[0] = pp[1] = kBandBias * 0x10001u;
+            l1 = kBandBias;
+          } else {
+            const int lo_p = band_lo(p, V, L);
+            if (sl < kSlotGlobal) {
+              band_load(lds + static_cast<uint32_t>(sl) * row_bytes, lane,
+                        min(max(lo - lo_p, 0) >> 2, kWave + 1), pp, &l1);
+            } else {
+              // a row kept in the slot's global matrix (absolute columns)
+              const int32_t* row = s.H_row(p, pitch);
+              uint32_t v[kBandW + 1];
+#pragma unroll
+              for (int u = 0; u <= kBandW; ++u) {
+                const int j = j0 - 1 + u;
+                const bool valid = (j > lo_p && j <= lo_p + kBand && j <= L) || (j == 0 && lo_p == 0);
+                v[u] = valid ? static_cast<uint32_t>(row[j]) & 0xffffu : kBandNeg;
+              }
+              wait_stores();
+              pp[0] = v[1] | v[2] << 16;
+              pp[1] = v[3] | v[4] << 16;
+              l1 = __builtin_amdgcn_readlane(static_cast<int>(v[0]), 0);
+            }
+          }
           const uint32_t ks = static_cast<uint32_t>(k) * 0x10001u;
 #pragma unroll
           for (int q = 0; q < 2; ++q) {
-            const uint32_t m = pk_max(mx[q], pp[q]);
-            kx[q] = pk_mad(pk_min_u(pk_sub(m, mx[q]), ps.one), pk_sub(ks, kx[q]), kx[q]);
-            mx[q] = m;
+            const uint32_t g = pk_min_u(pk_sub_sat(pp[q], mx[q]), one);
+            kx[q] = pk_mad(g, pk_sub(ks, kx[q]), kx[q]);
+            mx[q] = pk_max_u(mx[q], pp[q]);
           }
-          const uint32_t m = pk_max(m0, hk);
-          k0 = pk_mad(pk_min_u(pk_sub(m, m0), ps.one), pk_sub(ks, k0), k0);
-          m0 = m;
+          k_left = l1 > left ? static_cast<uint32_t>(k) : k_left;
+          left = max(left, l1);
         }
-        h_last = band_row<true>(ps, mx, m0, kx, k0, b, 0u, lane, lo, L, gap, own, pitch, ring,
-                                Hg, Cr);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          uint32_t x = 0;
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const int idx = j0 + 2 * q + u - 1;
+            const bool same = idx < L && static_cast<int>(seq[idx]) == (meta & 0xff);
+            x |= (static_cast<uint32_t>((same ? match : mismatch) - gap) & 0xffffu) << (16 * u);
+          }
+          sub[q] = x;
+        }
+        band_scores(mx, left, sub, gap_pair, lane, lo, excl, cur, &cur_left, bd, bv);
+        if (own < kSlotGlobal) {
+          const uint32_t at = lds + static_cast<uint32_t>(own) * row_bytes;
+          *(LPair*)(size_t)(at + 8 + 8 * static_cast<uint32_t>(lane)) = U32x2{cur[0], cur[1]};
+          if (lane == 0) *(LHalf*)(size_t)(at + 6) = static_cast<uint16_t>(cur_left);
+        } else if (own == kSlotGlobal) {
+          int32_t* Hg = s.H_row(r, meta, pitch);
+#pragma unroll
+          for (int u = 0; u < kBandW; ++u) {
+            if (j0 + u <= L) Hg[j0 + u] = static_cast<int32_t>((cur[u / 2] >> (16 * (u & 1))) & 0xffffu);
+          }
+          if (lane == 0) Hg[0] = static_cast<int32_t>(cur_left);
+          wait_stores();
+          wave_fence();
+        }
+        // 16-bit codes, column j at element j + 3
+        const uint32_t kprev = shift_into(k_left << 16, kx[1]);
+        uint16_t* Cr = s.code() + static_cast<int64_t>(r) * pitch;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const uint32_t kd = __builtin_amdgcn_alignbit(kx[q], q == 0 ? kprev : kx[0], 16);
+          uint32_t code = 0;
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const uint32_t hu = (cur[q] >> (16 * u)) & 0xffffu;
+            const bool dg = ((bd[q] >> (16 * u)) & 0xffffu) == hu;
+            const bool vt = ((bv[q] >> (16 * u)) & 0xffffu) == hu;
+            const uint32_t kdu = (kd >> (16 * u)) & 0xffffu, kvu = (kx[q] >> (16 * u)) & 0xffffu;
+            const uint32_t c = dg ? (kCodeDiag | kCodeViaK | kdu)
+                                  : (vt ? (kCodeVert | kCodeViaK | kvu) : kCodeHorz);
+            code |= c << (16 * u);
+          }
+          *reinterpret_cast<uint32_t*>(Cr + j0 + kBandColumn + 2 * q) = code;
+        }
+        if (lane == 0 && lo == 0) {
+          Cr[kBandColumn] = static_cast<uint16_t>(kCodeVert | kCodeViaK | k_left);
+        }
       }
-      if ((meta & kRowMetaSink) != 0) {
+      if ((d & kRecSink) != 0) {
+        const int e = L - 1 - lo;  // column L in the band: lane e / 4, column e % 4
+        int32_t h_last = kNegInf;
+        if (e >= 0 && e < kBand) {
+          const uint32_t w = (e & 2) != 0 ? cur[1] : cur[0];
+          const uint32_t g = static_cast<uint32_t>(
+              __builtin_amdgcn_readlane(static_cast<int>(w), e / kBandW));
+          h_last = static_cast<int32_t>((e & 1) ? g >> 16 : g & 0xffffu) -
+                   static_cast<int32_t>(kBandBias) + L * gap;
+        }
         if (lane == 0) s.sink_score()[r] = h_last;
         if (h_last > best) {
           best = h_last;
@@ -1487,8 +1516,8 @@ __device__ __forceinline__ int dp_layer_band(CParams& P, const Slot& s, uint8_t*
           ++ties;
         }
       }
-      if (own == kSlotGlobal) wait_stores();
-      wave_fence();
+      record += row_bytes;
+      wave_fence();  // (a lane reads what another lane wrote)
     }
   }
   *best_score = best;
@@ -1546,7 +1575,7 @@ __device__ __noinline__ uint64_t dp_layer_call(CParams* params, GByte* base, CLa
   } else if constexpr (kKind == kDpRows20) {
     row = dp_rows<20>(P, s, lds_addr, V, L, bias, &best_score, &tied);
   } else if constexpr (kKind == kDpBand4) {
-    row = dp_layer_band(P, s, lds, V, L, &best_score, &tied);
+    row = dp_band(P, s, lds_addr, V, L, &best_score, &tied);
   } else if constexpr (kKind == kDpGeneric16) {
     row = dp_layer<int16_t>(P, s, lds, V, L, &best_score, &tied);
   } else {
@@ -2001,10 +2030,10 @@ __device__ __forceinline__ int32_t wave_prefix_sum(int32_t x) {
 // reader of every row in LDS with an atomic maximum, so no out-edge list is
 // walked. The second pass goes over 64 rows at a time, with the next rows
 // already loaded: slots one row after the other (ten instructions each), then
-// records and lists from the slots kept in LDS. With `records` (dp_rows) a row
-// whose only reader is the next row, which reads nothing else, takes no slot
-// (the DP still holds it in registers), and only rows of the general form get
-// a predecessor list. Walking both edge lists of every row instead took
+// records and lists from the slots kept in LDS. With `records` (1 dp_rows, 2
+// band rows) only rows of the general form get a predecessor list, and in
+// dp_rows a row whose only reader is the next row, which reads nothing else,
+// takes no slot (the DP still holds it in registers). Walking both edge lists of every row instead took
 // 187 us a layer in a full batch of 500 bp windows at 52 layers and 79 us
 // alone; this takes 146 and 67.
 __device__ __noinline__ int build_rows(GByte* slot_base, CLayout* layout, int V, int n_slots,
@@ -2150,7 +2179,7 @@ __device__ __noinline__ int build_rows(GByte* slot_base, CLayout* layout, int V,
         last = max(last, row_of[s.e_head()[e]]);
       }
     }
-    const bool chained = records != 0 && last == r + 2 && ((after >> 8) & 0xff) == 1;
+    const bool chained = records == 1 && last == r + 2 && ((after >> 8) & 0xff) == 1;
     int my_slot = kSlotNone;
     int my_pool = 0;
     for (unsigned long long need = __ballot(in && last != 0 && !chained); need != 0;
@@ -2188,7 +2217,7 @@ __device__ __noinline__ int build_rows(GByte* slot_base, CLayout* layout, int V,
     }
     const bool sink = last == 0;
     if (in) {
-      row_meta[r] = letter | (sink ? kRowMetaSink : 0) | (np <= 1 ? kRowMetaSingle : 0) |
+      row_meta[r] = letter | (sink ? kRowMetaSink : 0) |
                     (my_slot << kRowMetaSlotShift) | (my_pool << kRowMetaGShift);
       if (words) {
         word[r] = static_cast<uint32_t>(my_slot);
@@ -2464,7 +2493,8 @@ __device__ __noinline__ int include_ranks(GByte* slot_base, CLayout* layout, uin
 // Traceback over the move records of dp_rows (W <= 16), from the end cell
 // (row, L) up to the virtual start row; the graph node of the diagonal move
 // into column p + 1, or -1 for a horizontal one, goes to path()[p] (s.path).
-// Returns the column reached in row 0, or -1 when a move leads outside.
+// Returns the column reached in row 0, -1 when a move leads outside, or, over
+// band rows (kBanded, V DP rows), -2 when one leaves the band.
 //
 // A tile is 64 rows, one per lane, and the columns of the last few strip
 // records at and before the current one: one round trip brings every row's
@@ -2475,13 +2505,16 @@ __device__ __noinline__ int include_ranks(GByte* slot_base, CLayout* layout, uin
 // columns with successor indices per cell took 66 round trips a layer of 490
 // columns instead of 20, 106 us alone and 216 us in a full batch.) Rows of the
 // general form are decoded one move at a time.
-template <int W>
-__device__ __noinline__ int trace_rows(GByte* slot_base, CLayout* layout, int pitch, int L, int row,
-                                       int plain) {
+template <int W, bool kBanded>
+__device__ __noinline__ int trace_rows(GByte* slot_base, CLayout* layout, int pitch, int V, int L,
+                                       int row, int plain) {
   static_assert(W == 4 || W == 8 || W == 12 || W == 16, "strip width");
   const Slot s = carve(uniform_ptr(slot_base), *uniform_ptr(layout));
   pitch = uniform(pitch);
   plain = uniform(plain);
+  V = uniform(V);
+  const int length = uniform(L);
+  constexpr int kShift = kBanded ? kBandColumn : 0;  // record column of column j: j + kShift
   const int lane = lane_id();
   constexpr int kRecord = W == 4 ? 2 : W == 8 ? 4 : 8;  // bytes
   constexpr int kRecords = 16 / kRecord;                // records of a tile
@@ -2494,7 +2527,7 @@ __device__ __noinline__ int trace_rows(GByte* slot_base, CLayout* layout, int pi
     const int ri = i0 - lane;
     const int rc = max(ri, 1);
     const GByte* mrow = codes + static_cast<int64_t>(rc) * pitch * 2;
-    const int q = j0 / W;
+    const int q = (j0 + kShift) / W;
     const int first = max(0, q - (kRecords - 1));  // first record of the tile
     U32x4 w;
     __builtin_memcpy(&w, (const uint8_t*)(mrow + first * kRecord), 16);
@@ -2553,8 +2586,14 @@ __device__ __noinline__ int trace_rows(GByte* slot_base, CLayout* layout, int pi
         preds = static_cast<uint64_t>(order(r[3])) << (2 * W) | order(r[1]);
       }
     }
+    if (kBanded) {
+      // column 0 is always vertical; records of rows with one predecessor
+      // leave the index left of the band unwritten
+      if (first == 0) kinds = (kinds & ~(3ull << (2 * kShift))) | 2ull << (2 * kShift);
+      if ((rec.x & kRecPreds) == 1) preds = 0;
+    }
     // the current column's field on top
-    const int at = j0 - first * W;
+    const int at = j0 + kShift - first * W;
     kinds <<= 62 - 2 * at;
     preds <<= 62 - 2 * at;
     // lanes that end the walk inside the tile: rows of the general form and
@@ -2563,6 +2602,8 @@ __device__ __noinline__ int trace_rows(GByte* slot_base, CLayout* layout, int pi
     const int node_v = static_cast<int>(rec.y | (stop ? 0x80000000u : 0u));
     // columns the tile can step: a diagonal also reads the column before
     const int columns = first == 0 ? j0 + 1 : at;
+    const int lo_v = kBanded ? band_lo(rc, V, length) : 0;
+    int left_band = 0;
     int out = -1;  // lane t: the node of position j0 - 1 - t
     int l = 0, t = 0;
     int stopped = 0;
@@ -2593,14 +2634,27 @@ __device__ __noinline__ int trace_rows(GByte* slot_base, CLayout* layout, int pi
       kinds <<= 2 * step;
       preds <<= 2 * step;
       if (((kWave - 1 - l) | (columns - 1 - t)) < 0) break;
+      if (kBanded) {
+        // (rows past the start hold every column)
+        const int lo = __builtin_amdgcn_readlane(lo_v, l);
+        const uint32_t into = static_cast<uint32_t>(j0 - t - lo - 1);
+        if (into >= static_cast<uint32_t>(kBand) && i0 - l > 0 && !(j0 == t && lo == 0)) {
+          left_band = 1;
+          break;
+        }
+      }
     }
     i = i0 - l;
     j = j0 - t;
     if (lane < t && j0 - 1 - lane >= 0) pos_node[j0 - 1 - lane] = out;
     if (i < 0 || j < 0) return -1;
+    if (kBanded && i > 0) {
+      const int lo = uniform(band_lo(i, V, length));
+      if (left_band != 0 || !((j > lo && j <= lo + kBand) || (j == 0 && lo == 0))) return -2;
+    }
     if (i > 0 && stopped != 0) {
       // one move of a row of the general form, from its 16-bit code
-      const int c = uniform(static_cast<int>(s.code()[static_cast<int64_t>(i) * pitch + j]));
+      const int c = uniform(static_cast<int>(s.code()[static_cast<int64_t>(i) * pitch + j + kShift]));
       const int kind = c & 0xc000;
       if (kind == 0xc000 || (kind != kCodeVert && j == 0)) return -1;
       if (kind != kCodeVert) {
@@ -2624,6 +2678,10 @@ __device__ __noinline__ int trace_rows(GByte* slot_base, CLayout* layout, int pi
         if (delta <= 0) return -1;
         i -= delta;
         if (i < 0) return -1;
+      }
+      if (kBanded && i > 0) {
+        const int lo = uniform(band_lo(i, V, length));
+        if (!((j > lo && j <= lo + kBand) || (j == 0 && lo == 0))) return -2;
       }
     }
   }
@@ -3010,7 +3068,7 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
     const int ring_bytes = static_cast<int>(P.ring_rows) * pitch * 2;
     const int max_np =
         uniform(build_rows(s.p, s.L, V, n_slots, rows_lds, ring_bytes,
-                           rows16 && P.band == 0 && layer_plain ? 1 : 0));
+                           !rows16 || !layer_plain ? 0 : P.band != 0 && L > kBand ? 2 : 1));
     wave_sync();
     if (max_np < 0) {
       R.status = kPoaRowOverflow;  // the pooled global rows ran out: rerun exactly
@@ -3034,8 +3092,8 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
     // opaque to the optimizer: otherwise the callee would rebuild the address
     // from the dynamic LDS symbol (a table load) inside its loops
     asm volatile("" : "+v"(lds_addr));
-    // racon -b: band rows for layers longer than the band (approximation);
-    // their pairs keep H - j * gap in signed 16 bits
+    // racon -b: band rows for layers longer than the band (approximation),
+    // while their scores fit signed 16 bits
     const bool banded = P.band != 0 && L > kBand && max_abs <= 4096 && max_np <= 255 &&
                         static_cast<int64_t>(max_abs) * (V + 2 * L + 2) < 32000;
     // columns per lane of the packed rows
@@ -3111,15 +3169,16 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
     // the predecessor lists) is taken by the full single-step decoder. The
     // block's positions are collected in one register (lane t: position
     // j0 - 1 - t) and stored together.
-    if (rows16 && !banded && row_w <= 16) {
+    if (banded || (rows16 && row_w <= 16)) {
       const int plain = layer_plain ? 1 : 0;
       const int left = uniform(
-          row_w == 4    ? trace_rows<4>(s.p, s.L, pitch, L, best_row, plain)
-          : row_w == 8  ? trace_rows<8>(s.p, s.L, pitch, L, best_row, plain)
-          : row_w == 12 ? trace_rows<12>(s.p, s.L, pitch, L, best_row, plain)
-                        : trace_rows<16>(s.p, s.L, pitch, L, best_row, plain));
+          banded        ? trace_rows<4, true>(s.p, s.L, pitch, V, L, best_row, plain)
+          : row_w == 4  ? trace_rows<4, false>(s.p, s.L, pitch, V, L, best_row, plain)
+          : row_w == 8  ? trace_rows<8, false>(s.p, s.L, pitch, V, L, best_row, plain)
+          : row_w == 12 ? trace_rows<12, false>(s.p, s.L, pitch, V, L, best_row, plain)
+                        : trace_rows<16, false>(s.p, s.L, pitch, V, L, best_row, plain));
       if (left < 0) {
-        R.status = kPoaBadInput;
+        R.status = left == -2 ? kPoaBandMiss : kPoaBadInput;
         return;
       }
       // from the virtual start row only horizontal moves remain
@@ -3129,10 +3188,7 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
       const int32_t* pred_off = s.pred_off();
       const int32_t* pred_rows = s.pred_rows();
       const uint4* row_rec = s.row_rec();
-      const int32_t* row_meta = s.row_meta();
-      // the packed rows keep move records, the band rows move kinds for rows
-      // with one predecessor
-      const bool records = rows16 && !banded;
+      const bool records = rows16;
       const int record_half = row_record_bytes(row_w) / 2;
       const int row_inv = 65536 / row_w + 1;
       int32_t* pos_node = s.path();
@@ -3142,7 +3198,6 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
       int steps = 0;
       const int step_cap = uniform(V + L + 1);  // every move lowers i or j
       bool bad = false;
-      bool band_miss = false;
       while (i > 0 && !bad) {
         i = uniform(i);
         j = uniform(j);
@@ -3185,23 +3240,8 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
           }
         } else {
           rec = row_rec[rc - 1];
-          if (banded && (row_meta[rc - 1] & kRowMetaSingle) != 0) {
-            // a one-predecessor band row: its 2-bit move kinds, turned into
-            // the codes of moves to in-edge 0
-            const uint8_t* krow = reinterpret_cast<const uint8_t*>(crow);
-            auto kind_code = [&](int j) -> uint32_t {
-              if (j <= 0) return kCodeVert | kCodeViaK;
-              const uint32_t k =
-                  (static_cast<uint32_t>(krow[(j - 1) >> 2]) >> (2 * ((j - 1) & 3))) & 3u;
-              return k == kKindHorz ? kCodeHorz
-                                    : ((k == kKindVert ? kCodeVert : kCodeDiag) | kCodeViaK);
-            };
-            c0 = kind_code(cj);
-            c1 = kind_code(cj - 1);
-          } else {
-            c0 = crow[code_index(max(cj, 0), pitch)];
-            c1 = crow[code_index(max(cj - 1, 0), pitch)];
-          }
+          c0 = crow[code_index(max(cj, 0), pitch)];
+          c1 = crow[code_index(max(cj - 1, 0), pitch)];
         }
         const uint64_t d4 = static_cast<uint64_t>(rec.w) << 32 | rec.z;
         const int nrow = static_cast<int>(rec.y);  // graph node of the row
@@ -3228,9 +3268,6 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
             if (kind == kCodeDiag) ndj = dj + 1;
           }
           if (ndi >= 16 || ndj >= 8 || i0 - ndi <= 0) return kNextExit;
-          // band rows: a move out of the band is left to the decoder, which
-          // stops the walk there
-          if (banded && !in_band(i0 - ndi, j0 - ndj, V, L)) return kNextExit;
           return static_cast<uint32_t>(ndi * 8 + ndj) | (kind == kCodeDiag ? kDiagBit : 0u);
         };
         const int dja = 2 * (lane & 3);
@@ -3285,14 +3322,13 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
             i -= delta;
             bad = i < 0;
           }
-          if (!bad && banded && !in_band(i, j, V, L)) band_miss = bad = true;
         }
         if (lane < j0 - j) {
           pos_node[j0 - 1 - lane] = out;
         }
       }
       if (bad) {
-        R.status = band_miss ? kPoaBandMiss : kPoaBadInput;
+        R.status = kPoaBadInput;
         return;
       }
       // from the virtual start row only horizontal moves remain
