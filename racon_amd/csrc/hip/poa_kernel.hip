@@ -733,12 +733,13 @@ __device__ __forceinline__ uint32_t pk_splat(int32_t v) {
 // other than A, C, G, T) store 16-bit codes, column j at element j.
 //
 // The rows are bound by their instructions: a wave alone issues one about
-// every 8 cycles, and 4 waves per SIMD share the issue slots. A row with one
-// predecessor takes about 70 vector and 25 scalar instructions at W = 8
-// (the form before, with per-row predecessor lists, a separate column 0 and
-// 16-bit codes for rows of several predecessors, took 117 and 95 over all
-// rows). One 500 bp window at 30 layers: DP 17.5 -> 8.5 ms; 9,980 windows of
-// 500 bp at 52 layers: DP 521 -> 282 wave-seconds, kernel 250 -> 176 ms.
+// every 8 cycles, and 4 waves per SIMD share the issue slots. A row whose one
+// predecessor is the row before takes 93 instructions at W = 8, 22 of them
+// scalar (the form with per-row predecessor lists, a separate column 0 and
+// 16-bit codes took 212 over all rows; the one that prepared each row's
+// scores at its own start, with no-ops in the gaps of the chain, 122). One
+// 500 bp window at 30 layers: DP 17.5 -> 8.5 -> 6.8 ms; 9,980 windows of
+// 500 bp at 52 layers: DP 521 -> 291 -> 252 wave-seconds.
 
 // Row descriptor: number of predecessors (0: the general form), 8 x the code
 // of the row's base, own slot, slots of up to four predecessors, whether the
@@ -831,18 +832,29 @@ __device__ __forceinline__ void lds_row_store(uint32_t at, const uint32_t* v) {
 
 // Inclusive prefix max over the lanes of unsigned words (0 is the identity,
 // which lanes without a source read).
-__device__ __forceinline__ uint32_t wave_prefix_max_u(uint32_t x) {
+// fill(x, k), k = 0..5, is called after each step.
+template <typename Fill>
+__device__ __forceinline__ uint32_t wave_prefix_max_u(uint32_t x, Fill fill) {
   const auto step = [](uint32_t v, auto ctrl, auto rows) {
     return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(
         0, static_cast<int>(v), decltype(ctrl)::value, decltype(rows)::value, 0xf, false));
   };
   x = max(x, step(x, std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{}));
+  fill(x, 0);
   x = max(x, step(x, std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{}));
+  fill(x, 1);
   x = max(x, step(x, std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{}));
+  fill(x, 2);
   x = max(x, step(x, std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{}));
+  fill(x, 3);
   x = max(x, step(x, std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{}));
+  fill(x, 4);
   x = max(x, step(x, std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{}));
+  fill(x, 5);
   return x;
+}
+__device__ __forceinline__ uint32_t wave_prefix_max_u(uint32_t x) {
+  return wave_prefix_max_u(x, [](uint32_t&, int) {});
 }
 
 // x of the previous lane; lane 0 keeps its value of `old` (a register that
@@ -852,30 +864,60 @@ __device__ __forceinline__ uint32_t shift_into(uint32_t old, uint32_t x) {
       static_cast<int>(old), static_cast<int>(x), 0x138, 0xf, 0xf, false));
 }
 
-// One row from its best predecessor scores pp: diagonal (scores sub from the
-// letters) and vertical candidates, horizontal chain, scores into h, move
-// kinds into acc. prev and excl carry the lane-0 constants between rows.
-template <int W>
-__device__ __forceinline__ void row_scores(const uint32_t* pp, const uint32_t* sub,
-                                           uint32_t gap_pair, uint32_t& prev, uint32_t& excl,
-                                           uint32_t* h, uint32_t* bd, uint32_t* bv) {
+// Ties a value to its place among the other pinned ones (no instruction).
+__device__ __forceinline__ void pin(uint32_t& x) { asm volatile("" : "+v"(x)); }
+__device__ __forceinline__ void pin_scalar(uint32_t& x) { asm volatile("" : "+s"(x)); }
+
+// x of the previous lane, 0 in lane 0.
+__device__ __forceinline__ uint32_t shift_lanes(uint32_t x) {
+  return static_cast<uint32_t>(
+      __builtin_amdgcn_update_dpp(0, static_cast<int>(x), 0x138, 0xf, 0xf, true));
+}
+
+// One row from its best predecessor scores in h: diagonal (scores sub from
+// the letters; lane 0's column 0 has no letter: its first half is 0, which
+// keeps the diagonal below every score) and vertical candidates, horizontal
+// chain, scores into h.
+//
+// A packed instruction's result is read by the second instruction after it at
+// the earliest, a lane's by a DPP read in the third: the pairs go through each
+// step together, and fill(k), k = 0..8, issues a part of the next row's work
+// (one or two instructions, free of this row's results) in the gaps of the
+// chain and of the prefix max, which would be no-ops otherwise.
+template <int W, typename Fill>
+__device__ __forceinline__ void row_scores(uint32_t* h, const uint32_t* sub, uint32_t gap_pair,
+                                           uint32_t* bd, uint32_t* bv, Fill fill) {
   constexpr int H2 = W / 2;
-  prev = shift_into(prev, pp[H2 - 1]);
+  const uint32_t prev = shift_lanes(h[H2 - 1]);
   uint32_t pre[H2];
-  uint32_t carry = 0;
+#pragma unroll
+  for (int q = 0; q < H2; ++q) bv[q] = pk_add(h[q], gap_pair);
 #pragma unroll
   for (int q = 0; q < H2; ++q) {
     // G[p][j - 1] of the pair
-    const uint32_t d = __builtin_amdgcn_alignbit(pp[q], q == 0 ? prev : pp[q - 1], 16);
-    bd[q] = pk_add(d, sub[q]);
-    bv[q] = pk_add(pp[q], gap_pair);
-    const uint32_t t = pk_scan_u(pk_max_u(bd[q], bv[q]));
-    carry = q == 0 ? t : pk_max_hi_u(t, carry);
-    pre[q] = carry;
+    pre[q] = __builtin_amdgcn_alignbit(h[q], q == 0 ? prev : h[q - 1], 16);
+  }
+#pragma unroll
+  for (int q = 0; q < H2; ++q) bd[q] = pk_add(pre[q], sub[q]);
+#pragma unroll
+  for (int q = 0; q < H2; ++q) pre[q] = pk_max_u(bd[q], bv[q]);
+#pragma unroll
+  for (int q = 0; q < H2; ++q) pre[q] = pk_scan_u(pre[q]);
+#pragma unroll
+  for (int q = 0; q < H2; ++q) pin(pre[q]);
+#pragma unroll
+  for (int q = 1; q < H2; ++q) {
+    pre[q] = pk_max_hi_u(pre[q], pre[q - 1]);
+    pin(pre[q]);
+    if (q >= H2 - 3) fill(q - H2 + 3);
   }
   // (the whole word goes through the scan: its high half, the strip's
   // maximum, decides)
-  excl = shift_into(excl, wave_prefix_max_u(carry));
+  const uint32_t excl = shift_lanes(
+      wave_prefix_max_u(pre[H2 - 1], [&](uint32_t& x, int k) {
+        pin(x);
+        fill(3 + k);
+      }));
 #pragma unroll
   for (int q = 0; q < H2; ++q) h[q] = pk_max_hi_u(pre[q], excl);
 }
@@ -922,7 +964,8 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
       const int c = idx >= 0 && idx < L ? static_cast<int>(seq[idx]) : 'A';
       const int code = ((c >> 1) ^ (c >> 2)) & 3;
       plain &= static_cast<int>((0x54474341u >> (8 * code)) & 0xffu) == c;
-      x |= (static_cast<uint32_t>(code) * 0x0101u + 0x0400u) << (16 * u);
+      // (a selector byte of 0x0c gives 0: column 0)
+      x |= (idx < 0 ? 0x0c0cu : static_cast<uint32_t>(code) * 0x0101u + 0x0400u) << (16 * u);
     }
     sel[q] = x;
   }
@@ -935,13 +978,10 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
   const uint64_t table0 = static_cast<uint64_t>((miss >> 8) * 0x01010101u) << 32 |
                           (miss & 0xffu) * 0x01010101u;
   const uint64_t table1 = static_cast<uint64_t>(flip >> 8) << 32 | (flip & 0xffu);
-  const int max_abs = max(max(abs(match), abs(mismatch)), abs(gap));
   // 1 in both halves, opaque to the optimizer (a visible 1 turns min(x, 1)
   // into compares and selects per half)
   uint32_t one = 0x00010001u;
   asm volatile("" : "+s"(one));
-  uint32_t prev = pk_splat(2 * max_abs);  // lane 0: column -1, below every score
-  uint32_t excl = 0;                      // lane 0: nothing to its left
   const int end_lane = L / W, end_u = L % W;
   int32_t best = kNegInf;
   int best_row = 0;
@@ -951,16 +991,18 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
 #pragma unroll
   for (int q = 0; q < H2; ++q) cur[q] = 0;
   GByte* const codes = (GByte*)s.code();
-  const uint32_t rec_lane = static_cast<uint32_t>(lane * row_record_bytes(W));
-  for (int r0 = 1; r0 <= V; r0 += kWave) {
+  uint32_t rec_lane = static_cast<uint32_t>(lane * row_record_bytes(W));
+  // (chunks of 63 rows: the last lane's descriptor is 0 and ends the row loop)
+  constexpr int kChunk = kWave - 1;
+  for (int r0 = 1; r0 <= V; r0 += kChunk) {
     const int rk = r0 + lane;
     uint32_t desc_v = 0;
-    if (rk <= V) desc_v = s.row_rec()[rk - 1].x;
+    if (lane < kChunk && rk <= V) desc_v = s.row_rec()[rk - 1].x;
     if (!layer_plain) desc_v &= ~(kRecPreds | kRecChain);
-    const int chunk = uniform(min(kWave, V - r0 + 1));
+    const int chunk = uniform(min(kChunk, V - r0 + 1));
     // what the rows of the general form need of this chunk
     int off_v = 0, end_v = 0, meta_v = 0, base = 0, pr0 = 0, pr1 = 0;
-    if (__any(rk <= V && (desc_v & kRecPreds) == 0)) {
+    if (__any(lane < kChunk && rk <= V && (desc_v & kRecPreds) == 0)) {
       if (rk <= V) {
         off_v = s.pred_off()[rk - 1];
         end_v = s.pred_off()[rk];
@@ -974,55 +1016,91 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
     // them (and for every store issued before them) on each row
     wait_stores();
     if (lane < n_live) {
-      GByte* record = codes + static_cast<int64_t>(r0) * row_bytes;
-      for (int rr = 0; rr < chunk; ++rr) {
-        const uint32_t d = static_cast<uint32_t>(
-            __builtin_amdgcn_readlane(static_cast<int>(desc_v), rr));
-        const uint32_t np = d & kRecPreds;
-        uint32_t bd[H2], bv[H2];
-        if (np != 0) {
+      GByte* record = codes + static_cast<int64_t>(r0 - 1) * row_bytes;  // of the row before
+      // the next row's descriptor and substitution scores, a piece at a time
+      uint32_t d = 0, d_next = 0;
+      uint64_t table = 0;
+      uint32_t sub[H2];
+      const auto next_desc = [&](int rr) {
+        d_next = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(desc_v), rr));
+        pin_scalar(d_next);
+      };
+      const auto next_table = [&]() {
+        table = table0 ^ (table1 << (d_next & kRecBase));
+        asm volatile("" : "+s"(table));
+      };
+      const auto next_sub = [&](int q) {
+        sub[q] = __builtin_amdgcn_perm(static_cast<uint32_t>(table >> 32),
+                                       static_cast<uint32_t>(table), sel[q]);
+        pin(sub[q]);
+      };
+      const auto next_row = [&](int rr) {
+        next_desc(rr);
+        next_table();
+#pragma unroll
+        for (int q = 0; q < H2; ++q) next_sub(q);
+        d = d_next;
+      };
+      const auto sink_row = [&](int r) {
+        uint32_t last = cur[0];
+#pragma unroll
+        for (int q = 1; q < H2; ++q) {
+          uint32_t v = cur[q];
+          asm volatile("" : "+v"(v));  // (selected, not indexed through a stack copy)
+          if (q == (end_u >> 1)) last = v;
+        }
+        const uint32_t g = static_cast<uint32_t>(
+            __builtin_amdgcn_readlane(static_cast<int>(last), end_lane));
+        const int32_t h_last =
+            static_cast<int32_t>((end_u & 1) ? g >> 16 : g & 0xffffu) - bias + L * gap;
+        if (lane == 0) s.sink_score()[r] = h_last;
+        if (h_last > best) {
+          best = h_last;
+          best_row = r;
+          ties = 0;
+        } else if (h_last == best) {
+          ++ties;
+        }
+      };
+      next_row(0);
+      int rr = 0;
+      for (;;) {
+        // rows of up to four predecessors (a loop of their own: the common
+        // ones go through without a taken branch)
+        uint32_t np = d & kRecPreds, np_next = 0;
+        while (np != 0) {
           const auto slot_at = [&](int k) {
             return strip + ((d >> (kRecPredShift + 5 * k)) & 31u) * row_bytes;
           };
-          const uint64_t table = table0 ^ (table1 << (d & kRecBase));
-          uint32_t sub[H2];
-#pragma unroll
-          for (int q = 0; q < H2; ++q) {
-            sub[q] = __builtin_amdgcn_perm(static_cast<uint32_t>(table >> 32),
-                                           static_cast<uint32_t>(table), sel[q]);
-          }
-          uint32_t acc[NA], ack[NA];
+          uint32_t bd[H2], bv[H2], acc[NA], ack[NA];
 #pragma unroll
           for (int a = 0; a < NA; ++a) ack[a] = 0;
-          if (np == 1) {
-            if ((d & kRecChain) == 0) lds_row_load<W>(slot_at(0), cur);
-            row_scores<W>(cur, sub, gap_pair, prev, excl, cur, bd, bv);
-          } else {
+          if ((d & kRecChain) == 0) lds_row_load<W>(slot_at(0), cur);
+          if (np > 1) {
             // best predecessor score of each column and the first
             // predecessor reaching it (a later one only when better)
-            uint32_t mx[H2], kx[H2], p1[H2];
-            lds_row_load<W>(slot_at(0), mx);
+            uint32_t kx[H2], p1[H2];
             lds_row_load<W>(slot_at(1), p1);
 #pragma unroll
             for (int q = 0; q < H2; ++q) {
-              kx[q] = pk_min_u(pk_sub_sat(p1[q], mx[q]), one);
-              mx[q] = pk_max_u(mx[q], p1[q]);
+              kx[q] = pk_min_u(pk_sub_sat(p1[q], cur[q]), one);
+              cur[q] = pk_max_u(cur[q], p1[q]);
             }
             if (np > 2) {
               lds_row_load<W>(slot_at(2), p1);
 #pragma unroll
               for (int q = 0; q < H2; ++q) {
-                const uint32_t g = pk_min_u(pk_sub_sat(p1[q], mx[q]), one);
+                const uint32_t g = pk_min_u(pk_sub_sat(p1[q], cur[q]), one);
                 kx[q] = pk_max_u(kx[q], g << 1);
-                mx[q] = pk_max_u(mx[q], p1[q]);
+                cur[q] = pk_max_u(cur[q], p1[q]);
               }
               if (np > 3) {
                 lds_row_load<W>(slot_at(3), p1);
 #pragma unroll
                 for (int q = 0; q < H2; ++q) {
-                  const uint32_t g = pk_min_u(pk_sub_sat(p1[q], mx[q]), one);
+                  const uint32_t g = pk_min_u(pk_sub_sat(p1[q], cur[q]), one);
                   kx[q] = pk_max_u(kx[q], pk_mad(g, 0x00030003u, 0u));
-                  mx[q] = pk_max_u(mx[q], p1[q]);
+                  cur[q] = pk_max_u(cur[q], p1[q]);
                 }
               }
             }
@@ -1030,13 +1108,33 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
             for (int q = 0; q < H2; ++q) {
               ack[q / 8] = (q % 8) == 0 ? kx[q] : (ack[q / 8] << 2) | kx[q];
             }
-            row_scores<W>(mx, sub, gap_pair, prev, excl, cur, bd, bv);
           }
           const uint32_t own = (d >> kRecOwnShift) & 31u;
-          if (own != static_cast<uint32_t>(kSlotNone)) {
-            lds_row_store<W>(strip + own * row_bytes, cur);
-          }
+          uint32_t own_at = 0;
+          row_scores<W>(cur, sub, gap_pair, bd, bv, [&](int k) {
+            if (k == (H2 == 2 ? 2 : 1)) next_desc(rr + 1);
+            if (k == 2) next_table();
+            if (k == 3) {
+              own_at = strip + own * row_bytes;
+              pin(own_at);
+            }
+            constexpr int kShare = (H2 + 2) / 3;  // pairs per gap
+            if (k >= 4 && k < 7) {
+#pragma unroll
+              for (int q = (k - 4) * kShare; q < min(H2, (k - 3) * kShare); ++q) next_sub(q);
+            }
+            if (k == 7) {
+              record += row_bytes;
+              asm volatile("" : "+s"(record));
+            }
+            if (k == 8) {
+              np_next = d_next & kRecPreds;
+              pin_scalar(np_next);
+            }
+          });
+          if (own != static_cast<uint32_t>(kSlotNone)) lds_row_store<W>(own_at, cur);
           row_kinds<W>(cur, bd, bv, acc);
+          pin(rec_lane);  // (stays a 32-bit offset to the uniform row address)
           GByte* at = record + rec_lane;
           if constexpr (W == 4) {
             const uint32_t a = (acc[0] | (acc[0] >> 12)) & 0xffu;
@@ -1050,7 +1148,15 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
           } else {
             *(__attribute__((address_space(1))) U32x4*)at = U32x4{acc[0], acc[1], ack[0], ack[1]};
           }
-        } else {
+          if (__builtin_expect((d & kRecSink) != 0, 0)) sink_row(r0 + rr);
+          ++rr;
+          d = d_next;
+          np = np_next;
+        }
+        if (rr >= chunk) break;
+        record += row_bytes;
+        {
+          uint32_t bd[H2], bv[H2];
           // the general form: any number of predecessors, in LDS, in global
           // memory or the virtual start row; any letters; 16-bit codes
           const int r = r0 + rr;
@@ -1102,7 +1208,7 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
               mx[q] = pk_max_u(mx[q], pp[q]);
             }
           }
-          uint32_t sub[H2];
+          uint32_t scores[H2];
 #pragma unroll
           for (int q = 0; q < H2; ++q) {
             uint32_t x = 0;
@@ -1110,11 +1216,14 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
             for (int u = 0; u < 2; ++u) {
               const int idx = j0 + 2 * q + u - 1;
               const bool same = idx >= 0 && idx < L && static_cast<int>(seq[idx]) == (meta & 0xff);
-              x |= (static_cast<uint32_t>((same ? match : mismatch) - gap) & 0xffffu) << (16 * u);
+              const int v = idx < 0 ? 0 : (same ? match : mismatch) - gap;
+              x |= (static_cast<uint32_t>(v) & 0xffffu) << (16 * u);
             }
-            sub[q] = x;
+            scores[q] = x;
+            // (a move, so that mx and cur need not share registers)
+            asm volatile("v_mov_b32 %0, %1" : "=v"(cur[q]) : "v"(mx[q]));
           }
-          row_scores<W>(mx, sub, gap_pair, prev, excl, cur, bd, bv);
+          row_scores<W>(cur, scores, gap_pair, bd, bv, [](int) {});
           if (own < kSlotGlobal) {
             lds_row_store<W>(strip + static_cast<uint32_t>(own) * row_bytes, cur);
           } else if (own == kSlotGlobal) {
@@ -1143,30 +1252,10 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
             }
             *reinterpret_cast<uint32_t*>(Cr + j0 + 2 * q) = code;
           }
+          if ((d & kRecSink) != 0) sink_row(r);
         }
-        if ((d & kRecSink) != 0) {
-          const int r = r0 + rr;
-          uint32_t last = cur[0];
-#pragma unroll
-          for (int q = 1; q < H2; ++q) {
-            uint32_t v = cur[q];
-            asm volatile("" : "+v"(v));  // (selected, not indexed through a stack copy)
-            if (q == (end_u >> 1)) last = v;
-          }
-          const uint32_t g = static_cast<uint32_t>(
-              __builtin_amdgcn_readlane(static_cast<int>(last), end_lane));
-          const int32_t h_last =
-              static_cast<int32_t>((end_u & 1) ? g >> 16 : g & 0xffffu) - bias + L * gap;
-          if (lane == 0) s.sink_score()[r] = h_last;
-          if (h_last > best) {
-            best = h_last;
-            best_row = r;
-            ties = 0;
-          } else if (h_last == best) {
-            ++ties;
-          }
-        }
-        record += row_bytes;
+        ++rr;
+        next_row(rr);
       }
     }
   }
