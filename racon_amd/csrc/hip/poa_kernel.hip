@@ -758,22 +758,6 @@ constexpr uint32_t kRecMaxPreds = 4;
 // the highest bits (groups of eight column pairs for W > 16).
 __device__ __forceinline__ int row_record_bytes(int W) { return W == 4 ? 2 : W == 8 ? 4 : W <= 16 ? 8 : 16; }
 
-// Byte and bit of column j's kind in the row's record (its predecessor
-// index: half a lane record later).
-struct RecordBit {
-  int byte, bit;
-};
-__device__ __forceinline__ RecordBit record_bit(int j, int W, int inv) {
-  const int ln = (j * inv) >> 16;  // j / W (inv = 65536 / W + 1; j < 4096)
-  const int u = j - ln * W;
-  const int q = u >> 1;
-  const int group = q >> 3;
-  const int pairs = min(8, W / 2 - 8 * group);
-  const int half = W == 4 ? 4 : W == 8 ? 8 : 16;
-  const int at = 32 * group + half * (u & 1) + 2 * (pairs - 1 - (q & 7));
-  return RecordBit{ln * row_record_bytes(W) + (at >> 3), at & 7};
-}
-
 // 16-bit rows hold every value of the layer (see above), with room for the
 // sums formed on the way. bias: the value of G = 0.
 __device__ __forceinline__ bool rows_fit_16(int match, int mismatch, int gap, int V, int L,
@@ -2579,7 +2563,7 @@ __device__ __noinline__ int include_ranks(GByte* slot_base, CLayout* layout, uin
   return 0;
 }
 
-// Traceback over the move records of dp_rows (W <= 16), from the end cell
+// Traceback over the move records of dp_rows, from the end cell
 // (row, L) up to the virtual start row; the graph node of the diagonal move
 // into column p + 1, or -1 for a horizontal one, goes to path()[p] (s.path).
 // Returns the column reached in row 0, -1 when a move leads outside, or, over
@@ -2590,14 +2574,14 @@ __device__ __noinline__ int include_ranks(GByte* slot_base, CLayout* layout, uin
 // record (descriptor, node, predecessor deltas) and 16 or 32 bytes of moves.
 // The lanes put their fields in column order, the current column on top, so
 // that a column step is one shift of the tile and the walk reads its row's
-// move with v_readlane: about 35 instructions a move, most of them scalar. (Tiles of 16 rows x 8
-// columns with successor indices per cell took 66 round trips a layer of 490
-// columns instead of 20, 106 us alone and 216 us in a full batch.) Rows of the
-// general form are decoded one move at a time.
+// move with v_readlane: 29 instructions a move, most of them scalar. (Tiles of
+// 16 rows x 8 columns with successor indices per cell took 66 round trips a
+// layer of 490 columns instead of 20, 106 us alone and 216 us in a full
+// batch.) Rows of the general form are decoded one move at a time.
 template <int W, bool kBanded>
 __device__ __noinline__ int trace_rows(GByte* slot_base, CLayout* layout, int pitch, int V, int L,
                                        int row, int plain) {
-  static_assert(W == 4 || W == 8 || W == 12 || W == 16, "strip width");
+  static_assert(W == 4 || W == 8 || W == 12 || W == 16 || W == 20, "strip width");
   const Slot s = carve(uniform_ptr(slot_base), *uniform_ptr(layout));
   pitch = uniform(pitch);
   plain = uniform(plain);
@@ -2605,8 +2589,8 @@ __device__ __noinline__ int trace_rows(GByte* slot_base, CLayout* layout, int pi
   const int length = uniform(L);
   constexpr int kShift = kBanded ? kBandColumn : 0;  // record column of column j: j + kShift
   const int lane = lane_id();
-  constexpr int kRecord = W == 4 ? 2 : W == 8 ? 4 : 8;  // bytes
-  constexpr int kRecords = 16 / kRecord;                // records of a tile
+  constexpr int kRecord = W == 4 ? 2 : W == 8 ? 4 : W <= 16 ? 8 : 16;  // bytes
+  constexpr int kRecords = W <= 16 ? 16 / kRecord : 2;  // records of a tile
   const GByte* codes = (const GByte*)s.code();
   const uint4* row_rec = s.row_rec();
   int32_t* pos_node = s.path();
@@ -2619,13 +2603,38 @@ __device__ __noinline__ int trace_rows(GByte* slot_base, CLayout* layout, int pi
     const int q = (j0 + kShift) / W;
     const int first = max(0, q - (kRecords - 1));  // first record of the tile
     U32x4 w;
+    [[maybe_unused]] U32x4 w_last;  // W = 20: the current column's record
     __builtin_memcpy(&w, (const uint8_t*)(mrow + first * kRecord), 16);
+    if constexpr (W == 20) __builtin_memcpy(&w_last, (const uint8_t*)(mrow + q * kRecord), 16);
     const uint4 rec = row_rec[rc - 1];
     // fields of columns first * W .. in ascending order (two bits each, the
     // bits of a field swapped: 1 diagonal, 2 vertical; predecessor indices 1
     // and 2 trade places)
     uint64_t kinds, preds;
-    {
+    const int at = j0 + kShift - first * W;
+    if constexpr (W == 20) {
+      // words: kinds of 16 and of 4 columns, then indices; 32 columns end at
+      // the current one, from its record and the one before
+      const auto spread = [](uint32_t x) {  // 16 bits of fields to every second field
+        x = (x | x << 8) & 0x00ff00ffu;
+        x = (x | x << 4) & 0x0f0f0f0fu;
+        return (x | x << 2) & 0x33333333u;
+      };
+      const auto order = [&](uint32_t a, uint32_t b) -> uint64_t {
+        a = __builtin_bitreverse32(a);
+        b = __builtin_bitreverse32(b);
+        const uint32_t low = spread(a >> 16) | spread(a & 0xffffu) << 2;
+        const uint32_t high = spread(b >> 28) | spread((b >> 12) & 0xfu) << 2;
+        return static_cast<uint64_t>(high) << 32 | low;
+      };
+      const int up = 62 - 2 * (j0 - q * W);  // 24..62
+      const auto top = [&](uint64_t before, uint64_t last) -> uint64_t {
+        before = up >= 2 * W ? before << (up - 2 * W) : before >> (2 * W - up);
+        return last << up | (first < q ? before : 0);
+      };
+      kinds = top(order(w.x, w.y), order(w_last.x, w_last.y));
+      preds = top(order(w.z, w.w), order(w_last.z, w_last.w));
+    } else {
       const uint32_t r[4] = {__builtin_bitreverse32(w.x), __builtin_bitreverse32(w.y),
                              __builtin_bitreverse32(w.z), __builtin_bitreverse32(w.w)};
       if constexpr (W == 4) {
@@ -2675,73 +2684,102 @@ __device__ __noinline__ int trace_rows(GByte* slot_base, CLayout* layout, int pi
         preds = static_cast<uint64_t>(order(r[3])) << (2 * W) | order(r[1]);
       }
     }
+    // the current column's field on top
+    if constexpr (W < 20) {
+      kinds <<= 62 - 2 * at;
+      preds <<= 62 - 2 * at;
+    }
     if (kBanded) {
       // column 0 is always vertical; records of rows with one predecessor
       // leave the index left of the band unwritten
-      if (first == 0) kinds = (kinds & ~(3ull << (2 * kShift))) | 2ull << (2 * kShift);
+      const int field = 62 - 2 * j0;
+      if (first == 0) kinds = (kinds & ~(3ull << field)) | 2ull << field;
       if ((rec.x & kRecPreds) == 1) preds = 0;
     }
-    // the current column's field on top
-    const int at = j0 + kShift - first * W;
-    kinds <<= 62 - 2 * at;
-    preds <<= 62 - 2 * at;
+    // A cell takes one move: diagonal before vertical. Its predecessor index is
+    // the one kept at the column before for a diagonal, at its own column for
+    // a vertical.
+    kinds &= ~((kinds & 0x5555555555555555ull) << 1);
+    {
+      const uint64_t diagonal = (kinds & 0x5555555555555555ull) * 3;
+      preds = ((preds << 2) & diagonal) | (preds & ~diagonal);
+    }
+    // the four row deltas as bytes, in the order of the swapped indices; 255
+    // and more lead out of the tile and are made exact after the walk
+    const auto clamp = [](uint32_t x) { return pk_min_u(pk_max_u(x, 0x00010001u), 0x00ff00ffu); };
+    const uint32_t deltas = clamp(rec.z) | clamp(rec.w) << 8;
     // lanes that end the walk inside the tile: rows of the general form and
     // rows past the start (their node's sign bit set)
     const bool stop = ri < 1 || plain == 0 || (rec.x & kRecPreds) == 0;
     const int node_v = static_cast<int>(rec.y | (stop ? 0x80000000u : 0u));
     // columns the tile can step: a diagonal also reads the column before
-    const int columns = first == 0 ? j0 + 1 : at;
+    const int columns = first == 0 && (W < 20 || j0 < 32) ? j0 + 1 : min(at, 31);
     const int lo_v = kBanded ? band_lo(rc, V, length) : 0;
     int left_band = 0;
-    int out = -1;  // lane t: the node of position j0 - 1 - t
-    int l = 0, t = 0;
-    int stopped = 0;
+    int out = -1;  // lane (t - columns) mod 64: the node of position j0 - 1 - t
+    // Rows and columns walked, l and t, in one word: l + 0x8000 - 64 below,
+    // t + 0x8000 - columns above, so that the low bits of each half number
+    // lanes and one test finds the walk at the tile's end.
+    constexpr uint32_t kRow0 = 0x8000u - kWave;
+    const uint32_t col0 = 0x8000u - static_cast<uint32_t>(columns);
+    uint32_t c = col0 << 16 | kRow0;
+    uint32_t delta = 0, index = 0;
+    int node = __builtin_amdgcn_readlane(node_v, 0);
     // (no branch on the kind of move: every move reads the same lanes and
     // selects in scalar registers; a vertical move's -1 in lane t is written
     // over by the move that leaves the column)
-    for (;;) {
-      const int node = __builtin_amdgcn_readlane(node_v, l);
-      if (node < 0) {
-        stopped = 1;
-        break;
-      }
-      uint32_t kx = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(kinds >> 32), l));
-      uint32_t px = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(preds >> 32), l));
-      uint32_t da = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(rec.z), l));
-      uint32_t db = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(rec.w), l));
+    while (((c | (static_cast<uint32_t>(node) & 0x80000000u)) & 0x80008000u) == 0 &&
+           (!kBanded || left_band == 0)) {
+      uint32_t kx = static_cast<uint32_t>(
+          __builtin_amdgcn_readlane(static_cast<int>(kinds >> 32), c & 63u));
+      const uint32_t px = static_cast<uint32_t>(
+          __builtin_amdgcn_readlane(static_cast<int>(preds >> 32), c & 63u));
+      const uint32_t ds = static_cast<uint32_t>(
+          __builtin_amdgcn_readlane(static_cast<int>(deltas), c & 63u));
       // (opaque, so that the tests below stay on one word)
       asm volatile("" : "+s"(kx));
-      const uint32_t kind = kx >> 30;
-      const uint32_t k = px >> ((kind & 1u) != 0 ? 28 : 30);  // (low two bits; 1 and 2 swapped)
-      const uint32_t pair = (k & 1u) != 0 ? db : da;
-      uint32_t delta = max((pair >> ((k & 2u) << 3)) & 0xffffu, 1u);
-      delta = kind != 0 ? delta : 0u;
-      uint32_t step = kind != 2u ? 1u : 0u;
-      out = lane_write((kind & 1u) != 0 ? node : -1, t, out);
-      l += static_cast<int>(delta);
-      t += static_cast<int>(step);
-      kinds <<= 2 * step;
-      preds <<= 2 * step;
-      if (((kWave - 1 - l) | (columns - 1 - t)) < 0) break;
-      if (kBanded) {
+      index = (px >> 27) & 24u;
+      delta = (ds >> index) & 0xffu;
+      delta = kx > 0x3fffffffu ? delta : 0u;
+      out = lane_write((kx & 0x40000000u) != 0 ? node : -1, static_cast<int>(c >> 16) & 63, out);
+      const bool vertical = (kx >> 31) != 0;
+      const uint32_t fields = vertical ? 0u : 2u;
+      c += vertical ? 0u : 0x10000u;
+      c += delta;
+      kinds <<= fields;
+      preds <<= fields;
+      node = __builtin_amdgcn_readlane(node_v, c & 63u);
+      if (kBanded && (c & 0x80008000u) == 0) {
         // (rows past the start hold every column)
+        const int l = static_cast<int>((c & 0xffffu) - kRow0);
+        const int col = j0 - static_cast<int>((c >> 16) - col0);
         const int lo = __builtin_amdgcn_readlane(lo_v, l);
-        const uint32_t into = static_cast<uint32_t>(j0 - t - lo - 1);
-        if (into >= static_cast<uint32_t>(kBand) && i0 - l > 0 && !(j0 == t && lo == 0)) {
+        if (static_cast<uint32_t>(col - lo - 1) >= static_cast<uint32_t>(kBand) && i0 - l > 0 &&
+            !(col == 0 && lo == 0)) {
           left_band = 1;
-          break;
         }
       }
     }
+    const bool stopped = (c & 0x80008000u) == 0;  // at a row that ends the walk
+    int l = static_cast<int>((c & 0xffffu) - kRow0);
+    const int t = static_cast<int>((c >> 16) - col0);
+    asm volatile("" : "+s"(delta));  // (tested here, not on every move)
+    if (delta == 0xffu) {
+      l -= 0xff;
+      const uint32_t pair = static_cast<uint32_t>(__builtin_amdgcn_readlane(
+          static_cast<int>((index & 8u) != 0 ? rec.w : rec.z), l));
+      l += static_cast<int>((index & 16u) != 0 ? pair >> 16 : pair & 0xffffu);
+    }
     i = i0 - l;
     j = j0 - t;
-    if (lane < t && j0 - 1 - lane >= 0) pos_node[j0 - 1 - lane] = out;
+    const int mine = (lane + columns) & (kWave - 1);  // the lane's t
+    if (mine < t && j0 - 1 - mine >= 0) pos_node[j0 - 1 - mine] = out;
     if (i < 0 || j < 0) return -1;
     if (kBanded && i > 0) {
       const int lo = uniform(band_lo(i, V, length));
       if (left_band != 0 || !((j > lo && j <= lo + kBand) || (j == 0 && lo == 0))) return -2;
     }
-    if (i > 0 && stopped != 0) {
+    if (i > 0 && stopped) {
       // one move of a row of the general form, from its 16-bit code
       const int c = uniform(static_cast<int>(s.code()[static_cast<int64_t>(i) * pitch + j + kShift]));
       const int kind = c & 0xc000;
@@ -3258,28 +3296,26 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
     // the predecessor lists) is taken by the full single-step decoder. The
     // block's positions are collected in one register (lane t: position
     // j0 - 1 - t) and stored together.
-    if (banded || (rows16 && row_w <= 16)) {
+    if (banded || rows16) {
       const int plain = layer_plain ? 1 : 0;
       const int left = uniform(
           banded        ? trace_rows<4, true>(s.p, s.L, pitch, V, L, best_row, plain)
           : row_w == 4  ? trace_rows<4, false>(s.p, s.L, pitch, V, L, best_row, plain)
           : row_w == 8  ? trace_rows<8, false>(s.p, s.L, pitch, V, L, best_row, plain)
           : row_w == 12 ? trace_rows<12, false>(s.p, s.L, pitch, V, L, best_row, plain)
-                        : trace_rows<16, false>(s.p, s.L, pitch, V, L, best_row, plain));
+          : row_w == 16 ? trace_rows<16, false>(s.p, s.L, pitch, V, L, best_row, plain)
+                        : trace_rows<20, false>(s.p, s.L, pitch, V, L, best_row, plain));
       if (left < 0) {
         R.status = left == -2 ? kPoaBandMiss : kPoaBadInput;
         return;
       }
       // from the virtual start row only horizontal moves remain
       for (int p = lane; p < left; p += kWave) s.path()[p] = -1;
-    } else{
+    } else {
       const uint16_t* code = s.code();
       const int32_t* pred_off = s.pred_off();
       const int32_t* pred_rows = s.pred_rows();
       const uint4* row_rec = s.row_rec();
-      const bool records = rows16;
-      const int record_half = row_record_bytes(row_w) / 2;
-      const int row_inv = 65536 / row_w + 1;
       int32_t* pos_node = s.path();
       constexpr uint32_t kNextExit = 0xff;  // successor: the decoder takes the move
       constexpr uint32_t kDiagBit = 0x100;
@@ -3299,39 +3335,9 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
         const int rc = max(ri, 1);
         const int cj = j0 - 2 * (lane & 3);
         const uint16_t* crow = code + static_cast<int64_t>(rc) * pitch;
-        uint32_t c0, c1;
-        uint4 rec;  // descriptor, graph node, first four predecessor row deltas
-        if (records) {
-          // the row's record and both halves of its move record in one round
-          // trip: kinds of columns cj and cj - 1, predecessor indices of
-          // cj, cj - 1 and cj - 2
-          const uint8_t* mrow = reinterpret_cast<const uint8_t*>(crow);
-          const RecordBit b0 = record_bit(max(cj, 0), row_w, row_inv);
-          const RecordBit b1 = record_bit(max(cj - 1, 0), row_w, row_inv);
-          const RecordBit b2 = record_bit(max(cj - 2, 0), row_w, row_inv);
-          rec = row_rec[rc - 1];
-          const uint32_t m0 = mrow[b0.byte], m1 = mrow[b1.byte];
-          const uint32_t x0 = mrow[b0.byte + record_half], x1 = mrow[b1.byte + record_half];
-          const uint32_t x2 = mrow[b2.byte + record_half];
-          const uint32_t k0 = (x0 >> b0.bit) & 3u, k1 = (x1 >> b1.bit) & 3u;
-          const uint32_t k2 = (x2 >> b2.bit) & 3u;
-          auto move_code = [&](uint32_t kind, uint32_t above, uint32_t left) -> uint32_t {
-            return (kind & 2u) != 0   ? (kCodeDiag | kCodeViaK | left)
-                   : (kind & 1u) != 0 ? (kCodeVert | kCodeViaK | above)
-                                      : static_cast<uint32_t>(kCodeHorz);
-          };
-          c0 = move_code((m0 >> b0.bit) & 3u, k0, k1);
-          c1 = move_code((m1 >> b1.bit) & 3u, k1, k2);
-          if (!layer_plain || (rec.x & kRecPreds) == 0) {
-            // a row of the general form: 16-bit codes
-            c0 = crow[max(cj, 0)];
-            c1 = crow[max(cj - 1, 0)];
-          }
-        } else {
-          rec = row_rec[rc - 1];
-          c0 = crow[code_index(max(cj, 0), pitch)];
-          c1 = crow[code_index(max(cj - 1, 0), pitch)];
-        }
+        const uint4 rec = row_rec[rc - 1];  // graph node, first four predecessor row deltas
+        const uint32_t c0 = crow[code_index(max(cj, 0), pitch)];
+        const uint32_t c1 = crow[code_index(max(cj - 1, 0), pitch)];
         const uint64_t d4 = static_cast<uint64_t>(rec.w) << 32 | rec.z;
         const int nrow = static_cast<int>(rec.y);  // graph node of the row
         const uint32_t cw = ri >= 1 ? ((cj >= 0 ? c0 : 0u) | ((cj >= 1 ? c1 : 0u) << 16)) : 0u;
