@@ -729,7 +729,7 @@ __device__ __forceinline__ uint32_t pk_splat(int32_t v) {
 // score (2 bits each): the diagonal into column j takes the one of column
 // j - 1, the vertical the one of column j, which is spoa's choice. Rows
 // outside this form (more than four predecessors, the virtual start row or a
-// row in global memory among them, their own row in global memory, letters
+// row in global memory among them, their own row in global memory, a base
 // other than A, C, G, T) store 16-bit codes, column j at element j.
 //
 // The rows are bound by their instructions: a wave alone issues one about
@@ -919,9 +919,18 @@ __device__ __forceinline__ void row_kinds(const uint32_t* h, const uint32_t* bd,
   }
 }
 
+// Scores of a pair whose letters are not all A, C, G or T: those match no row
+// of the descriptor form (a row of another letter takes the general form).
+constexpr uint32_t kOddLetter = 0x0d0du;  // their selector
+__device__ __forceinline__ uint32_t odd_letters(uint32_t sub, uint32_t sel, uint32_t miss) {
+  const uint32_t m = ((sel >> 3) & sel & 0x00010001u) * 0xffffu;
+  return (sub & ~m) | (miss & m);
+}
+
 // One DP layer in packed rows; the end cell as dp_layer. W: 4, 8, 12, 16 or
-// 20 with 64 W > L.
-template <int W>
+// 20 with 64 W > L. kPlain: the layer holds A, C, G and T only (functions of
+// their own: a test per row cost 2%).
+template <int W, bool kPlain>
 __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, int V, int L,
                                        int bias, int* best_score, bool* tied) {
   constexpr int H2 = W / 2;
@@ -932,13 +941,17 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
   const int32_t match = uniform(P.match);
   const int32_t mismatch = uniform(P.mismatch);
   const uint32_t row_bytes = static_cast<uint32_t>(pitch) * 2;
-  const uint32_t strip = lds + static_cast<uint32_t>(lane) * (2 * W);
   const LByte* seq = (const LByte*)(size_t)(
       lds + static_cast<uint32_t>(align_up(static_cast<uint64_t>(P.ring_rows) * row_bytes, 16)));
-  const int n_live = (L + W) / W;
+  // Lanes past the last column run along (every lane's registers stay whole for
+  // the row loop's readlanes): their scores and moves go to the row's columns
+  // past L, those that find no room there to its last ones (a row has at least
+  // L + 24 columns, so these are past L as well).
+  const bool live = lane < (L + W) / W;
+  const uint32_t strip =
+      lds + min(static_cast<uint32_t>(lane) * (2 * W), row_bytes - 2 * W);
   // letters of the strip (column j holds letter j - 1) as table selectors
   uint32_t sel[H2];
-  bool plain = true;
 #pragma unroll
   for (int q = 0; q < H2; ++q) {
     uint32_t x = 0;
@@ -947,13 +960,15 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
       const int idx = lane * W + 2 * q + u - 1;
       const int c = idx >= 0 && idx < L ? static_cast<int>(seq[idx]) : 'A';
       const int code = ((c >> 1) ^ (c >> 2)) & 3;
-      plain &= static_cast<int>((0x54474341u >> (8 * code)) & 0xffu) == c;
+      const bool is_base = static_cast<int>((0x54474341u >> (8 * code)) & 0xffu) == c;
       // (a selector byte of 0x0c gives 0: column 0)
-      x |= (idx < 0 ? 0x0c0cu : static_cast<uint32_t>(code) * 0x0101u + 0x0400u) << (16 * u);
+      x |= (idx < 0    ? 0x0c0cu
+            : !kPlain && !is_base ? kOddLetter
+                       : static_cast<uint32_t>(code) * 0x0101u + 0x0400u)
+           << (16 * u);
     }
     sel[q] = x;
   }
-  const bool layer_plain = __all(plain);
   const uint32_t gap_pair = pk_splat(gap);
   // score tables: s - gap of a mismatch in every byte pair, and the change
   // to the match in the pair of code 0
@@ -975,14 +990,14 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
 #pragma unroll
   for (int q = 0; q < H2; ++q) cur[q] = 0;
   GByte* const codes = (GByte*)s.code();
-  uint32_t rec_lane = static_cast<uint32_t>(lane * row_record_bytes(W));
+  uint32_t rec_lane = min(static_cast<uint32_t>(lane * row_record_bytes(W)),
+                          row_bytes - static_cast<uint32_t>(row_record_bytes(W)));
   // (chunks of 63 rows: the last lane's descriptor is 0 and ends the row loop)
   constexpr int kChunk = kWave - 1;
   for (int r0 = 1; r0 <= V; r0 += kChunk) {
     const int rk = r0 + lane;
     uint32_t desc_v = 0;
     if (lane < kChunk && rk <= V) desc_v = s.row_rec()[rk - 1].x;
-    if (!layer_plain) desc_v &= ~(kRecPreds | kRecChain);
     const int chunk = uniform(min(kChunk, V - r0 + 1));
     // what the rows of the general form need of this chunk
     int off_v = 0, end_v = 0, meta_v = 0, base = 0, pr0 = 0, pr1 = 0;
@@ -999,254 +1014,263 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
     // complete the chunk's loads here: otherwise the row loop would wait for
     // them (and for every store issued before them) on each row
     wait_stores();
-    if (lane < n_live) {
-      GByte* record = codes + static_cast<int64_t>(r0 - 1) * row_bytes;  // of the row before
-      // the next row's descriptor and substitution scores, a piece at a time
-      uint32_t d = 0, d_next = 0;
-      uint64_t table = 0;
-      uint32_t sub[H2];
-      const auto next_desc = [&](int rr) {
-        d_next = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(desc_v), rr));
-        pin_scalar(d_next);
-      };
-      const auto next_table = [&]() {
-        table = table0 ^ (table1 << (d_next & kRecBase));
-        asm volatile("" : "+s"(table));
-      };
-      const auto next_sub = [&](int q) {
-        sub[q] = __builtin_amdgcn_perm(static_cast<uint32_t>(table >> 32),
-                                       static_cast<uint32_t>(table), sel[q]);
-        pin(sub[q]);
-      };
-      const auto next_row = [&](int rr) {
-        next_desc(rr);
-        next_table();
+    GByte* record = codes + static_cast<int64_t>(r0 - 1) * row_bytes;  // of the row before
+    // the next row's descriptor and substitution scores, a piece at a time
+    uint32_t d = 0, d_next = 0;
+    uint64_t table = 0;
+    uint32_t sub[H2];
+    const auto next_desc = [&](int rr) {
+      d_next = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(desc_v), rr));
+      pin_scalar(d_next);
+    };
+    const auto next_table = [&]() {
+      table = table0 ^ (table1 << (d_next & kRecBase));
+      asm volatile("" : "+s"(table));
+    };
+    const auto next_sub = [&](int q) {
+      sub[q] = __builtin_amdgcn_perm(static_cast<uint32_t>(table >> 32),
+                                     static_cast<uint32_t>(table), sel[q]);
+      pin(sub[q]);
+    };
+    const auto next_odd = [&]() {
+      if constexpr (!kPlain) {
 #pragma unroll
-        for (int q = 0; q < H2; ++q) next_sub(q);
-        d = d_next;
-      };
-      const auto sink_row = [&](int r) {
-        uint32_t last = cur[0];
-#pragma unroll
-        for (int q = 1; q < H2; ++q) {
-          uint32_t v = cur[q];
-          asm volatile("" : "+v"(v));  // (selected, not indexed through a stack copy)
-          if (q == (end_u >> 1)) last = v;
+        for (int q = 0; q < H2; ++q) {
+          uint32_t letters = sel[q];
+          pin(letters);  // (its masks are not kept in registers)
+          sub[q] = odd_letters(sub[q], letters, miss * 0x10001u);
         }
-        const uint32_t g = static_cast<uint32_t>(
-            __builtin_amdgcn_readlane(static_cast<int>(last), end_lane));
-        const int32_t h_last =
-            static_cast<int32_t>((end_u & 1) ? g >> 16 : g & 0xffffu) - bias + L * gap;
-        if (lane == 0) s.sink_score()[r] = h_last;
-        if (h_last > best) {
-          best = h_last;
-          best_row = r;
-          ties = 0;
-        } else if (h_last == best) {
-          ++ties;
-        }
-      };
-      next_row(0);
-      int rr = 0;
-      for (;;) {
-        // rows of up to four predecessors (a loop of their own: the common
-        // ones go through without a taken branch)
-        uint32_t np = d & kRecPreds, np_next = 0;
-        while (np != 0) {
-          const auto slot_at = [&](int k) {
-            return strip + ((d >> (kRecPredShift + 5 * k)) & 31u) * row_bytes;
-          };
-          uint32_t bd[H2], bv[H2], acc[NA], ack[NA];
+      }
+    };
+    const auto next_row = [&](int rr) {
+      next_desc(rr);
+      next_table();
 #pragma unroll
-          for (int a = 0; a < NA; ++a) ack[a] = 0;
-          if ((d & kRecChain) == 0) lds_row_load<W>(slot_at(0), cur);
-          if (np > 1) {
-            // best predecessor score of each column and the first
-            // predecessor reaching it (a later one only when better)
-            uint32_t kx[H2], p1[H2];
-            lds_row_load<W>(slot_at(1), p1);
+      for (int q = 0; q < H2; ++q) next_sub(q);
+      next_odd();
+      d = d_next;
+    };
+    const auto sink_row = [&](int r) {
+      uint32_t last = cur[0];
+#pragma unroll
+      for (int q = 1; q < H2; ++q) {
+        uint32_t v = cur[q];
+        asm volatile("" : "+v"(v));  // (selected, not indexed through a stack copy)
+        if (q == (end_u >> 1)) last = v;
+      }
+      const uint32_t g = static_cast<uint32_t>(
+          __builtin_amdgcn_readlane(static_cast<int>(last), end_lane));
+      const int32_t h_last =
+          static_cast<int32_t>((end_u & 1) ? g >> 16 : g & 0xffffu) - bias + L * gap;
+      if (lane == 0) s.sink_score()[r] = h_last;
+      if (h_last > best) {
+        best = h_last;
+        best_row = r;
+        ties = 0;
+      } else if (h_last == best) {
+        ++ties;
+      }
+    };
+    next_row(0);
+    int rr = 0;
+    for (;;) {
+      // rows of up to four predecessors (a loop of their own: the common
+      // ones go through without a taken branch)
+      uint32_t np = d & kRecPreds, np_next = 0;
+      while (np != 0) {
+        const auto slot_at = [&](int k) {
+          return strip + ((d >> (kRecPredShift + 5 * k)) & 31u) * row_bytes;
+        };
+        uint32_t bd[H2], bv[H2], acc[NA], ack[NA];
+#pragma unroll
+        for (int a = 0; a < NA; ++a) ack[a] = 0;
+        if ((d & kRecChain) == 0) lds_row_load<W>(slot_at(0), cur);
+        if (np > 1) {
+          // best predecessor score of each column and the first
+          // predecessor reaching it (a later one only when better)
+          uint32_t kx[H2], p1[H2];
+          lds_row_load<W>(slot_at(1), p1);
+#pragma unroll
+          for (int q = 0; q < H2; ++q) {
+            kx[q] = pk_min_u(pk_sub_sat(p1[q], cur[q]), one);
+            cur[q] = pk_max_u(cur[q], p1[q]);
+          }
+          if (np > 2) {
+            lds_row_load<W>(slot_at(2), p1);
 #pragma unroll
             for (int q = 0; q < H2; ++q) {
-              kx[q] = pk_min_u(pk_sub_sat(p1[q], cur[q]), one);
+              const uint32_t g = pk_min_u(pk_sub_sat(p1[q], cur[q]), one);
+              kx[q] = pk_max_u(kx[q], g << 1);
               cur[q] = pk_max_u(cur[q], p1[q]);
             }
-            if (np > 2) {
-              lds_row_load<W>(slot_at(2), p1);
+            if (np > 3) {
+              lds_row_load<W>(slot_at(3), p1);
 #pragma unroll
               for (int q = 0; q < H2; ++q) {
                 const uint32_t g = pk_min_u(pk_sub_sat(p1[q], cur[q]), one);
-                kx[q] = pk_max_u(kx[q], g << 1);
+                kx[q] = pk_max_u(kx[q], pk_mad(g, 0x00030003u, 0u));
                 cur[q] = pk_max_u(cur[q], p1[q]);
               }
-              if (np > 3) {
-                lds_row_load<W>(slot_at(3), p1);
-#pragma unroll
-                for (int q = 0; q < H2; ++q) {
-                  const uint32_t g = pk_min_u(pk_sub_sat(p1[q], cur[q]), one);
-                  kx[q] = pk_max_u(kx[q], pk_mad(g, 0x00030003u, 0u));
-                  cur[q] = pk_max_u(cur[q], p1[q]);
-                }
-              }
-            }
-#pragma unroll
-            for (int q = 0; q < H2; ++q) {
-              ack[q / 8] = (q % 8) == 0 ? kx[q] : (ack[q / 8] << 2) | kx[q];
             }
           }
-          const uint32_t own = (d >> kRecOwnShift) & 31u;
-          uint32_t own_at = 0;
-          row_scores<W>(cur, sub, gap_pair, bd, bv, [&](int k) {
-            if (k == (H2 == 2 ? 2 : 1)) next_desc(rr + 1);
-            if (k == 2) next_table();
-            if (k == 3) {
-              own_at = strip + own * row_bytes;
-              pin(own_at);
-            }
-            constexpr int kShare = (H2 + 2) / 3;  // pairs per gap
-            if (k >= 4 && k < 7) {
-#pragma unroll
-              for (int q = (k - 4) * kShare; q < min(H2, (k - 3) * kShare); ++q) next_sub(q);
-            }
-            if (k == 7) {
-              record += row_bytes;
-              asm volatile("" : "+s"(record));
-            }
-            if (k == 8) {
-              np_next = d_next & kRecPreds;
-              pin_scalar(np_next);
-            }
-          });
-          if (own != static_cast<uint32_t>(kSlotNone)) lds_row_store<W>(own_at, cur);
-          row_kinds<W>(cur, bd, bv, acc);
-          pin(rec_lane);  // (stays a 32-bit offset to the uniform row address)
-          GByte* at = record + rec_lane;
-          if constexpr (W == 4) {
-            const uint32_t a = (acc[0] | (acc[0] >> 12)) & 0xffu;
-            const uint32_t k = (ack[0] | (ack[0] >> 12)) & 0xffu;
-            *(__attribute__((address_space(1))) uint16_t*)at = static_cast<uint16_t>(a | (k << 8));
-          } else if constexpr (W == 8) {
-            *(__attribute__((address_space(1))) uint32_t*)at =
-                __builtin_amdgcn_perm(ack[0], acc[0], 0x06040200u);
-          } else if constexpr (NA == 1) {
-            *(__attribute__((address_space(1))) U32x2*)at = U32x2{acc[0], ack[0]};
-          } else {
-            *(__attribute__((address_space(1))) U32x4*)at = U32x4{acc[0], acc[1], ack[0], ack[1]};
-          }
-          if (__builtin_expect((d & kRecSink) != 0, 0)) sink_row(r0 + rr);
-          ++rr;
-          d = d_next;
-          np = np_next;
-        }
-        if (rr >= chunk) break;
-        record += row_bytes;
-        {
-          uint32_t bd[H2], bv[H2];
-          // the general form: any number of predecessors, in LDS, in global
-          // memory or the virtual start row; any letters; 16-bit codes
-          const int r = r0 + rr;
-          const int off = __builtin_amdgcn_readlane(off_v, rr);
-          const int n_preds = __builtin_amdgcn_readlane(end_v, rr) - off;
-          const int meta = __builtin_amdgcn_readlane(meta_v, rr);
-          const int own = (meta >> kRowMetaSlotShift) & 31;
-          const int j0 = lane * W;
-          uint32_t mx[H2], kx[H2];
-#pragma unroll
-          for (int q = 0; q < H2; ++q) mx[q] = kx[q] = 0;
-          for (int k = 0; k < n_preds; ++k) {
-            const int idx = off + k - base;
-            int e;
-            if (idx < kWave) {
-              e = __builtin_amdgcn_readlane(pr0, idx);
-            } else if (idx < 2 * kWave) {
-              e = __builtin_amdgcn_readlane(pr1, idx - kWave);
-            } else {
-              e = uniform(s.pred_rows()[off + k]);
-            }
-            const int p = e & kPredRowMask;
-            const int sl = static_cast<int>(static_cast<unsigned>(e) >> kPredRowBits);
-            uint32_t pp[H2];
-            if (p == 0) {
-#pragma unroll
-              for (int q = 0; q < H2; ++q) pp[q] = pk_splat(bias);
-            } else if (sl == kSlotNone) {
-              // the row before, kept in registers only
-#pragma unroll
-              for (int q = 0; q < H2; ++q) pp[q] = cur[q];
-            } else if (sl < kSlotGlobal) {
-              lds_row_load<W>(strip + static_cast<uint32_t>(sl) * row_bytes, pp);
-            } else {
-              const int32_t* row = s.H_row(p, pitch);
-#pragma unroll
-              for (int q = 0; q < H2; ++q) {
-                // (columns past L are never stored: any value does)
-                const int ja = min(j0 + 2 * q, L), jb = min(j0 + 2 * q + 1, L);
-                pp[q] = (static_cast<uint32_t>(row[ja]) & 0xffffu) |
-                        (static_cast<uint32_t>(row[jb]) << 16);
-              }
-            }
-            const uint32_t ks = static_cast<uint32_t>(k) * 0x10001u;
-#pragma unroll
-            for (int q = 0; q < H2; ++q) {
-              const uint32_t g = pk_min_u(pk_sub_sat(pp[q], mx[q]), one);
-              kx[q] = pk_mad(g, pk_sub(ks, kx[q]), kx[q]);
-              mx[q] = pk_max_u(mx[q], pp[q]);
-            }
-          }
-          uint32_t scores[H2];
 #pragma unroll
           for (int q = 0; q < H2; ++q) {
-            uint32_t x = 0;
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-              const int idx = j0 + 2 * q + u - 1;
-              const bool same = idx >= 0 && idx < L && static_cast<int>(seq[idx]) == (meta & 0xff);
-              const int v = idx < 0 ? 0 : (same ? match : mismatch) - gap;
-              x |= (static_cast<uint32_t>(v) & 0xffffu) << (16 * u);
-            }
-            scores[q] = x;
-            // (a move, so that mx and cur need not share registers)
-            asm volatile("v_mov_b32 %0, %1" : "=v"(cur[q]) : "v"(mx[q]));
+            ack[q / 8] = (q % 8) == 0 ? kx[q] : (ack[q / 8] << 2) | kx[q];
           }
-          row_scores<W>(cur, scores, gap_pair, bd, bv, [](int) {});
-          if (own < kSlotGlobal) {
-            lds_row_store<W>(strip + static_cast<uint32_t>(own) * row_bytes, cur);
-          } else if (own == kSlotGlobal) {
-            int32_t* Hg = s.H_row(r, meta, pitch);
-#pragma unroll
-            for (int u = 0; u < W; ++u) {
-              if (j0 + u <= L) Hg[j0 + u] = static_cast<int32_t>((cur[u / 2] >> (16 * (u & 1))) & 0xffffu);
-            }
-          }
-          // codes: kCodeViaK | index of the predecessor
-          uint32_t kprev = shift_into(0u, kx[H2 - 1]);
-          uint16_t* Cr = s.code() + static_cast<int64_t>(r) * pitch;
-#pragma unroll
-          for (int q = 0; q < H2; ++q) {
-            const uint32_t kd = __builtin_amdgcn_alignbit(kx[q], q == 0 ? kprev : kx[q - 1], 16);
-            uint32_t code = 0;
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-              const uint32_t hu = (cur[q] >> (16 * u)) & 0xffffu;
-              const bool dg = ((bd[q] >> (16 * u)) & 0xffffu) == hu;
-              const bool vt = ((bv[q] >> (16 * u)) & 0xffffu) == hu;
-              const uint32_t kdu = (kd >> (16 * u)) & 0xffffu, kvu = (kx[q] >> (16 * u)) & 0xffffu;
-              const uint32_t c = dg ? (kCodeDiag | kCodeViaK | kdu)
-                                    : (vt ? (kCodeVert | kCodeViaK | kvu) : kCodeHorz);
-              code |= c << (16 * u);
-            }
-            *reinterpret_cast<uint32_t*>(Cr + j0 + 2 * q) = code;
-          }
-          if ((d & kRecSink) != 0) sink_row(r);
         }
+        const uint32_t own = (d >> kRecOwnShift) & 31u;
+        uint32_t own_at = 0;
+        row_scores<W>(cur, sub, gap_pair, bd, bv, [&](int k) {
+          if (k == (H2 == 2 ? 2 : 1)) next_desc(rr + 1);
+          if (k == 2) next_table();
+          if (k == 3) {
+            own_at = strip + own * row_bytes;
+            pin(own_at);
+          }
+          constexpr int kShare = (H2 + 2) / 3;  // pairs per gap
+          if (k >= 4 && k < 7) {
+#pragma unroll
+            for (int q = (k - 4) * kShare; q < min(H2, (k - 3) * kShare); ++q) next_sub(q);
+          }
+          if (k == 7) {
+            record += row_bytes;
+            asm volatile("" : "+s"(record));
+          }
+          if (k == 8) {
+            np_next = d_next & kRecPreds;
+            pin_scalar(np_next);
+            next_odd();
+          }
+        });
+        if (own != static_cast<uint32_t>(kSlotNone)) lds_row_store<W>(own_at, cur);
+        row_kinds<W>(cur, bd, bv, acc);
+        pin(rec_lane);  // (stays a 32-bit offset to the uniform row address)
+        GByte* at = record + rec_lane;
+        if constexpr (W == 4) {
+          const uint32_t a = (acc[0] | (acc[0] >> 12)) & 0xffu;
+          const uint32_t k = (ack[0] | (ack[0] >> 12)) & 0xffu;
+          *(__attribute__((address_space(1))) uint16_t*)at = static_cast<uint16_t>(a | (k << 8));
+        } else if constexpr (W == 8) {
+          *(__attribute__((address_space(1))) uint32_t*)at =
+              __builtin_amdgcn_perm(ack[0], acc[0], 0x06040200u);
+        } else if constexpr (NA == 1) {
+          *(__attribute__((address_space(1))) U32x2*)at = U32x2{acc[0], ack[0]};
+        } else {
+          *(__attribute__((address_space(1))) U32x4*)at = U32x4{acc[0], acc[1], ack[0], ack[1]};
+        }
+        if (__builtin_expect((d & kRecSink) != 0, 0)) sink_row(r0 + rr);
         ++rr;
-        next_row(rr);
+        d = d_next;
+        np = np_next;
       }
+      if (rr >= chunk) break;
+      record += row_bytes;
+      {
+        uint32_t bd[H2], bv[H2];
+        // the general form: any number of predecessors, in LDS, in global
+        // memory or the virtual start row; any letters; 16-bit codes
+        const int r = r0 + rr;
+        const int off = __builtin_amdgcn_readlane(off_v, rr);
+        const int n_preds = __builtin_amdgcn_readlane(end_v, rr) - off;
+        const int meta = __builtin_amdgcn_readlane(meta_v, rr);
+        const int own = (meta >> kRowMetaSlotShift) & 31;
+        const int j0 = lane * W;
+        uint32_t mx[H2], kx[H2];
+#pragma unroll
+        for (int q = 0; q < H2; ++q) mx[q] = kx[q] = 0;
+        for (int k = 0; k < n_preds; ++k) {
+          const int idx = off + k - base;
+          int e;
+          if (idx < kWave) {
+            e = __builtin_amdgcn_readlane(pr0, idx);
+          } else if (idx < 2 * kWave) {
+            e = __builtin_amdgcn_readlane(pr1, idx - kWave);
+          } else {
+            e = uniform(s.pred_rows()[off + k]);
+          }
+          const int p = e & kPredRowMask;
+          const int sl = static_cast<int>(static_cast<unsigned>(e) >> kPredRowBits);
+          uint32_t pp[H2];
+          if (p == 0) {
+#pragma unroll
+            for (int q = 0; q < H2; ++q) pp[q] = pk_splat(bias);
+          } else if (sl == kSlotNone) {
+            // the row before, kept in registers only
+#pragma unroll
+            for (int q = 0; q < H2; ++q) pp[q] = cur[q];
+          } else if (sl < kSlotGlobal) {
+            lds_row_load<W>(strip + static_cast<uint32_t>(sl) * row_bytes, pp);
+          } else {
+            const int32_t* row = s.H_row(p, pitch);
+#pragma unroll
+            for (int q = 0; q < H2; ++q) {
+              // (columns past L are never stored: any value does)
+              const int ja = min(j0 + 2 * q, L), jb = min(j0 + 2 * q + 1, L);
+              pp[q] = (static_cast<uint32_t>(row[ja]) & 0xffffu) |
+                      (static_cast<uint32_t>(row[jb]) << 16);
+            }
+          }
+          const uint32_t ks = static_cast<uint32_t>(k) * 0x10001u;
+#pragma unroll
+          for (int q = 0; q < H2; ++q) {
+            const uint32_t g = pk_min_u(pk_sub_sat(pp[q], mx[q]), one);
+            kx[q] = pk_mad(g, pk_sub(ks, kx[q]), kx[q]);
+            mx[q] = pk_max_u(mx[q], pp[q]);
+          }
+        }
+        uint32_t scores[H2];
+#pragma unroll
+        for (int q = 0; q < H2; ++q) {
+          uint32_t x = 0;
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const int idx = j0 + 2 * q + u - 1;
+            const bool same = idx >= 0 && idx < L && static_cast<int>(seq[idx]) == (meta & 0xff);
+            const int v = idx < 0 ? 0 : (same ? match : mismatch) - gap;
+            x |= (static_cast<uint32_t>(v) & 0xffffu) << (16 * u);
+          }
+          scores[q] = x;
+          // (a move, so that mx and cur need not share registers)
+          asm volatile("v_mov_b32 %0, %1" : "=v"(cur[q]) : "v"(mx[q]));
+        }
+        row_scores<W>(cur, scores, gap_pair, bd, bv, [](int) {});
+        if (own < kSlotGlobal) {
+          lds_row_store<W>(strip + static_cast<uint32_t>(own) * row_bytes, cur);
+        } else if (own == kSlotGlobal) {
+          int32_t* Hg = s.H_row(r, meta, pitch);
+#pragma unroll
+          for (int u = 0; u < W; ++u) {
+            if (j0 + u <= L) Hg[j0 + u] = static_cast<int32_t>((cur[u / 2] >> (16 * (u & 1))) & 0xffffu);
+          }
+        }
+        // codes: kCodeViaK | index of the predecessor
+        uint32_t kprev = shift_into(0u, kx[H2 - 1]);
+        uint16_t* Cr = s.code() + static_cast<int64_t>(r) * pitch;
+#pragma unroll
+        for (int q = 0; q < H2; ++q) {
+          const uint32_t kd = __builtin_amdgcn_alignbit(kx[q], q == 0 ? kprev : kx[q - 1], 16);
+          uint32_t code = 0;
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const uint32_t hu = (cur[q] >> (16 * u)) & 0xffffu;
+            const bool dg = ((bd[q] >> (16 * u)) & 0xffffu) == hu;
+            const bool vt = ((bv[q] >> (16 * u)) & 0xffffu) == hu;
+            const uint32_t kdu = (kd >> (16 * u)) & 0xffffu, kvu = (kx[q] >> (16 * u)) & 0xffffu;
+            const uint32_t c = dg ? (kCodeDiag | kCodeViaK | kdu)
+                                  : (vt ? (kCodeVert | kCodeViaK | kvu) : kCodeHorz);
+            code |= c << (16 * u);
+          }
+          if (live) *reinterpret_cast<uint32_t*>(Cr + j0 + 2 * q) = code;
+        }
+        if ((d & kRecSink) != 0) sink_row(r);
+      }
+      ++rr;
+      next_row(rr);
     }
   }
-  // (tracked under the live lanes' execution mask: uniform there)
-  *best_score = uniform(best);
-  *tied = uniform(ties) > 0;
-  return uniform(best_row);
+  *best_score = best;
+  *tied = ties > 0;
+  return best_row;
 }
 
 // ---- banded rows: the opt-in approximation of racon -b ----
@@ -1381,7 +1405,6 @@ __device__ __forceinline__ int dp_band(CParams& P, const Slot& s, uint32_t lds, 
         shift_v |= static_cast<uint32_t>(min(max(by, 0), kWave + 1)) << (8 * k);
       }
     }
-    if (!layer_plain) desc_v &= ~(kRecPreds | kRecChain);
     const int chunk = uniform(min(kWave, V - r0 + 1));
     int off_v = 0, end_v = 0, meta_v = 0, base = 0, pr0 = 0, pr1 = 0;
     if (__any(rk <= V && (desc_v & kRecPreds) == 0)) {
@@ -1413,6 +1436,15 @@ __device__ __forceinline__ int dp_band(CParams& P, const Slot& s, uint32_t lds, 
           const uint32_t c = ((w >> 1) ^ (w >> 2)) & 0x03030303u;
           sel[0] = __builtin_amdgcn_perm(0u, c, 0x01010000u) + 0x04000400u;
           sel[1] = __builtin_amdgcn_perm(0u, c, 0x03030202u) + 0x04000400u;
+          if (!layer_plain) {
+            const uint32_t other = __builtin_amdgcn_perm(0u, 0x54474341u, c) ^ w;
+#pragma unroll
+            for (int u = 0; u < kBandW; ++u) {
+              if (((other >> (8 * u)) & 0xffu) != 0) {
+                sel[u / 2] = (sel[u / 2] & (0xffffu << (16 * (~u & 1)))) | kOddLetter << (16 * (u & 1));
+              }
+            }
+          }
           sel_lo = lo;
         }
         const uint64_t table = table0 ^ (table1 << (d & kRecBase));
@@ -1420,6 +1452,10 @@ __device__ __forceinline__ int dp_band(CParams& P, const Slot& s, uint32_t lds, 
         for (int q = 0; q < 2; ++q) {
           sub[q] = __builtin_amdgcn_perm(static_cast<uint32_t>(table >> 32),
                                          static_cast<uint32_t>(table), sel[q]);
+        }
+        if (!layer_plain) {
+          sub[0] = odd_letters(sub[0], sel[0], miss * 0x10001u);
+          sub[1] = odd_letters(sub[1], sel[1], miss * 0x10001u);
         }
         const auto row_at = [&](int k) {
           return lds + ((d >> (kRecPredShift + 5 * k)) & 31u) * row_bytes;
@@ -1622,7 +1658,7 @@ enum DpKind : int {
 // allocation of their own instead of sharing one with the rest of the window
 // loop. Arguments arrive in vector registers and are made uniform again on
 // entry. Returns the end-cell row, its score and whether sinks tied.
-template <int kKind>
+template <int kKind, bool kPlain = true>
 __device__ __noinline__ uint64_t dp_layer_call(CParams* params, GByte* base, CLayout* layout,
                                                uint32_t lds_addr, int V, int L, int bias) {
   CParams& P = *uniform_ptr(params);
@@ -1638,15 +1674,15 @@ __device__ __noinline__ uint64_t dp_layer_call(CParams* params, GByte* base, CLa
   bool tied = false;
   int row;
   if constexpr (kKind == kDpRows4) {
-    row = dp_rows<4>(P, s, lds_addr, V, L, bias, &best_score, &tied);
+    row = dp_rows<4, kPlain>(P, s, lds_addr, V, L, bias, &best_score, &tied);
   } else if constexpr (kKind == kDpRows8) {
-    row = dp_rows<8>(P, s, lds_addr, V, L, bias, &best_score, &tied);
+    row = dp_rows<8, kPlain>(P, s, lds_addr, V, L, bias, &best_score, &tied);
   } else if constexpr (kKind == kDpRows12) {
-    row = dp_rows<12>(P, s, lds_addr, V, L, bias, &best_score, &tied);
+    row = dp_rows<12, kPlain>(P, s, lds_addr, V, L, bias, &best_score, &tied);
   } else if constexpr (kKind == kDpRows16) {
-    row = dp_rows<16>(P, s, lds_addr, V, L, bias, &best_score, &tied);
+    row = dp_rows<16, kPlain>(P, s, lds_addr, V, L, bias, &best_score, &tied);
   } else if constexpr (kKind == kDpRows20) {
-    row = dp_rows<20>(P, s, lds_addr, V, L, bias, &best_score, &tied);
+    row = dp_rows<20, kPlain>(P, s, lds_addr, V, L, bias, &best_score, &tied);
   } else if constexpr (kKind == kDpBand4) {
     row = dp_band(P, s, lds_addr, V, L, &best_score, &tied);
   } else if constexpr (kKind == kDpGeneric16) {
@@ -2580,11 +2616,10 @@ __device__ __noinline__ int include_ranks(GByte* slot_base, CLayout* layout, uin
 // batch.) Rows of the general form are decoded one move at a time.
 template <int W, bool kBanded>
 __device__ __noinline__ int trace_rows(GByte* slot_base, CLayout* layout, int pitch, int V, int L,
-                                       int row, int plain) {
+                                       int row) {
   static_assert(W == 4 || W == 8 || W == 12 || W == 16 || W == 20, "strip width");
   const Slot s = carve(uniform_ptr(slot_base), *uniform_ptr(layout));
   pitch = uniform(pitch);
-  plain = uniform(plain);
   V = uniform(V);
   const int length = uniform(L);
   constexpr int kShift = kBanded ? kBandColumn : 0;  // record column of column j: j + kShift
@@ -2710,7 +2745,7 @@ __device__ __noinline__ int trace_rows(GByte* slot_base, CLayout* layout, int pi
     const uint32_t deltas = clamp(rec.z) | clamp(rec.w) << 8;
     // lanes that end the walk inside the tile: rows of the general form and
     // rows past the start (their node's sign bit set)
-    const bool stop = ri < 1 || plain == 0 || (rec.x & kRecPreds) == 0;
+    const bool stop = ri < 1 || (rec.x & kRecPreds) == 0;
     const int node_v = static_cast<int>(rec.y | (stop ? 0x80000000u : 0u));
     // columns the tile can step: a diagonal also reads the column before
     const int columns = first == 0 && (W < 20 || j0 < 32) ? j0 + 1 : min(at, 31);
@@ -3195,7 +3230,7 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
     const int ring_bytes = static_cast<int>(P.ring_rows) * pitch * 2;
     const int max_np =
         uniform(build_rows(s.p, s.L, V, n_slots, rows_lds, ring_bytes,
-                           !rows16 || !layer_plain ? 0 : P.band != 0 && L > kBand ? 2 : 1));
+                           !rows16 ? 0 : P.band != 0 && L > kBand ? 2 : 1));
     wave_sync();
     if (max_np < 0) {
       R.status = kPoaRowOverflow;  // the pooled global rows ran out: rerun exactly
@@ -3229,15 +3264,20 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
     if (banded) {
       dp = dp_layer_call<kDpBand4>(pp, s.p, ly, lds_addr, V, L, 0);
     } else if (rows16 && row_w == 4) {
-      dp = dp_layer_call<kDpRows4>(pp, s.p, ly, lds_addr, V, L, bias);
+      dp = layer_plain ? dp_layer_call<kDpRows4, true>(pp, s.p, ly, lds_addr, V, L, bias)
+                       : dp_layer_call<kDpRows4, false>(pp, s.p, ly, lds_addr, V, L, bias);
     } else if (rows16 && row_w == 8) {
-      dp = dp_layer_call<kDpRows8>(pp, s.p, ly, lds_addr, V, L, bias);
+      dp = layer_plain ? dp_layer_call<kDpRows8, true>(pp, s.p, ly, lds_addr, V, L, bias)
+                       : dp_layer_call<kDpRows8, false>(pp, s.p, ly, lds_addr, V, L, bias);
     } else if (rows16 && row_w == 12) {
-      dp = dp_layer_call<kDpRows12>(pp, s.p, ly, lds_addr, V, L, bias);
+      dp = layer_plain ? dp_layer_call<kDpRows12, true>(pp, s.p, ly, lds_addr, V, L, bias)
+                       : dp_layer_call<kDpRows12, false>(pp, s.p, ly, lds_addr, V, L, bias);
     } else if (rows16 && row_w == 16) {
-      dp = dp_layer_call<kDpRows16>(pp, s.p, ly, lds_addr, V, L, bias);
+      dp = layer_plain ? dp_layer_call<kDpRows16, true>(pp, s.p, ly, lds_addr, V, L, bias)
+                       : dp_layer_call<kDpRows16, false>(pp, s.p, ly, lds_addr, V, L, bias);
     } else if (rows16) {
-      dp = dp_layer_call<kDpRows20>(pp, s.p, ly, lds_addr, V, L, bias);
+      dp = layer_plain ? dp_layer_call<kDpRows20, true>(pp, s.p, ly, lds_addr, V, L, bias)
+                       : dp_layer_call<kDpRows20, false>(pp, s.p, ly, lds_addr, V, L, bias);
     } else if (narrow) {
       dp = dp_layer_call<kDpGeneric16>(pp, s.p, ly, lds_addr, V, L, 0);
     } else {
@@ -3286,25 +3326,24 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
     // 4. traceback, from the end cell to (0, 0). The alignment of layer
     // position p (the graph node of a diagonal move into column p + 1, or -1
     // for a horizontal move) goes to pos_node[p]; vertical moves align no
-    // layer position. Per round trip the wave loads the 16-row x 8-column
-    // block of codes at and before the current cell (the path falls about two
-    // rows per column) with the node and the predecessor-delta table of each
-    // block row, and every lane turns its two cells into their successor cell
-    // in the block (or "leaves the block", or "needs the lists"). The walk
-    // through the block is then a chase of successor indices read from lane
-    // registers; the move that leaves the block (and any the table left to
-    // the predecessor lists) is taken by the full single-step decoder. The
-    // block's positions are collected in one register (lane t: position
-    // j0 - 1 - t) and stored together.
+    // layer position. Packed and band rows: trace_rows. The tiled rows' 16-bit
+    // codes: per round trip the wave loads the 16-row x 8-column block of codes
+    // at and before the current cell (the path falls about two rows per column)
+    // with the node and the predecessor-delta table of each block row, and
+    // every lane turns its two cells into their successor cell in the block (or
+    // "leaves the block", or "needs the lists"). The walk through the block is
+    // then a chase of successor indices read from lane registers; the move that
+    // leaves the block (and any the table left to the predecessor lists) is
+    // taken by the full single-step decoder. The block's positions are collected
+    // in one register (lane t: position j0 - 1 - t) and stored together.
     if (banded || rows16) {
-      const int plain = layer_plain ? 1 : 0;
       const int left = uniform(
-          banded        ? trace_rows<4, true>(s.p, s.L, pitch, V, L, best_row, plain)
-          : row_w == 4  ? trace_rows<4, false>(s.p, s.L, pitch, V, L, best_row, plain)
-          : row_w == 8  ? trace_rows<8, false>(s.p, s.L, pitch, V, L, best_row, plain)
-          : row_w == 12 ? trace_rows<12, false>(s.p, s.L, pitch, V, L, best_row, plain)
-          : row_w == 16 ? trace_rows<16, false>(s.p, s.L, pitch, V, L, best_row, plain)
-                        : trace_rows<20, false>(s.p, s.L, pitch, V, L, best_row, plain));
+          banded        ? trace_rows<4, true>(s.p, s.L, pitch, V, L, best_row)
+          : row_w == 4  ? trace_rows<4, false>(s.p, s.L, pitch, V, L, best_row)
+          : row_w == 8  ? trace_rows<8, false>(s.p, s.L, pitch, V, L, best_row)
+          : row_w == 12 ? trace_rows<12, false>(s.p, s.L, pitch, V, L, best_row)
+          : row_w == 16 ? trace_rows<16, false>(s.p, s.L, pitch, V, L, best_row)
+                        : trace_rows<20, false>(s.p, s.L, pitch, V, L, best_row));
       if (left < 0) {
         R.status = left == -2 ? kPoaBandMiss : kPoaBadInput;
         return;

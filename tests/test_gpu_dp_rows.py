@@ -87,6 +87,23 @@ def test_letters_other_than_acgt():
     check(wins)
 
 
+@pytest.mark.parametrize("length", [60, 300, 600, 900, 1150])
+def test_odd_letters_at_every_strip_width(length):
+    """Layers with other letters, some at the strip edges, some equal to the
+    backbone's, beside plain layers of the same window."""
+    rng = np.random.default_rng(length)
+    win = window(rng, length, 6)
+    backbone = bytearray(win.backbone)
+    backbone[length // 2] = ord("N")
+    win.backbone = bytes(backbone)
+    for k in (0, 2, 3):
+        seq = bytearray(win.layers[k].sequence)
+        for at in [0, len(seq) - 1, len(seq) // 2, *rng.integers(0, len(seq), size=6)]:
+            seq[at] = ord("N") if at % 3 else ord("a")
+        win.layers[k].sequence = bytes(seq)
+    check([win])
+
+
 def test_many_predecessors():
     """Long random deletions give nodes with far more than four in-edges."""
     rng = np.random.default_rng(31)
