@@ -26,8 +26,9 @@
 //
 // Bound by the vector instructions of the steps. 12,000 pairs of 8 +- 4 kbp
 // at 12% error: 404 M wave steps of 59 instructions and 81 ms in the strip
-// form, 145 M steps of 34 and 36 ms now; 61 pairs of 30 +- 9 kbp at 20%
-// (teams): 140 -> 13.3 ms; one pair of 1 kbp: 0.89 -> 0.40 ms.
+// form, 145 M steps of 34 and 36 ms in one-wave pairs, 16 ms with the longest
+// in teams beside them; 61 pairs of 30 +- 9 kbp at 20% (teams): 140 -> 13.3
+// ms; one pair of 1 kbp: 0.89 -> 0.40 ms.
 #include <hip/hip_runtime.h>
 
 #include "align_types.hpp"
@@ -1149,17 +1150,17 @@ __device__ __forceinline__ void align_pair(const AlignParams& A, const AlignPair
           const int d = w.score >= 0 ? w.score : k_top;
           if (kWaves == kTeamWaves && lanes <= kTeamGroup) {
             if constexpr (kWaves == kTeamWaves) {
-            // both halves at once, four waves each
-            const Run r = split_run(w, wave >> 2, d);
-            const int n = max(run_chunks<kTeamGroup>(split_run(w, 0, d)),
-                              run_chunks<kTeamGroup>(split_run(w, 1, d)));
-            __syncthreads();
-            if (threadIdx.x < 3 * kWaves) mail[threadIdx.x] = threadIdx.x % 3 == 0 ? 0xffffu : 0u;
-            __syncthreads();
-            const FinalState f =
-                run_band<kTeamGroup, false>(v, r, true, n, (wave & 3) * kWave, eq, mail);
-            steps += static_cast<uint32_t>(n * kChunk);
-            dump_column(r, f, (r.rev ? v.col_right : v.col_left) + r.q0);
+              // both halves at once, four waves each
+              const Run r = split_run(w, wave >> 2, d);
+              const int n = max(run_chunks<kTeamGroup>(split_run(w, 0, d)),
+                                run_chunks<kTeamGroup>(split_run(w, 1, d)));
+              __syncthreads();
+              if (threadIdx.x < 3 * kWaves) mail[threadIdx.x] = threadIdx.x % 3 == 0 ? 0xffffu : 0u;
+              __syncthreads();
+              const FinalState f =
+                  run_band<kTeamGroup, false>(v, r, true, n, (wave & 3) * kWave, eq, mail);
+              steps += static_cast<uint32_t>(n * kChunk);
+              dump_column(r, f, (r.rev ? v.col_right : v.col_left) + r.q0);
             }
           } else {
             // wider than the lanes: strips of 64 blocks
