@@ -727,10 +727,14 @@ __device__ __forceinline__ uint32_t pk_splat(int32_t v) {
 // taken before vertical before horizontal) and, for rows with two to four
 // predecessors, the index of the first predecessor with the column's best
 // score (2 bits each): the diagonal into column j takes the one of column
-// j - 1, the vertical the one of column j, which is spoa's choice. Rows
-// outside this form (more than four predecessors, the virtual start row or a
-// row in global memory among them, their own row in global memory, a base
-// other than A, C, G, T) store 16-bit codes, column j at element j.
+// j - 1, the vertical the one of column j, which is spoa's choice. Rows of
+// more than four predecessors or of the virtual start row store 16-bit codes,
+// column j at element j. They take the general form of the DP, and so do rows
+// that live in global memory, read one that does, or have a base other than
+// A, C, G, T; these keep move records, because a 16-bit code costs the
+// traceback a round trip per move: with two LDS rows 3,000 windows of 500 bp
+// at 20 layers spent 22.7 wave-seconds in it and 3.7 with records (those of
+// lower-case letters 35 and 3.8).
 //
 // The rows are bound by their instructions: a wave alone issues one about
 // every 8 cycles, and 4 waves per SIMD share the issue slots. A row whose one
@@ -743,8 +747,10 @@ __device__ __forceinline__ uint32_t pk_splat(int32_t v) {
 
 // Row descriptor: number of predecessors (0: the general form), 8 x the code
 // of the row's base, own slot, slots of up to four predecessors, whether the
-// single predecessor is the row before, and the sink flag.
+// single predecessor is the row before, and the sink flag. The general form
+// has the sink flag and kRecMoves, set when the row keeps a move record.
 constexpr uint32_t kRecPreds = 7u;
+constexpr uint32_t kRecMoves = 8u;
 constexpr uint32_t kRecBase = 0x18u;
 constexpr int kRecOwnShift = 5;
 constexpr int kRecPredShift = 10;
@@ -1071,6 +1077,22 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
         ++ties;
       }
     };
+    const auto store_moves = [&](const uint32_t* acc, const uint32_t* ack) {
+      pin(rec_lane);  // (stays a 32-bit offset to the uniform row address)
+      GByte* at = record + rec_lane;
+      if constexpr (W == 4) {
+        const uint32_t a = (acc[0] | (acc[0] >> 12)) & 0xffu;
+        const uint32_t k = (ack[0] | (ack[0] >> 12)) & 0xffu;
+        *(__attribute__((address_space(1))) uint16_t*)at = static_cast<uint16_t>(a | (k << 8));
+      } else if constexpr (W == 8) {
+        *(__attribute__((address_space(1))) uint32_t*)at =
+            __builtin_amdgcn_perm(ack[0], acc[0], 0x06040200u);
+      } else if constexpr (NA == 1) {
+        *(__attribute__((address_space(1))) U32x2*)at = U32x2{acc[0], ack[0]};
+      } else {
+        *(__attribute__((address_space(1))) U32x4*)at = U32x4{acc[0], acc[1], ack[0], ack[1]};
+      }
+    };
     next_row(0);
     int rr = 0;
     for (;;) {
@@ -1144,20 +1166,7 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
         });
         if (own != static_cast<uint32_t>(kSlotNone)) lds_row_store<W>(own_at, cur);
         row_kinds<W>(cur, bd, bv, acc);
-        pin(rec_lane);  // (stays a 32-bit offset to the uniform row address)
-        GByte* at = record + rec_lane;
-        if constexpr (W == 4) {
-          const uint32_t a = (acc[0] | (acc[0] >> 12)) & 0xffu;
-          const uint32_t k = (ack[0] | (ack[0] >> 12)) & 0xffu;
-          *(__attribute__((address_space(1))) uint16_t*)at = static_cast<uint16_t>(a | (k << 8));
-        } else if constexpr (W == 8) {
-          *(__attribute__((address_space(1))) uint32_t*)at =
-              __builtin_amdgcn_perm(ack[0], acc[0], 0x06040200u);
-        } else if constexpr (NA == 1) {
-          *(__attribute__((address_space(1))) U32x2*)at = U32x2{acc[0], ack[0]};
-        } else {
-          *(__attribute__((address_space(1))) U32x4*)at = U32x4{acc[0], acc[1], ack[0], ack[1]};
-        }
+        store_moves(acc, ack);
         if (__builtin_expect((d & kRecSink) != 0, 0)) sink_row(r0 + rr);
         ++rr;
         d = d_next;
@@ -1243,24 +1252,34 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
             if (j0 + u <= L) Hg[j0 + u] = static_cast<int32_t>((cur[u / 2] >> (16 * (u & 1))) & 0xffffu);
           }
         }
-        // codes: kCodeViaK | index of the predecessor
-        uint32_t kprev = shift_into(0u, kx[H2 - 1]);
-        uint16_t* Cr = s.code() + static_cast<int64_t>(r) * pitch;
+        if ((d & kRecMoves) != 0) {
+          uint32_t acc[NA], ack[NA];
+          row_kinds<W>(cur, bd, bv, acc);
 #pragma unroll
-        for (int q = 0; q < H2; ++q) {
-          const uint32_t kd = __builtin_amdgcn_alignbit(kx[q], q == 0 ? kprev : kx[q - 1], 16);
-          uint32_t code = 0;
-#pragma unroll
-          for (int u = 0; u < 2; ++u) {
-            const uint32_t hu = (cur[q] >> (16 * u)) & 0xffffu;
-            const bool dg = ((bd[q] >> (16 * u)) & 0xffffu) == hu;
-            const bool vt = ((bv[q] >> (16 * u)) & 0xffffu) == hu;
-            const uint32_t kdu = (kd >> (16 * u)) & 0xffffu, kvu = (kx[q] >> (16 * u)) & 0xffffu;
-            const uint32_t c = dg ? (kCodeDiag | kCodeViaK | kdu)
-                                  : (vt ? (kCodeVert | kCodeViaK | kvu) : kCodeHorz);
-            code |= c << (16 * u);
+          for (int q = 0; q < H2; ++q) {
+            ack[q / 8] = (q % 8) == 0 ? kx[q] : (ack[q / 8] << 2) | kx[q];
           }
-          if (live) *reinterpret_cast<uint32_t*>(Cr + j0 + 2 * q) = code;
+          store_moves(acc, ack);
+        } else {
+          // codes: kCodeViaK | index of the predecessor
+          uint32_t kprev = shift_into(0u, kx[H2 - 1]);
+          uint16_t* Cr = s.code() + static_cast<int64_t>(r) * pitch;
+#pragma unroll
+          for (int q = 0; q < H2; ++q) {
+            const uint32_t kd = __builtin_amdgcn_alignbit(kx[q], q == 0 ? kprev : kx[q - 1], 16);
+            uint32_t code = 0;
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+              const uint32_t hu = (cur[q] >> (16 * u)) & 0xffffu;
+              const bool dg = ((bd[q] >> (16 * u)) & 0xffffu) == hu;
+              const bool vt = ((bv[q] >> (16 * u)) & 0xffffu) == hu;
+              const uint32_t kdu = (kd >> (16 * u)) & 0xffffu, kvu = (kx[q] >> (16 * u)) & 0xffffu;
+              const uint32_t c = dg ? (kCodeDiag | kCodeViaK | kdu)
+                                    : (vt ? (kCodeVert | kCodeViaK | kvu) : kCodeHorz);
+              code |= c << (16 * u);
+            }
+            if (live) *reinterpret_cast<uint32_t*>(Cr + j0 + 2 * q) = code;
+          }
         }
         if ((d & kRecSink) != 0) sink_row(r);
       }
@@ -1419,6 +1438,11 @@ __device__ __forceinline__ int dp_band(CParams& P, const Slot& s, uint32_t lds, 
     }
     wait_stores();  // (the chunk's loads, as in dp_rows)
     GByte* record = codes + static_cast<int64_t>(r0) * row_bytes;
+    const auto store_moves = [&](uint32_t acc, uint32_t ack, int lo) {
+      const uint32_t a = (acc | (acc >> 12)) & 0xffu;
+      const uint32_t k = (ack | (ack >> 12)) & 0xffu;
+      *(GHalf*)(record + ((lo >> 2) + 1 + lane) * 2) = static_cast<uint16_t>(a | (k << 8));
+    };
     for (int rr = 0; rr < chunk; ++rr) {
       const int r = r0 + rr;
       const uint32_t d = static_cast<uint32_t>(
@@ -1497,10 +1521,7 @@ __device__ __forceinline__ int dp_band(CParams& P, const Slot& s, uint32_t lds, 
         }
         uint32_t acc[1];
         row_kinds<kBandW>(cur, bd, bv, acc);
-        GByte* at = record + ((lo >> 2) + 1 + lane) * 2;
-        const uint32_t a = (acc[0] | (acc[0] >> 12)) & 0xffu;
-        const uint32_t k = (ack | (ack >> 12)) & 0xffu;
-        *(GHalf*)at = static_cast<uint16_t>(a | (k << 8));
+        store_moves(acc[0], ack, lo);
         if (np > 1 && lane == 0) record[(lo >> 2) * 2 + 1] = static_cast<uint8_t>(k_left << 4);
       } else {
         // the general form, as in dp_rows
@@ -1583,27 +1604,34 @@ __device__ __forceinline__ int dp_band(CParams& P, const Slot& s, uint32_t lds, 
           wait_stores();
           wave_fence();
         }
-        // 16-bit codes, column j at element j + 3
-        const uint32_t kprev = shift_into(k_left << 16, kx[1]);
-        uint16_t* Cr = s.code() + static_cast<int64_t>(r) * pitch;
+        if ((d & kRecMoves) != 0) {
+          uint32_t acc[1];
+          row_kinds<kBandW>(cur, bd, bv, acc);
+          store_moves(acc[0], (kx[0] << 2) | kx[1], lo);
+          if (lane == 0) record[(lo >> 2) * 2 + 1] = static_cast<uint8_t>(k_left << 4);
+        } else {
+          // 16-bit codes, column j at element j + 3
+          const uint32_t kprev = shift_into(k_left << 16, kx[1]);
+          uint16_t* Cr = s.code() + static_cast<int64_t>(r) * pitch;
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          const uint32_t kd = __builtin_amdgcn_alignbit(kx[q], q == 0 ? kprev : kx[0], 16);
-          uint32_t code = 0;
+          for (int q = 0; q < 2; ++q) {
+            const uint32_t kd = __builtin_amdgcn_alignbit(kx[q], q == 0 ? kprev : kx[0], 16);
+            uint32_t code = 0;
 #pragma unroll
-          for (int u = 0; u < 2; ++u) {
-            const uint32_t hu = (cur[q] >> (16 * u)) & 0xffffu;
-            const bool dg = ((bd[q] >> (16 * u)) & 0xffffu) == hu;
-            const bool vt = ((bv[q] >> (16 * u)) & 0xffffu) == hu;
-            const uint32_t kdu = (kd >> (16 * u)) & 0xffffu, kvu = (kx[q] >> (16 * u)) & 0xffffu;
-            const uint32_t c = dg ? (kCodeDiag | kCodeViaK | kdu)
-                                  : (vt ? (kCodeVert | kCodeViaK | kvu) : kCodeHorz);
-            code |= c << (16 * u);
+            for (int u = 0; u < 2; ++u) {
+              const uint32_t hu = (cur[q] >> (16 * u)) & 0xffffu;
+              const bool dg = ((bd[q] >> (16 * u)) & 0xffffu) == hu;
+              const bool vt = ((bv[q] >> (16 * u)) & 0xffffu) == hu;
+              const uint32_t kdu = (kd >> (16 * u)) & 0xffffu, kvu = (kx[q] >> (16 * u)) & 0xffffu;
+              const uint32_t c = dg ? (kCodeDiag | kCodeViaK | kdu)
+                                    : (vt ? (kCodeVert | kCodeViaK | kvu) : kCodeHorz);
+              code |= c << (16 * u);
+            }
+            *reinterpret_cast<uint32_t*>(Cr + j0 + kBandColumn + 2 * q) = code;
           }
-          *reinterpret_cast<uint32_t*>(Cr + j0 + kBandColumn + 2 * q) = code;
-        }
-        if (lane == 0 && lo == 0) {
-          Cr[kBandColumn] = static_cast<uint16_t>(kCodeVert | kCodeViaK | k_left);
+          if (lane == 0 && lo == 0) {
+            Cr[kBandColumn] = static_cast<uint16_t>(kCodeVert | kCodeViaK | k_left);
+          }
         }
       }
       if ((d & kRecSink) != 0) {
@@ -2417,7 +2445,10 @@ __device__ __noinline__ int build_rows(GByte* slot_base, CLayout* layout, int V,
       }
     }
     if (in) {
-      const uint32_t desc = (sink ? kRecSink : 0u) | (fast ? fields : 0u);
+      // (the general form keeps a record of its moves too while four indices
+      // name its predecessors)
+      const bool moves = packed && np >= 1 && np <= static_cast<int>(kRecMaxPreds);
+      const uint32_t desc = (sink ? kRecSink : 0u) | (fast ? fields : moves ? kRecMoves : 0u);
       row_rec[r] = make_uint4(desc, static_cast<uint32_t>(node), static_cast<uint32_t>(deltas),
                               static_cast<uint32_t>(deltas >> 32));
     }
@@ -2613,7 +2644,7 @@ __device__ __noinline__ int include_ranks(GByte* slot_base, CLayout* layout, uin
 // move with v_readlane: 29 instructions a move, most of them scalar. (Tiles of
 // 16 rows x 8 columns with successor indices per cell took 66 round trips a
 // layer of 490 columns instead of 20, 106 us alone and 216 us in a full
-// batch.) Rows of the general form are decoded one move at a time.
+// batch.) Rows of 16-bit codes are decoded one move at a time.
 template <int W, bool kBanded>
 __device__ __noinline__ int trace_rows(GByte* slot_base, CLayout* layout, int pitch, int V, int L,
                                        int row) {
@@ -2743,9 +2774,9 @@ __device__ __noinline__ int trace_rows(GByte* slot_base, CLayout* layout, int pi
     // and more lead out of the tile and are made exact after the walk
     const auto clamp = [](uint32_t x) { return pk_min_u(pk_max_u(x, 0x00010001u), 0x00ff00ffu); };
     const uint32_t deltas = clamp(rec.z) | clamp(rec.w) << 8;
-    // lanes that end the walk inside the tile: rows of the general form and
+    // lanes that end the walk inside the tile: rows of 16-bit codes and
     // rows past the start (their node's sign bit set)
-    const bool stop = ri < 1 || (rec.x & kRecPreds) == 0;
+    const bool stop = ri < 1 || (rec.x & (kRecPreds | kRecMoves)) == 0;
     const int node_v = static_cast<int>(rec.y | (stop ? 0x80000000u : 0u));
     // columns the tile can step: a diagonal also reads the column before
     const int columns = first == 0 && (W < 20 || j0 < 32) ? j0 + 1 : min(at, 31);
@@ -2815,7 +2846,7 @@ __device__ __noinline__ int trace_rows(GByte* slot_base, CLayout* layout, int pi
       if (left_band != 0 || !((j > lo && j <= lo + kBand) || (j == 0 && lo == 0))) return -2;
     }
     if (i > 0 && stopped) {
-      // one move of a row of the general form, from its 16-bit code
+      // one move of a row of 16-bit codes
       const int c = uniform(static_cast<int>(s.code()[static_cast<int64_t>(i) * pitch + j + kShift]));
       const int kind = c & 0xc000;
       if (kind == 0xc000 || (kind != kCodeVert && j == 0)) return -1;

@@ -117,3 +117,35 @@ def test_many_predecessors():
             layers.append(Layer(seq, None, 0, 399))
         wins.append(Window(backbone, b"!" * 400, layers))
     check(wins)
+
+
+def run_phases(windows, ring=0):
+    b = _lib.PoaBatch(3, -5, -4, trim=True)
+    if ring:
+        b.set_tuning(0, 0, ring)
+    for _ in range(2):  # (the first run also loads the code)
+        b.upload(windows)
+        b.run(_lib.RH_POA_BATCHED)
+    phases = b.phase_seconds()
+    b.close()
+    return phases
+
+
+def lower(w):
+    layers = [Layer(l.sequence.lower(), l.quality, l.begin, l.end) for l in w.layers]
+    return Window(w.backbone.lower(), w.backbone_quality, layers)
+
+
+@pytest.mark.parametrize("form", ["global rows", "lower case"])
+def test_rows_of_the_general_form_trace_in_tiles(form):
+    """The moves of rows in global memory and of rows with another letter are
+    as cheap to follow as the others' (one round trip per move took 5 and 8
+    times as long; the bound leaves room for a busy device)."""
+    rng = np.random.default_rng(37)
+    wins = [window(rng, 500, 12) for _ in range(24)] * 50
+    plain = run_phases(wins)["traceback"]
+    if form == "global rows":
+        general = run_phases(wins, ring=2)["traceback"]
+    else:
+        general = run_phases([lower(w) for w in wins])["traceback"]
+    assert general < 2 * plain
