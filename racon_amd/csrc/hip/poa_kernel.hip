@@ -91,6 +91,9 @@ constexpr uint32_t kCodePayload = 0x1fff;
 constexpr int kRowMetaGShift = 16;
 constexpr int kRowMetaGMask = 127;
 static_assert(kPoaHPoolRows <= kRowMetaGMask + 1, "pool entries fit the meta bits");
+// Bits 24..26: the number of predecessors, at most 7.
+constexpr int kRowMetaPredShift = 24;
+constexpr int kRowMetaPredMask = 7;
 
 __device__ __forceinline__ int lane_id() { return threadIdx.x; }
 
@@ -730,11 +733,13 @@ __device__ __forceinline__ uint32_t pk_splat(int32_t v) {
 // j - 1, the vertical the one of column j, which is spoa's choice. Rows of
 // more than four predecessors or of the virtual start row store 16-bit codes,
 // column j at element j. They take the general form of the DP, and so do rows
-// that live in global memory, read one that does, or have a base other than
-// A, C, G, T; these keep move records, because a 16-bit code costs the
-// traceback a round trip per move: with two LDS rows 3,000 windows of 500 bp
-// at 20 layers spent 22.7 wave-seconds in it and 3.7 with records (those of
-// lower-case letters 35 and 3.8).
+// that live in global memory or read one that does; these keep move records,
+// because a 16-bit code costs the traceback a round trip per move: with two
+// LDS rows 3,000 windows of 500 bp at 20 layers spent 22.7 wave-seconds in it
+// and 3.7 with records. A row of a letter other than A, C, G and T compares it
+// with the layer's letters and goes the way of the others from there: those
+// windows in lower case take 19.7 wave-seconds of DP, 11.1 in upper case and
+// 36.6 in the general form.
 //
 // The rows are bound by their instructions: a wave alone issues one about
 // every 8 cycles, and 4 waves per SIMD share the issue slots. A row whose one
@@ -747,10 +752,13 @@ __device__ __forceinline__ uint32_t pk_splat(int32_t v) {
 
 // Row descriptor: number of predecessors (0: the general form), 8 x the code
 // of the row's base, own slot, slots of up to four predecessors, whether the
-// single predecessor is the row before, and the sink flag. The general form
-// has the sink flag and kRecMoves, set when the row keeps a move record.
+// single predecessor is the row before, and the sink flag. A row of another
+// letter has kRecOther and no number and code (the number is in its meta
+// word); the general form has the sink flag and kRecMoves, set when the row
+// keeps a move record (also with kRecOther).
 constexpr uint32_t kRecPreds = 7u;
 constexpr uint32_t kRecMoves = 8u;
+constexpr uint32_t kRecOther = 16u;
 constexpr uint32_t kRecBase = 0x18u;
 constexpr int kRecOwnShift = 5;
 constexpr int kRecPredShift = 10;
@@ -926,7 +934,7 @@ __device__ __forceinline__ void row_kinds(const uint32_t* h, const uint32_t* bd,
 }
 
 // Scores of a pair whose letters are not all A, C, G or T: those match no row
-// of the descriptor form (a row of another letter takes the general form).
+// of these four (a row of another letter compares letters).
 constexpr uint32_t kOddLetter = 0x0d0du;  // their selector
 __device__ __forceinline__ uint32_t odd_letters(uint32_t sub, uint32_t sel, uint32_t miss) {
   const uint32_t m = ((sel >> 3) & sel & 0x00010001u) * 0xffffu;
@@ -995,6 +1003,9 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
   uint32_t cur[H2];  // the scores of the row before
 #pragma unroll
   for (int q = 0; q < H2; ++q) cur[q] = 0;
+  // position in seq of the letter of the strip's first column (-1: column 0
+  // has none; lanes past the last column read the bytes behind the layer)
+  const int letters = min(lane * W, pitch - W) - 1;
   GByte* const codes = (GByte*)s.code();
   uint32_t rec_lane = min(static_cast<uint32_t>(lane * row_record_bytes(W)),
                           row_bytes - static_cast<uint32_t>(row_record_bytes(W)));
@@ -1093,12 +1104,27 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
         *(__attribute__((address_space(1))) U32x4*)at = U32x4{acc[0], acc[1], ack[0], ack[1]};
       }
     };
+    // scores of the strip's letters against a row's, letter by letter
+    const auto letter_scores = [&](uint32_t letter, uint32_t* out) {
+      const uint32_t other = (letter & 0xffu) * 0x10001u;
+      const uint32_t hit = miss ^ flip;
+#pragma unroll
+      for (int q = 0; q < H2; ++q) {
+        // (column 0's position is before the first)
+        const uint32_t a = seq[q == 0 ? max(letters, 0) : letters + 2 * q];
+        const uint32_t b = seq[letters + 2 * q + 1];
+        const uint32_t differ = pk_min_u((a | b << 16) ^ other, one);
+        out[q] = pk_mad(differ, pk_sub(miss * 0x10001u, hit * 0x10001u), hit * 0x10001u);
+      }
+      if (lane == 0) out[0] &= 0xffff0000u;  // column 0 has no letter
+    };
     next_row(0);
     int rr = 0;
+    uint32_t np = d & kRecPreds;
     for (;;) {
       // rows of up to four predecessors (a loop of their own: the common
       // ones go through without a taken branch)
-      uint32_t np = d & kRecPreds, np_next = 0;
+      uint32_t np_next = 0;
       while (np != 0) {
         const auto slot_at = [&](int k) {
           return strip + ((d >> (kRecPredShift + 5 * k)) & 31u) * row_bytes;
@@ -1173,6 +1199,20 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
         np = np_next;
       }
       if (rr >= chunk) break;
+      if ((d & (kRecPreds | kRecOther)) == kRecOther) {
+        // a row of another letter: it goes through the loop above with its
+        // own scores
+        const uint32_t meta = static_cast<uint32_t>(__builtin_amdgcn_readlane(meta_v, rr));
+        np = (meta >> kRowMetaPredShift) & kRowMetaPredMask;
+        if constexpr (kPlain) {
+          table = table0;  // it matches none of the layer's
+#pragma unroll
+          for (int q = 0; q < H2; ++q) next_sub(q);
+        } else {
+          letter_scores(meta, sub);
+        }
+        continue;
+      }
       record += row_bytes;
       {
         uint32_t bd[H2], bv[H2];
@@ -1228,17 +1268,9 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
           }
         }
         uint32_t scores[H2];
+        letter_scores(static_cast<uint32_t>(meta), scores);
 #pragma unroll
         for (int q = 0; q < H2; ++q) {
-          uint32_t x = 0;
-#pragma unroll
-          for (int u = 0; u < 2; ++u) {
-            const int idx = j0 + 2 * q + u - 1;
-            const bool same = idx >= 0 && idx < L && static_cast<int>(seq[idx]) == (meta & 0xff);
-            const int v = idx < 0 ? 0 : (same ? match : mismatch) - gap;
-            x |= (static_cast<uint32_t>(v) & 0xffffu) << (16 * u);
-          }
-          scores[q] = x;
           // (a move, so that mx and cur need not share registers)
           asm volatile("v_mov_b32 %0, %1" : "=v"(cur[q]) : "v"(mx[q]));
         }
@@ -1285,6 +1317,7 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
       }
       ++rr;
       next_row(rr);
+      np = d & kRecPreds;
     }
   }
   *best_score = best;
@@ -1448,11 +1481,10 @@ __device__ __forceinline__ int dp_band(CParams& P, const Slot& s, uint32_t lds, 
       const uint32_t d = static_cast<uint32_t>(
           __builtin_amdgcn_readlane(static_cast<int>(desc_v), rr));
       const int lo = __builtin_amdgcn_readlane(lo_v, rr);
-      const uint32_t np = d & kRecPreds;
+      uint32_t np = d & kRecPreds;
       uint32_t bd[2], bv[2], sub[2];
+      bool general = false;
       if (np != 0) {
-        const uint32_t shifts = static_cast<uint32_t>(
-            __builtin_amdgcn_readlane(static_cast<int>(shift_v), rr));
         if (lo != sel_lo) {
           // letters of columns lo + 1 + 4 lane .. (bytes past the layer are
           // never read back)
@@ -1481,6 +1513,24 @@ __device__ __forceinline__ int dp_band(CParams& P, const Slot& s, uint32_t lds, 
           sub[0] = odd_letters(sub[0], sel[0], miss * 0x10001u);
           sub[1] = odd_letters(sub[1], sel[1], miss * 0x10001u);
         }
+      } else if ((d & kRecOther) != 0) {
+        // a row of another letter
+        const uint32_t meta = static_cast<uint32_t>(__builtin_amdgcn_readlane(meta_v, rr));
+        np = (meta >> kRowMetaPredShift) & kRowMetaPredMask;
+        const uint32_t w = *(const LWord*)(size_t)(seq_at + static_cast<uint32_t>(lo + kBandW * lane));
+        const uint32_t hit = miss ^ flip;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const uint32_t pair = __builtin_amdgcn_perm(0u, w, q == 0 ? 0x0c010c00u : 0x0c030c02u);
+          const uint32_t differ = pk_min_u(pair ^ (meta & 0xffu) * 0x10001u, one);
+          sub[q] = pk_mad(differ, pk_sub(miss * 0x10001u, hit * 0x10001u), hit * 0x10001u);
+        }
+      } else {
+        general = true;
+      }
+      if (!general) {
+        const uint32_t shifts = static_cast<uint32_t>(
+            __builtin_amdgcn_readlane(static_cast<int>(shift_v), rr));
         const auto row_at = [&](int k) {
           return lds + ((d >> (kRecPredShift + 5 * k)) & 31u) * row_bytes;
         };
@@ -1608,7 +1658,9 @@ __device__ __forceinline__ int dp_band(CParams& P, const Slot& s, uint32_t lds, 
           uint32_t acc[1];
           row_kinds<kBandW>(cur, bd, bv, acc);
           store_moves(acc[0], (kx[0] << 2) | kx[1], lo);
-          if (lane == 0) record[(lo >> 2) * 2 + 1] = static_cast<uint8_t>(k_left << 4);
+          if (n_preds > 1 && lane == 0) {
+            record[(lo >> 2) * 2 + 1] = static_cast<uint8_t>(k_left << 4);
+          }
         } else {
           // 16-bit codes, column j at element j + 3
           const uint32_t kprev = shift_into(k_left << 16, kx[1]);
@@ -2355,7 +2407,8 @@ __device__ __noinline__ int build_rows(GByte* slot_base, CLayout* layout, int V,
     const bool sink = last == 0;
     if (in) {
       row_meta[r] = letter | (sink ? kRowMetaSink : 0) |
-                    (my_slot << kRowMetaSlotShift) | (my_pool << kRowMetaGShift);
+                    (my_slot << kRowMetaSlotShift) | (my_pool << kRowMetaGShift) |
+                    min(np, kRowMetaPredMask) << kRowMetaPredShift;
       if (words) {
         word[r] = static_cast<uint32_t>(my_slot);
       } else if (bytes) {
@@ -2374,9 +2427,10 @@ __device__ __noinline__ int build_rows(GByte* slot_base, CLayout* layout, int V,
     };
     // the row's descriptor, unless it takes the general form
     const int code = ((letter >> 1) ^ (letter >> 2)) & 3;
-    bool fast = packed && np >= 1 && np <= static_cast<int>(kRecMaxPreds) && my_slot != kSlotGlobal &&
-                static_cast<int>((0x54474341u >> (8 * code)) & 0xffu) == letter;
-    uint32_t fields = static_cast<uint32_t>(np) | static_cast<uint32_t>(code << 3) |
+    bool fast = packed && np >= 1 && np <= static_cast<int>(kRecMaxPreds) && my_slot != kSlotGlobal;
+    const bool base = static_cast<int>((0x54474341u >> (8 * code)) & 0xffu) == letter;
+    uint32_t fields = (base ? static_cast<uint32_t>(np) | static_cast<uint32_t>(code << 3)
+                            : kRecMoves | kRecOther) |
                       static_cast<uint32_t>(my_slot) << kRecOwnShift;
     uint64_t deltas = 0;  // row deltas of the first four predecessors (0: none or too far)
     int p[kInline], sl[kInline];
@@ -2760,7 +2814,7 @@ __device__ __noinline__ int trace_rows(GByte* slot_base, CLayout* layout, int pi
       // leave the index left of the band unwritten
       const int field = 62 - 2 * j0;
       if (first == 0) kinds = (kinds & ~(3ull << field)) | 2ull << field;
-      if ((rec.x & kRecPreds) == 1) preds = 0;
+      if (rec.z < 0x10000u) preds = 0;
     }
     // A cell takes one move: diagonal before vertical. Its predecessor index is
     // the one kept at the column before for a diagonal, at its own column for

@@ -93,3 +93,28 @@ def test_many_predecessors():
             layers.append(Layer(seq, None, 0, 399))
         wins.append(Window(backbone, b"!" * 400, layers))
     check(wins)
+
+
+def consensus(windows, ring):
+    b = _lib.PoaBatch(3, -5, -4, trim=True)
+    b.set_band(256)
+    if ring:
+        b.set_tuning(0, 0, ring)
+    b.upload(windows)
+    b.run(_lib.RH_POA_BATCHED)
+    out, _ = b.download()
+    b.close()
+    return out
+
+
+@pytest.mark.parametrize("ring", [0, 2])
+def test_rows_of_another_letter(ring):
+    """Alignments depend on which letters are equal only: windows in lower
+    case give the same consensus in lower case, also where the band is an
+    approximation (the oracle has no band)."""
+    rng = np.random.default_rng(37)
+    wins = [window(rng, n, 9) for n in (280, 505, 900, 1400)]
+    lower = [Window(w.backbone.lower(), w.backbone_quality,
+                    [Layer(l.sequence.lower(), l.quality, l.begin, l.end) for l in w.layers])
+             for w in wins]
+    assert consensus(lower, ring) == [c.lower() for c in consensus(wins, ring)]

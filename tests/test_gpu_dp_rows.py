@@ -149,3 +149,26 @@ def test_rows_of_the_general_form_trace_in_tiles(form):
     else:
         general = run_phases([lower(w) for w in wins])["traceback"]
     assert general < 2 * plain
+
+
+def test_rows_of_another_letter_stay_near_the_others():
+    """The DP of rows of other letters costs about what the others' does (the
+    general form took 3.3 times as long, a row of byte compares 2.4)."""
+    rng = np.random.default_rng(41)
+    wins = [window(rng, 500, 12) for _ in range(24)] * 50
+    assert run_phases([lower(w) for w in wins])["dp"] < 2.4 * run_phases(wins)["dp"]
+
+
+@pytest.mark.parametrize("length", [60, 300, 600, 900, 1150])
+@pytest.mark.parametrize("ring", [0, 2])
+def test_windows_of_two_cases(length, ring):
+    """Rows of other letters beside the rest, with and without an LDS slot:
+    layers in lower case, half in lower case, and in upper case."""
+    rng = np.random.default_rng(length + 1)
+    win = window(rng, length, 9, error=0.2)
+    half = length // 2
+    win.backbone = win.backbone[:half].lower() + win.backbone[half:]
+    for k, layer in enumerate(win.layers):
+        seq = layer.sequence
+        layer.sequence = (seq.lower(), seq[:half].lower() + seq[half:], seq)[k % 3]
+    check([win, lower(win)], ring=ring)
