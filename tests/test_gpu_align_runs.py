@@ -93,3 +93,40 @@ def test_other_bytes_at_chunk_edges(letter):
             q[at] = letter[0]
         pairs.append((bytes(q), bytes(t)))
     check(pairs)
+
+
+@pytest.mark.parametrize("length", [63, 64, 65, 129, 500, 1500])
+def test_long_gaps(length):
+    """Leaves whose paths are mostly gaps: bands of insertions over block
+    edges, bands of deletions, and both at the ends of a pair, one wave per
+    pair and in teams."""
+    rng = np.random.default_rng(length)
+    t = random_seq(rng, 8000)
+    q = mutate(rng, t, 0.1)
+    long_t = random_seq(rng, 14000)
+    check([(q[:length], t), (q[-length:], t), (q, t[:length]), (q, t[-length:]),
+           (q, t[:4000] + t[4000 + length:]), (q[:4000] + q[4000 + length:], t),
+           (random_seq(rng, length), t), (t, random_seq(rng, length)),
+           (long_t, random_seq(rng, length)), (random_seq(rng, length), long_t)])
+
+
+def test_long_gaps_cost_no_more_than_matches():
+    """An op of a gap is no round trip of its own: a pair of unequal lengths
+    takes less than the square pair of the longer one (up to 2.9 times as long
+    with a round trip per op)."""
+    rng = np.random.default_rng(31)
+    pairs = [make_pair(rng, 8000, 0.12) for _ in range(20)]
+
+    def kernel_ms(batch):
+        b = _lib.AlignBatch()
+        b.upload(batch)
+        times = []
+        for _ in range(4):
+            b.run()
+            times.append(b.stats().kernel_ms)
+        b.close()
+        return min(times)
+
+    square = kernel_ms(pairs)
+    assert kernel_ms([(q, t[:200]) for q, t in pairs]) < square
+    assert kernel_ms([(q[:200], t) for q, t in pairs]) < 2 * square
