@@ -300,34 +300,45 @@ int32_t rh_align_run(rh_align_batch* b) {
   RH_HIP_CHECK(b->d_queue.reserve(2 * sizeof(uint32_t)), RH_ERR_MEMORY);
   RH_HIP_CHECK(hipMemsetAsync(b->d_queue.ptr, 0, 2 * sizeof(uint32_t), b->stream), RH_ERR_DEVICE);
   RH_HIP_CHECK(hipEventRecord(b->ev0, b->stream), RH_ERR_DEVICE);
-  for (size_t k = 0; k < parts.size(); ++k) {
-    const Part& part = parts[k];
-    rh::AlignParams p{};
-    p.pairs = b->d_pairs.as<rh::AlignPair>();
-    p.arena = b->d_arena.as<uint8_t>();
-    p.ops = b->d_ops.as<uint8_t>();
-    p.results = b->d_results.as<rh::AlignResult>();
-    p.order = b->d_order.as<uint32_t>() + part.first;
-    p.n_order = part.n;
-    p.queue_head = b->d_queue.as<uint32_t>() + k;
-    p.scratch = part.scratch->as<uint8_t>();
-    p.slot_bytes = part.slot_bytes;
-    p.caps = part.caps;
-    p.layout = part.layout;
-    p.band0 = b->band0;
-    p.waves = part.waves;
-    if (part.stream != b->stream) {
-      RH_HIP_CHECK(hipStreamWaitEvent(part.stream, b->ev0, 0), RH_ERR_DEVICE);
+  const auto launch_and_wait = [&]() -> int32_t {
+    for (size_t k = 0; k < parts.size(); ++k) {
+      const Part& part = parts[k];
+      rh::AlignParams p{};
+      p.pairs = b->d_pairs.as<rh::AlignPair>();
+      p.arena = b->d_arena.as<uint8_t>();
+      p.ops = b->d_ops.as<uint8_t>();
+      p.results = b->d_results.as<rh::AlignResult>();
+      p.order = b->d_order.as<uint32_t>() + part.first;
+      p.n_order = part.n;
+      p.queue_head = b->d_queue.as<uint32_t>() + k;
+      p.scratch = part.scratch->as<uint8_t>();
+      p.slot_bytes = part.slot_bytes;
+      p.caps = part.caps;
+      p.layout = part.layout;
+      p.band0 = b->band0;
+      p.waves = part.waves;
+      if (part.stream != b->stream) {
+        RH_HIP_CHECK(hipStreamWaitEvent(part.stream, b->ev0, 0), RH_ERR_DEVICE);
+      }
+      RH_HIP_CHECK(rh::launch_align_batch(p, static_cast<uint32_t>(part.slots), part.stream),
+                   RH_ERR_KERNEL);
+      if (part.stream != b->stream) {
+        RH_HIP_CHECK(hipEventRecord(b->ev_team, part.stream), RH_ERR_DEVICE);
+      }
     }
-    RH_HIP_CHECK(rh::launch_align_batch(p, static_cast<uint32_t>(part.slots), part.stream),
-                 RH_ERR_KERNEL);
-    if (part.stream != b->stream) {
-      RH_HIP_CHECK(hipEventRecord(b->ev_team, part.stream), RH_ERR_DEVICE);
-    }
+    if (teams > 0) RH_HIP_CHECK(hipStreamWaitEvent(b->stream, b->ev_team, 0), RH_ERR_DEVICE);
+    RH_HIP_CHECK(hipEventRecord(b->ev1, b->stream), RH_ERR_DEVICE);
+    RH_HIP_CHECK(hipEventSynchronize(b->ev1), RH_ERR_KERNEL);
+    return RH_OK;
+  };
+  const int32_t rc = launch_and_wait();
+  if (rc != RH_OK) {
+    // a kernel may be running on either stream, and only b->stream is what the
+    // batch's next upload or run is ordered by
+    (void)hipStreamSynchronize(b->team_stream);
+    (void)hipStreamSynchronize(b->stream);
+    return rc;
   }
-  if (teams > 0) RH_HIP_CHECK(hipStreamWaitEvent(b->stream, b->ev_team, 0), RH_ERR_DEVICE);
-  RH_HIP_CHECK(hipEventRecord(b->ev1, b->stream), RH_ERR_DEVICE);
-  RH_HIP_CHECK(hipEventSynchronize(b->ev1), RH_ERR_KERNEL);
   float ms = 0;
   RH_HIP_CHECK(hipEventElapsedTime(&ms, b->ev0, b->ev1), RH_ERR_DEVICE);
   b->stats.kernel_ms = ms;
