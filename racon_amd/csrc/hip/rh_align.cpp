@@ -265,7 +265,7 @@ int32_t rh_align_run(rh_align_batch* b) {
   // their own, beside the rest
   int waves_per_cu = 0;
   RH_HIP_CHECK(rh::align_occupancy(&waves_per_cu, 1), RH_ERR_DEVICE);
-  const uint32_t teams = rh::align_team_pairs(
+  uint32_t teams = rh::align_team_pairs(
       b->pairs, b->order, static_cast<uint64_t>(std::max(1, waves_per_cu)) * std::max(1, cus));
   struct Part {
     uint32_t first, n, waves;
@@ -276,25 +276,48 @@ int32_t rh_align_run(rh_align_batch* b) {
     hipStream_t stream;
   };
   std::vector<Part> parts;
-  if (teams > 0) parts.push_back(Part{0, teams, rh::kAlignTeamWaves, 0, 0, {}, {}, &b->d_team, b->team_stream});
-  if (teams < n) parts.push_back(Part{teams, n - teams, 1, 0, 0, {}, {}, &b->d_scratch, b->stream});
-  // (the slots of both parts within 60% of the free memory)
-  const uint64_t budget =
-      (free_b + b->d_scratch.bytes + b->d_team.bytes) * 6 / 10 / parts.size();
-  for (Part& part : parts) {
-    uint32_t max_q = 0, max_t = 0;
-    for (uint32_t k = part.first; k < part.first + part.n; ++k) {
-      max_q = std::max(max_q, b->pairs[b->order[k]].q_len);
-      max_t = std::max(max_t, b->pairs[b->order[k]].t_len);
+  // slots of both parts within 60% of what is free or in the batch's scratch
+  const uint64_t room = (free_b + b->d_scratch.bytes + b->d_team.bytes) * 6 / 10;
+  for (bool fits = false; !fits;) {
+    parts.clear();
+    if (teams > 0) parts.push_back(Part{0, teams, rh::kAlignTeamWaves, 0, 0, {}, {}, &b->d_team, b->team_stream});
+    if (teams < n) parts.push_back(Part{teams, n - teams, 1, 0, 0, {}, {}, &b->d_scratch, b->stream});
+    const uint64_t budget = room / parts.size();
+    fits = true;
+    for (Part& part : parts) {
+      uint32_t max_q = 0, max_t = 0;
+      for (uint32_t k = part.first; k < part.first + part.n; ++k) {
+        max_q = std::max(max_q, b->pairs[b->order[k]].q_len);
+        max_t = std::max(max_t, b->pairs[b->order[k]].t_len);
+      }
+      part.caps = rh::align_caps_for(max_q, max_t);
+      part.layout = rh::align_slot_layout(part.caps, part.waves);
+      part.slot_bytes = rh::align_up_a(part.layout.total, 4096);
+      int per_cu = 0;
+      RH_HIP_CHECK(rh::align_occupancy(&per_cu, part.waves), RH_ERR_DEVICE);
+      uint64_t slots = static_cast<uint64_t>(std::max(1, per_cu)) * std::max(1, cus);
+      slots = std::min<uint64_t>(slots, std::max<uint64_t>(1, budget / part.slot_bytes));
+      part.slots = std::min<uint64_t>(slots, part.n);
+      fits = fits && part.slot_bytes <= budget;
     }
-    part.caps = rh::align_caps_for(max_q, max_t);
-    part.layout = rh::align_slot_layout(part.caps, part.waves);
-    part.slot_bytes = rh::align_up_a(part.layout.total, 4096);
-    int per_cu = 0;
-    RH_HIP_CHECK(rh::align_occupancy(&per_cu, part.waves), RH_ERR_DEVICE);
-    uint64_t slots = static_cast<uint64_t>(std::max(1, per_cu)) * std::max(1, cus);
-    slots = std::min<uint64_t>(slots, std::max<uint64_t>(1, budget / part.slot_bytes));
-    part.slots = std::min<uint64_t>(slots, part.n);
+    // (a team's slot is six times a wave's: with little memory every pair
+    // runs on one wave)
+    if (teams == 0) break;
+    if (!fits) teams = 0;
+  }
+  // where a buffer grows, what both keep of earlier batches counts too:
+  // together they stay within the room, or one would grow into what the other
+  // holds, and the next upload find nothing left
+  const uint64_t held = b->d_scratch.bytes + b->d_team.bytes;
+  uint64_t kept = held;
+  for (const Part& part : parts) {
+    kept += std::max(part.slots * part.slot_bytes, part.scratch->bytes) - part.scratch->bytes;
+  }
+  if (kept > held && kept > room) {
+    b->d_scratch.release();
+    b->d_team.release();
+  }
+  for (const Part& part : parts) {
     RH_HIP_CHECK(part.scratch->reserve(part.slots * part.slot_bytes), RH_ERR_MEMORY);
   }
   RH_HIP_CHECK(b->d_queue.reserve(2 * sizeof(uint32_t)), RH_ERR_MEMORY);

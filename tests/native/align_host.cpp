@@ -173,10 +173,54 @@ int errors() {
   }
   return bad("no run without a failure");
 }
+
+// Batches of few long, many short and both kinds of pairs on one object, in
+// every order: what a batch kept for the last one never refuses the next.
+int memory() {
+  std::vector<rh_pair> kinds[3];
+  add(kinds[0], 40, 8000);    // one wave each
+  add(kinds[1], 8, 40000);    // teams
+  add(kinds[2], 8, 40000);
+  add(kinds[2], 200, 8000);   // both
+  for (size_t mb : {48u, 64u, 96u, 160u, 400u}) {
+    pool = mb << 20;
+    for (int order = 0; order < 27; ++order) {
+      rh_align_batch* b = nullptr;
+      if (rh_align_create(0, &b) != RH_OK) return bad("create");
+      for (int at = order, k = 0; k < 3; ++k, at /= 3) {
+        const std::vector<rh_pair>& pairs = kinds[at % 3];
+        if (rh_align_upload(b, pairs.size(), pairs.data()) != RH_OK) return bad("upload");
+        if (rh_align_run(b) != RH_OK) {
+          return bad("order " + std::to_string(order) + " batch " + std::to_string(k) + " of " +
+                     std::to_string(mb) + " MB refused");
+        }
+      }
+      rh_align_destroy(b);
+      if (in_use != 0 || !problem.empty()) return bad("left: " + problem);
+    }
+  }
+  return 0;
+}
+
+// A team's slot that outgrows the memory: its pairs run one wave each, as
+// long as one such slot fits.
+int small() {
+  std::vector<rh_pair> pairs;
+  add(pairs, 4, 100000);
+  pool = 16u << 20;
+  rh_align_batch* b = nullptr;
+  if (rh_align_create(0, &b) != RH_OK) return bad("create");
+  if (rh_align_upload(b, pairs.size(), pairs.data()) != RH_OK) return bad("upload");
+  if (rh_align_run(b) != RH_OK) return bad("refused");
+  rh_align_destroy(b);
+  return problem.empty() ? 0 : bad(problem);
+}
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::string scenario = argc > 1 ? argv[1] : "";
   if (scenario == "errors") return errors();
+  if (scenario == "memory") return memory();
+  if (scenario == "small") return small();
   return bad("unknown scenario " + scenario);
 }
