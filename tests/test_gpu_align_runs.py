@@ -1,9 +1,9 @@
 """The banded runs of the overlap aligner at the edges of their forms, against
 the CPU oracle: block and chunk remainders, every group of lanes (8 to 64, and
-256 over the four waves of a team), bands too wide for the lanes (strips),
-band guesses that must grow, few long pairs (a team of waves per pair) beside
-many (one wave per pair), and target bytes other than A, C, G and T at chunk
-edges.
+256 over the four waves of a team), bands too wide for the lanes of a wave and
+of a team (strips), band guesses that must grow, few long pairs (a team of
+waves per pair) alone and beside many (one wave per pair), long pairs on one
+wave each, long gaps, and target bytes other than A, C, G and T at chunk edges.
 """
 import sys
 
@@ -12,6 +12,7 @@ import pytest
 
 from racon_amd import _lib
 from synth import make_pair, mutate, random_seq
+from test_zz_no_alloc import Hip, noalloc_align
 
 sys.path.insert(0, _lib.PKG_DIR + "/../oracle")
 import oracle_py  # noqa: E402
@@ -19,14 +20,20 @@ import oracle_py  # noqa: E402
 pytestmark = pytest.mark.gpu
 
 
-def check(pairs, band=0, only=None):
+def check(pairs, band=0, only=None, launches=None):
+    """launches: 2 for teams beside one wave per pair, 1 for either alone."""
     b = _lib.AlignBatch()
     if band:
         b.set_band(band)
     b.upload(pairs)
     b.run()
     ops, dist = b.download()
+    assert launches in (None, b.stats().launches)
     b.close()
+    compare(pairs, ops, dist, only)
+
+
+def compare(pairs, ops, dist, only=None):
     for i, (q, t) in enumerate(pairs):
         if only is not None and i not in only:
             continue
@@ -69,15 +76,40 @@ def test_few_long_pairs_take_a_team():
     t = random_seq(rng, 14000)
     pairs.append((mutate(rng, t[:5000] + t[9000:], 0.1), t))
     pairs.append((random_seq(rng, 5000), random_seq(rng, 11000)))
-    check(pairs)
+    check(pairs, launches=2)
 
 
-def test_one_wave_per_pair_with_wide_bands():
+def test_strips_of_a_team():
+    """Bands of more than 16,400 diagonals, too wide for the 256 lanes of half
+    a team: strips, dealt to the team's waves."""
+    rng = np.random.default_rng(43)
+    pairs = [make_pair(rng, 20000, 0.1), make_pair(rng, 17000, 0.3), make_pair(rng, 300, 0.1)]
+    t = random_seq(rng, 22000)
+    pairs += [(mutate(rng, t[3000:20500], 0.1), t), (t, mutate(rng, t[:18000], 0.1))]
+    check(pairs, band=20000, launches=2)
+
+
+def test_long_pairs_on_one_wave():
+    """Pairs that a batch would give to teams, through the entry point that
+    runs one wave per pair: strips at the top of the recursion."""
+    rng = np.random.default_rng(47)
+    pairs = [make_pair(rng, 24000, 0.15), make_pair(rng, 12000, 0.12), make_pair(rng, 19500, 0.05),
+             (random_seq(rng, 6000), random_seq(rng, 12000)), make_pair(rng, 300, 0.1)]
+    hip = Hip()
+    try:
+        ops, dist, status = noalloc_align(pairs, hip)
+    finally:
+        hip.free()
+    assert status == [0] * len(pairs)
+    compare(pairs, ops, dist)
+
+
+def test_long_pairs_beside_many_short_ones():
     rng = np.random.default_rng(23)
     pairs = [make_pair(rng, 200, 0.1) for _ in range(2100)]
     pairs[7] = make_pair(rng, 24000, 0.15)
     pairs[900] = (random_seq(rng, 6000), random_seq(rng, 12000))
-    check(pairs, only=(0, 7, 8, 900, 2099))
+    check(pairs, only=(0, 7, 8, 900, 2099), launches=2)
 
 
 @pytest.mark.parametrize("letter", [b"N", b"n", b"R"])
