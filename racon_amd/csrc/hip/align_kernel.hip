@@ -417,11 +417,6 @@ __device__ __forceinline__ int nth_bit(unsigned long long m, int n) {
   return __ffsll(static_cast<long long>(m)) - 1;
 }
 
-template <int kWaves>
-__device__ __forceinline__ void team_sync() {
-  __syncthreads();
-}
-
 // ---- banded runs: blocks on lanes, cyclically along the band ----
 //
 // A run is one bit-vector DP of a (sub)problem over its diagonal band: the
@@ -600,7 +595,6 @@ struct FinalState {
 struct PairView {
   const uint8_t* Q;
   const uint8_t* T;
-  int QL, TL;
   const PlaneWord* planes;  // word w: rows 64 (w - 1) .. (one guard word in front)
   U4* store;                // this wave's leaf columns
   int32_t* col_left;
@@ -1146,8 +1140,6 @@ __device__ __forceinline__ void align_pair(const AlignParams& A, const AlignPair
   PairView v;
   v.Q = A.arena + pr.q_off;
   v.T = A.arena + pr.t_off;
-  v.QL = QL;
-  v.TL = TL;
   v.planes = planes;
   v.store = reinterpret_cast<U4*>(slot + A.layout.store) + static_cast<uint64_t>(wave) * A.caps.store_words;
   v.col_left = reinterpret_cast<int32_t*>(slot + A.layout.col_left);
@@ -1179,7 +1171,7 @@ __device__ __forceinline__ void align_pair(const AlignParams& A, const AlignPair
     team_steps = 0;
     cur[0] = AlignTask{0, QL, 0, TL, -1};
   }
-  team_sync<kWaves>();
+  __syncthreads();
   int n_cur = 1;
   int best = -1;
 
@@ -1267,11 +1259,10 @@ __device__ __forceinline__ void align_pair(const AlignParams& A, const AlignPair
         }
       }
     }
-    team_sync<kWaves>();
+    __syncthreads();
     // ---- split rows ----
-    bool retry = false;
     int number = 0;
-    for (int i = 0; i < n_cur && !retry; ++i) {
+    for (int i = 0; i < n_cur; ++i) {
       const AlignTask t = uniform_task(cur[i]);
       if (t.ql == 0 || t.tl == 0 || is_leaf(t.ql, t.tl)) continue;
       if (number++ % kWaves != wave) continue;
@@ -1343,7 +1334,7 @@ __device__ __forceinline__ void align_pair(const AlignParams& A, const AlignPair
         }
       }
     }
-    team_sync<kWaves>();
+    __syncthreads();
     const AlignTask top = uniform_task(cur[0]);
     const bool unknown = top.score < 0;
     if (unknown && !is_leaf(top.ql, top.tl)) {
@@ -1351,7 +1342,7 @@ __device__ __forceinline__ void align_pair(const AlignParams& A, const AlignPair
       if (m > k_top && !full_band(band_for(top.ql, top.tl, k_top), top.ql, top.tl)) {
         // outside the guess: nothing was added to the next level
         k_top *= 2;
-        team_sync<kWaves>();
+        __syncthreads();
         continue;
       }
       best = m;
@@ -1486,14 +1477,14 @@ __device__ __forceinline__ void align_pair(const AlignParams& A, const AlignPair
         wave_done();
       }
     }
-    team_sync<kWaves>();
+    __syncthreads();
     n_cur = uniform(team_next);
     AlignTask* x = cur;
     cur = next;
     next = x;
-    team_sync<kWaves>();
+    __syncthreads();
     if (threadIdx.x == 0) team_next = 0;
-    team_sync<kWaves>();
+    __syncthreads();
   }
   // ---- pack the ops ----
   const int total = QL + TL;
@@ -1519,7 +1510,7 @@ __device__ __forceinline__ void align_pair(const AlignParams& A, const AlignPair
     }
     for (int s = 1; s < kWave; s <<= 1) c += __shfl_xor(c, s, kWave);
     if (lane == 0) team_ops[wave] = c;
-    team_sync<kWaves>();
+    __syncthreads();
     for (int w = 0; w < wave; ++w) count += team_ops[w];
   }
   for (int i0 = from; i0 < to; i0 += kWave * 16) {
@@ -1547,7 +1538,7 @@ __device__ __forceinline__ void align_pair(const AlignParams& A, const AlignPair
   if (kWaves > 1) {
     if (wave == kWaves - 1 && lane == 0) team_next = count;
     if (lane == 0) atomicAdd(&team_steps, steps);
-    team_sync<kWaves>();
+    __syncthreads();
     count = uniform(team_next);
     steps = uniform(static_cast<int>(team_steps));
   }

@@ -20,12 +20,14 @@
 // After the last layer: heaviest-bundle path with branch completion,
 // per-position coverage and racon's trimming (window.cpp:115-139).
 //
-// The graph walks (steps 1, 2, 4, 5 and the consensus) are inherently
-// sequential; the wave runs them lane-uniformly (every lane executes the same
-// loads and branches) so no lane-0 divergence or broadcast is needed, and the
-// slot stays L2-resident for small windows. Parallelism comes from thousands
-// of windows in flight (persistent kernel over a size-ordered queue) and from
-// the 64-lane DP rows.
+// The subgraph closure, the row tables, the insertion and the new order work on
+// 64 ranks, rows or layer positions at a time. What is sequential by nature
+// (the walk along the recorded moves, the exact DFS order where a tie asks for
+// it, the insertion of a path whose nodes share an aligned set, the consensus
+// path) the wave runs lane-uniformly: every lane executes the same loads and
+// branches, so no lane-0 divergence or broadcast is needed. Parallelism comes
+// from thousands of windows in flight (persistent kernel over a size-ordered
+// queue) and from the 64-lane DP rows.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -78,13 +80,11 @@ constexpr int kStrip = 4;                  // DP columns per lane per tile
 constexpr int kTile = kWave * kStrip;      // 256 columns per tile
 constexpr int32_t kNegInf = -(1 << 29);
 // Move codes (16 bits per DP cell): bits 15-14 the move (diagonal,
-// vertical, horizontal); for diagonal and vertical moves bits 12-0 name the
-// predecessor row, as the row delta r - p, or, with kCodeViaK set, as the
-// index k of the predecessor in the row's in-edge list.
+// vertical, horizontal); for diagonal and vertical moves bits 12-0 are the
+// index of the predecessor in the row's in-edge list.
 constexpr uint16_t kCodeDiag = 0x0000;
 constexpr uint16_t kCodeVert = 0x4000;
 constexpr uint16_t kCodeHorz = 0x8000;
-constexpr uint16_t kCodeViaK = 0x2000;
 constexpr uint32_t kCodePayload = 0x1fff;
 // Bits 16..22 of a row's meta word: the row's entry in the slot's pool of
 // global score rows (a row that found no LDS slot, in a pass with a pool).
@@ -535,7 +535,7 @@ __device__ __forceinline__ int dp_layer(CParams& P, const Slot& s, uint8_t* lds,
     if (lane == 0) {
       if (own < kSlotGlobal) Hr[kColShift] = static_cast<T>(c0);
       if (own == kSlotGlobal) Hg[0] = c0;
-      Cr[pitch - 1] = kCodeVert | kCodeViaK | static_cast<uint16_t>(k0);
+      Cr[pitch - 1] = kCodeVert | static_cast<uint16_t>(k0);
     }
     int32_t carry = c0;
     int32_t h_last = kNegInf;
@@ -612,8 +612,8 @@ __device__ __forceinline__ int dp_layer(CParams& P, const Slot& s, uint8_t* lds,
 #pragma unroll
       for (int u = 0; u < kStrip; ++u) {
         h[u] = max(pre[u], in_carry) + (j0 + u) * gap;
-        const uint32_t c_diag = kCodeDiag | kCodeViaK | (kk[u] & 0xffffu);
-        const uint32_t c_vert = kCodeVert | kCodeViaK | (kk[u] >> 16);
+        const uint32_t c_diag = kCodeDiag | (kk[u] & 0xffffu);
+        const uint32_t c_vert = kCodeVert | (kk[u] >> 16);
         cd[u] = bd[u] == h[u] ? c_diag : (bv[u] == h[u] ? c_vert : kCodeHorz);
       }
       if (live) {
@@ -1293,7 +1293,7 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
           }
           store_moves(acc, ack);
         } else {
-          // codes: kCodeViaK | index of the predecessor
+          // 16-bit codes
           uint32_t kprev = shift_into(0u, kx[H2 - 1]);
           uint16_t* Cr = s.code() + static_cast<int64_t>(r) * pitch;
 #pragma unroll
@@ -1306,8 +1306,8 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
               const bool dg = ((bd[q] >> (16 * u)) & 0xffffu) == hu;
               const bool vt = ((bv[q] >> (16 * u)) & 0xffffu) == hu;
               const uint32_t kdu = (kd >> (16 * u)) & 0xffffu, kvu = (kx[q] >> (16 * u)) & 0xffffu;
-              const uint32_t c = dg ? (kCodeDiag | kCodeViaK | kdu)
-                                    : (vt ? (kCodeVert | kCodeViaK | kvu) : kCodeHorz);
+              const uint32_t c = dg ? (kCodeDiag | kdu)
+                                    : (vt ? (kCodeVert | kvu) : kCodeHorz);
               code |= c << (16 * u);
             }
             if (live) *reinterpret_cast<uint32_t*>(Cr + j0 + 2 * q) = code;
@@ -1675,14 +1675,14 @@ __device__ __forceinline__ int dp_band(CParams& P, const Slot& s, uint32_t lds, 
               const bool dg = ((bd[q] >> (16 * u)) & 0xffffu) == hu;
               const bool vt = ((bv[q] >> (16 * u)) & 0xffffu) == hu;
               const uint32_t kdu = (kd >> (16 * u)) & 0xffffu, kvu = (kx[q] >> (16 * u)) & 0xffffu;
-              const uint32_t c = dg ? (kCodeDiag | kCodeViaK | kdu)
-                                    : (vt ? (kCodeVert | kCodeViaK | kvu) : kCodeHorz);
+              const uint32_t c = dg ? (kCodeDiag | kdu)
+                                    : (vt ? (kCodeVert | kvu) : kCodeHorz);
               code |= c << (16 * u);
             }
             *reinterpret_cast<uint32_t*>(Cr + j0 + kBandColumn + 2 * q) = code;
           }
           if (lane == 0 && lo == 0) {
-            Cr[kBandColumn] = static_cast<uint16_t>(kCodeVert | kCodeViaK | k_left);
+            Cr[kBandColumn] = static_cast<uint16_t>(kCodeVert | k_left);
           }
         }
       }
@@ -3472,10 +3472,7 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
         auto successor = [&](uint32_t c, int dj) -> uint32_t {
           const int kind = static_cast<int>(c & 0xc000u);
           const int pay = static_cast<int>(c & kCodePayload);
-          int delta = pay;
-          if ((c & kCodeViaK) != 0) {
-            delta = pay < 4 ? static_cast<int>((d4 >> (16 * pay)) & 0xffffu) : 0;
-          }
+          const int delta = pay < 4 ? static_cast<int>((d4 >> (16 * pay)) & 0xffffu) : 0;
           const int jj = j0 - dj;
           if (ri < 1 || jj < 0 || (kind != kCodeVert && jj == 0) || kind == 0xc000) return kNextExit;
           int ndi = di_l, ndj = dj;
@@ -3523,20 +3520,17 @@ __device__ __forceinline__ void process_window(CParams& P, Slot& s, uint8_t* lds
               --j;
             }
             const int pay = c & static_cast<int>(kCodePayload);
-            int delta = pay;
-            if ((c & kCodeViaK) != 0) {
-              // predecessor by in-edge index: the row's delta table, else the lists
-              delta = 0;
-              if (pay < 4) {
-                const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(d4), (idx >> 3) * 4);
-                const uint32_t hi =
-                    __builtin_amdgcn_readlane(static_cast<uint32_t>(d4 >> 32), (idx >> 3) * 4);
-                const uint32_t w = pay < 2 ? lo : hi;
-                delta = static_cast<int>((w >> (16 * (pay & 1))) & 0xffffu);
-              }
-              if (delta == 0) {
-                delta = i - (uniform(pred_rows[uniform(pred_off[i - 1]) + pay]) & kPredRowMask);
-              }
+            // predecessor by in-edge index: the row's delta table, else the lists
+            int delta = 0;
+            if (pay < 4) {
+              const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(d4), (idx >> 3) * 4);
+              const uint32_t hi =
+                  __builtin_amdgcn_readlane(static_cast<uint32_t>(d4 >> 32), (idx >> 3) * 4);
+              const uint32_t w = pay < 2 ? lo : hi;
+              delta = static_cast<int>((w >> (16 * (pay & 1))) & 0xffffu);
+            }
+            if (delta == 0) {
+              delta = i - (uniform(pred_rows[uniform(pred_off[i - 1]) + pay]) & kPredRowMask);
             }
             i -= delta;
             bad = i < 0;

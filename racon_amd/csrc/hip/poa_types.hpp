@@ -97,8 +97,10 @@ constexpr uint32_t kPoaHPoolRows = 128;
 constexpr uint32_t kMaxAligned = 8;
 constexpr uint32_t kMaxAlignedWide = 16;
 
-// DP row pitch >= layer length + kPoaColPad: strips that end past column L
-// (up to 12 columns, stored from column + 3) stay inside their row.
+// DP row pitch >= layer length + kPoaColPad: the last strip (up to 20 columns
+// a lane, so up to 19 past column L), a band's last columns with their offset
+// of 3, and column 0 of the tiled rows at the end stay inside their row, and
+// idle lanes find 20 columns past L to write to.
 constexpr uint32_t kPoaColPad = 24;
 
 // Byte offsets of every array inside one slot.
