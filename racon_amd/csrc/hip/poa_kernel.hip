@@ -1675,8 +1675,9 @@ __device__ __forceinline__ int dp_band(CParams& P, const Slot& s, uint32_t lds, 
               const bool dg = ((bd[q] >> (16 * u)) & 0xffffu) == hu;
               const bool vt = ((bv[q] >> (16 * u)) & 0xffffu) == hu;
               const uint32_t kdu = (kd >> (16 * u)) & 0xffffu, kvu = (kx[q] >> (16 * u)) & 0xffffu;
-              const uint32_t c = dg ? (kCodeDiag | kdu)
-                                    : (vt ? (kCodeVert | kvu) : kCodeHorz);
+              uint32_t c = vt ? (kCodeVert | kvu) : kCodeHorz;
+              if (dg) c = kCodeDiag | kdu;
+              pin(c);  // (without it the compiler's loop of the common rows takes 3% longer)
               code |= c << (16 * u);
             }
             *reinterpret_cast<uint32_t*>(Cr + j0 + kBandColumn + 2 * q) = code;
