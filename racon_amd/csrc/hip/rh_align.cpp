@@ -317,14 +317,8 @@ int32_t rh_align_run(rh_align_batch* b) {
     b->d_scratch.release();
     b->d_team.release();
   }
-  // (slots follow the longest pair, which differs from chunk to chunk: a
-  // buffer that had to grow once takes headroom, since growing waits for the
-  // other streams' kernels)
-  const bool spare = kept + kept / 4 <= room;
   for (const Part& part : parts) {
-    RH_HIP_CHECK(part.scratch->reserve(part.slots * part.slot_bytes,
-                                       spare && part.scratch->bytes != 0),
-                 RH_ERR_MEMORY);
+    RH_HIP_CHECK(part.scratch->reserve(part.slots * part.slot_bytes), RH_ERR_MEMORY);
   }
   RH_HIP_CHECK(b->d_queue.reserve(2 * sizeof(uint32_t)), RH_ERR_MEMORY);
   RH_HIP_CHECK(hipMemsetAsync(b->d_queue.ptr, 0, 2 * sizeof(uint32_t), b->stream), RH_ERR_DEVICE);

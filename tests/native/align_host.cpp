@@ -215,25 +215,6 @@ int small() {
   rh_align_destroy(b);
   return problem.empty() ? 0 : bad(problem);
 }
-
-// Chunks of about one size: the buffers grow once, not with every longest
-// pair so far.
-int growth() {
-  pool = size_t(4) << 30;
-  rh_align_batch* b = nullptr;
-  if (rh_align_create(0, &b) != RH_OK) return bad("create");
-  for (uint32_t k = 0; k < 12; ++k) {
-    std::vector<rh_pair> pairs;
-    add(pairs, 8, 30000 + 500 * k);
-    add(pairs, 40, 8000 + 100 * k);
-    if (rh_align_upload(b, pairs.size(), pairs.data()) != RH_OK) return bad("upload");
-    const int before_run = frees;
-    if (rh_align_run(b) != RH_OK) return bad("run");
-    if (k >= 2 && frees != before_run) return bad("chunk " + std::to_string(k) + " grew a buffer");
-  }
-  rh_align_destroy(b);
-  return problem.empty() ? 0 : bad(problem);
-}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -241,6 +222,5 @@ int main(int argc, char** argv) {
   if (scenario == "errors") return errors();
   if (scenario == "memory") return memory();
   if (scenario == "small") return small();
-  if (scenario == "growth") return growth();
   return bad("unknown scenario " + scenario);
 }

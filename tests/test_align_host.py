@@ -24,7 +24,7 @@ def align_host(tmp_path_factory):
     return str(exe)
 
 
-@pytest.mark.parametrize("scenario", ["errors", "memory", "small", "growth"])
+@pytest.mark.parametrize("scenario", ["errors", "memory", "small"])
 def test_batch(align_host, scenario):
     done = subprocess.run([align_host, scenario], capture_output=True, text=True, timeout=60)
     assert done.returncode == 0, done.stdout + done.stderr
