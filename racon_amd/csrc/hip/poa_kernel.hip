@@ -1005,7 +1005,7 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
   for (int q = 0; q < H2; ++q) cur[q] = 0;
   // position in seq of the letter of the strip's first column (-1: column 0
   // has none; lanes past the last column read the bytes behind the layer)
-  const int letters = min(lane * W, pitch - W) - 1;
+  [[maybe_unused]] const int letters = min(lane * W, pitch - W) - 1;
   GByte* const codes = (GByte*)s.code();
   uint32_t rec_lane = min(static_cast<uint32_t>(lane * row_record_bytes(W)),
                           row_bytes - static_cast<uint32_t>(row_record_bytes(W)));
@@ -1104,19 +1104,31 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
         *(__attribute__((address_space(1))) U32x4*)at = U32x4{acc[0], acc[1], ack[0], ack[1]};
       }
     };
-    // scores of the strip's letters against a row's, letter by letter
-    const auto letter_scores = [&](uint32_t letter, uint32_t* out) {
-      const uint32_t other = (letter & 0xffu) * 0x10001u;
-      const uint32_t hit = miss ^ flip;
+    // scores of the strip's letters against a row's of any letter: from the
+    // table in a plain layer, letter by letter in another
+    const auto letter_scores = [&](uint32_t meta, uint32_t* out) {
+      const uint32_t letter = meta & 0xffu;
+      if constexpr (kPlain) {
+        const uint32_t code = ((letter >> 1) ^ (letter >> 2)) & 3u;
+        const bool base = ((0x54474341u >> (8 * code)) & 0xffu) == letter;
+        const uint64_t t = base ? table0 ^ (table1 << (8 * code)) : table0;
 #pragma unroll
-      for (int q = 0; q < H2; ++q) {
-        // (column 0's position is before the first)
-        const uint32_t a = seq[q == 0 ? max(letters, 0) : letters + 2 * q];
-        const uint32_t b = seq[letters + 2 * q + 1];
-        const uint32_t differ = pk_min_u((a | b << 16) ^ other, one);
-        out[q] = pk_mad(differ, pk_sub(miss * 0x10001u, hit * 0x10001u), hit * 0x10001u);
+        for (int q = 0; q < H2; ++q) {
+          out[q] = __builtin_amdgcn_perm(static_cast<uint32_t>(t >> 32),
+                                         static_cast<uint32_t>(t), sel[q]);
+        }
+      } else {
+        const uint32_t hit = miss ^ flip;
+#pragma unroll
+        for (int q = 0; q < H2; ++q) {
+          // (column 0's position is before the first)
+          const uint32_t a = seq[q == 0 ? max(letters, 0) : letters + 2 * q];
+          const uint32_t b = seq[letters + 2 * q + 1];
+          const uint32_t differ = pk_min_u((a | b << 16) ^ letter * 0x10001u, one);
+          out[q] = pk_mad(differ, pk_sub(miss * 0x10001u, hit * 0x10001u), hit * 0x10001u);
+        }
+        if (lane == 0) out[0] &= 0xffff0000u;  // column 0 has no letter
       }
-      if (lane == 0) out[0] &= 0xffff0000u;  // column 0 has no letter
     };
     next_row(0);
     int rr = 0;
@@ -1204,13 +1216,7 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
         // own scores
         const uint32_t meta = static_cast<uint32_t>(__builtin_amdgcn_readlane(meta_v, rr));
         np = (meta >> kRowMetaPredShift) & kRowMetaPredMask;
-        if constexpr (kPlain) {
-          table = table0;  // it matches none of the layer's
-#pragma unroll
-          for (int q = 0; q < H2; ++q) next_sub(q);
-        } else {
-          letter_scores(meta, sub);
-        }
+        letter_scores(meta, sub);
         continue;
       }
       record += row_bytes;
@@ -1267,14 +1273,13 @@ __device__ __forceinline__ int dp_rows(CParams& P, const Slot& s, uint32_t lds, 
             mx[q] = pk_max_u(mx[q], pp[q]);
           }
         }
-        uint32_t scores[H2];
-        letter_scores(static_cast<uint32_t>(meta), scores);
 #pragma unroll
         for (int q = 0; q < H2; ++q) {
           // (a move, so that mx and cur need not share registers)
           asm volatile("v_mov_b32 %0, %1" : "=v"(cur[q]) : "v"(mx[q]));
         }
-        row_scores<W>(cur, scores, gap_pair, bd, bv, [](int) {});
+        letter_scores(static_cast<uint32_t>(meta), sub);
+        row_scores<W>(cur, sub, gap_pair, bd, bv, [](int) {});
         if (own < kSlotGlobal) {
           lds_row_store<W>(strip + static_cast<uint32_t>(own) * row_bytes, cur);
         } else if (own == kSlotGlobal) {
